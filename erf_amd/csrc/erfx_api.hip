@@ -365,7 +365,7 @@ int erfx_ctx_create(const erfx_config* cfg, void* stream, erfx_ctx** out) {
     c->stream = static_cast<hipStream_t>(stream);
     const size_t ne = (size_t)lay.nelem;
     const size_t sh = row_shift(c->P.L);
-    double** bufs[] = {&c->fw.extrap, &c->fw.drw, &c->fw.soln, &c->sw.pp,
+    double** bufs[] = {&c->fw.drw, &c->fw.soln, &c->sw.pp,
                        &c->sw.tau[0], &c->sw.tau[1], &c->sw.tau[2], &c->sw.tau[3], &c->sw.tau[4], &c->sw.tau[5]};
     for (double** b : bufs)
         if ((rc = dalloc(c->allocs, b, ne, sh))) { erfx_ctx_destroy(c); return rc; }
@@ -1065,11 +1065,12 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
         for (int ks = 0; ks < (nosub ? 0 : nsub); ++ks) {
             // On a laterally periodic box the apply_bcs between two substeps is
             // folded into the next substep (round trip of the momenta on read,
-            // ghost layer 1 of rho and rho*theta written by the column kernel);
-            // the full fill runs after the stage's last substep.
+            // ghost cells read at their images); the full fill runs after the
+            // stage's last substep.
             FastChain ch;
+            ch.active = chain;
             ch.rt_prev = chain && ks > 0;
-            ch.ghost_writes = chain && ks < nsub - 1 && !P.terrain;   // the terrain substep reads images
+            ch.last = ks == nsub - 1;
             ch.w_lo = P.vel_extdir[2][2];
             ch.w_hi = P.vel_extdir[2][5];
             if (ks == 0) make_fast_coeffs(P, s->fast_coeffs, Sn, s->prim, s->pi_stage, s->r0, s->pi0, dtau, beta_s, st);

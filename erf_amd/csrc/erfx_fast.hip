@@ -2,13 +2,15 @@
 // erf_fast_rhs_N as gfx950 kernels.
 //
 // Launch structure per substep:
-//   K1  cells grown by 1: Delta(rho theta), extrapolated theta, lagged update
-//   K2  x- and y-faces (one launch): horizontal momentum update, written
-//       straight into the current state (each lane reads prev and writes cur
-//       at its own index, so the S_prev == S_data aliasing is safe)
+//   K1-2 x- and y-faces (one launch): Delta(rho theta) of the face's two cells
+//       extrapolated forward, horizontal momentum update, written straight into
+//       the current state (each lane reads prev and writes cur at its own
+//       index, so the S_prev == S_data aliasing is safe)
 //   K3-5 columns (one lane per (i, j), k loops): horizontal divergence of the
 //       increments, tridiagonal RHS, Thomas sweep, new rho*w, vertical
-//       fluxes, time-averaged rho*w, rho and rho*theta update
+//       fluxes, time-averaged rho*w, rho and rho*theta update; the lagged
+//       Delta(rho theta), which K1-2 of this substep has read, is replaced by
+//       the new one here, where each lane owns its column
 // The arithmetic of every point keeps the reference's operation order.
 #include "erfx_common.h"
 #include "erfx_internal.h"
@@ -139,6 +141,35 @@ void no_substep(const Params& P, const erfx_state& ssum, const erfx_state& sold,
     });
 }
 
+// The grown box's ghost layer (one cell all round, edges and corners included)
+// of the lagged increment rt_prev - rt_stage, in one launch: the z rows, the y
+// rows, then the x sides with the lanes along j.  With `cons` and `from`, rho and
+// rho*theta of those cells are copied from `from` as well (the terrain form's
+// first substep).
+void lagged_shell(const Params& P, const double* prt, const double* srt, double* lagged, double* cons,
+                  const double* from, hipStream_t s) {
+    const Lay L = P.L;
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    const long ne = L.ne;
+    const int nzr = 2 * (ny + 2), nyr = 2 * nz, w = nx + 2 > ny ? nx + 2 : ny;
+    launch_box(Box(0, 0, 0, w - 1, nzr + 2 * nyr - 1, 0), s, [=] __device__(int t, int r, int) {
+        int i, j, k;
+        if (r < nzr) {
+            if (t > nx + 1) return;
+            i = t - 1; j = r / 2 - 1; k = (r & 1) ? nz : -1;
+        } else if (r < nzr + nyr) {
+            if (t > nx + 1) return;
+            i = t - 1; k = (r - nzr) / 2; j = ((r - nzr) & 1) ? ny : -1;
+        } else {
+            if (t > ny - 1) return;
+            j = t; k = (r - nzr - nyr) / 2; i = ((r - nzr - nyr) & 1) ? nx : -1;
+        }
+        const long q = L.ix(i, j, k);
+        if (cons) { cons[q] = from[q]; cons[q + ne] = from[q + ne]; }
+        lagged[q] = prt[q] - srt[q];
+    });
+}
+
 void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erfx_state& slow_rhs,
                 const erfx_state& prev, const erfx_state& stage, const double* prim, const double* pi_stage,
                 const double* fc, const erfx_state& data, const erfx_state& scratch, double dtau,
@@ -151,7 +182,6 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     const double beta_d = 0.1;
     const double dxi = P.dxInv[0], dyi = P.dxInv[1], dzi = P.dxInv[2];
     const bool implicit = P.cfg.implicit_substepping != 0;
-    double* extrap = W.extrap;
     double* drw = W.drw;
     double* tr0 = W.trhs;
     double* tr1 = W.trhs + ne;
@@ -160,67 +190,79 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     const double* srt = stage.cons + ne;
     double* lagged = scratch.cons + ne;
 
-    // K1 (ERF_fast_rhs_N.cpp:115-152)
-    launch_box(Box(-1, -1, -1, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
-        const long q = L.ix(i, j, k);
-        double d = prt[q] - srt[q];
-        extrap[q] = (step == 0) ? d : d + beta_d * (d - lagged[q]);
-        lagged[q] = d;
-    });
-
-    // K2 (:161-257).  With rt_prev the previous substep's apply_bcs is folded in:
-    // its momentum -> velocity -> momentum round trip (ERF_MomentumToVelocity.cpp,
-    // ERF_VelocityToMomentum.cpp) is applied to prev as it is read.
+    // K1 + K2 (:115-257), one lane per x- and y-face.  Delta(rho theta) of a
+    // cell, extrapolated forward with the lagged increment (:115-152), is formed
+    // by each of the four faces that read it: 3 fields of neighbour reads, which
+    // the four rows of a work-group share, in place of a field written and read
+    // again by a launch of its own.  HBM bound at 13 fields read and 4 written
+    // (256 x 256 x 128: 283 us as two launches, 250 us as one, 4.6 TB/s).  With rt_prev the previous substep's
+    // apply_bcs is folded in: its momentum -> velocity -> momentum round trip
+    // (ERF_MomentumToVelocity.cpp, ERF_VelocityToMomentum.cpp) is applied to
+    // prev as it is read, and ghost cells are read at their periodic images.
     const bool first = (nrk == 0 && step == 0);
     const bool rt = ch.rt_prev && step > 0;
+    const bool use_lag = step > 0;
     const double* prho = prev.cons;
     const double gr = -Gamma * R_d;
     const bool moist = P.moist;
     const double* pq1 = prim + PRIM_Q1 * ne;
     const double* pq2 = prim + PRIM_Q2 * ne;
+    // Every load is issued before the first store: the stores may alias the
+    // inputs as far as the compiler knows, so loads of the y-face after the
+    // stores of the x-face would wait for a second round trip to memory.  (The
+    // loads of a face outside its box stay inside the layout; only the stores
+    // are guarded.)
+    const double *pxm = prev.xmom, *pym = prev.ymom, *sxm = stage.xmom, *sym = stage.ymom;
+    const double *slx = slow_rhs.xmom, *sly = slow_rhs.ymom;
+    double *axm = scratch.xmom, *aym = scratch.ymom, *dxm = data.xmom, *dym = data.ymom;
     launch_box(Box(0, 0, 0, nx, ny, nz - 1), s, [=] __device__(int i, int j, int k) {
         const long q = L.ix(i, j, k);
+        // the faces' cells: c (i, j), x (i-1, j), y (i, j-1); images in the chain
+        const long qc = rt ? q - (i == nx ? nx : 0) - (j == ny ? (long)ny * sy : 0) : q;
+        const long qx = (rt && i == 0) ? q + nx - 1 : q - 1;
+        const long qy = (rt && j == 0) ? q + (long)(ny - 1) * sy : q - sy;
+        double pmx = pxm[q], pmy = pym[q];
+        const double sx = sxm[q], sy_ = sym[q], lx = slx[q], ly = sly[q], ax = axm[q], ay = aym[q];
+        double rc = 0.0, rx = 0.0, ry = 0.0;
+        if (rt) { rc = prho[qc]; rx = prho[qx]; ry = prho[qy]; }
+        double frx = 0.0, fry = 0.0;
+        if (!first) {
+            double ec = prt[qc] - srt[qc], ex = prt[qx] - srt[qx], ey = prt[qy] - srt[qy];
+            const double pc = pi_stage[q], px = pi_stage[q - 1], py = pi_stage[q - sy];
+            if (use_lag) {
+                const double lc = lagged[qc], lgx = lagged[qx], lgy = lagged[qy];
+                ec = ec + beta_d * (ec - lc);
+                ex = ex + beta_d * (ex - lgx);
+                ey = ey + beta_d * (ey - lgy);
+            }
+            double gpx = (ec - ex) * dxi, gpy = (ec - ey) * dyi;
+            if (moist) {   // :215-219, :238-242
+                gpx /= (1.0 + face_q(pq1, pq2, q, q - 1));
+                gpy /= (1.0 + face_q(pq1, pq2, q, q - sy));
+            }
+            frx = gr * (0.5 * (px + pc)) * gpx;
+            fry = gr * (0.5 * (py + pc)) * gpy;
+        }
+        if (rt) {
+            const double d = rc + rx, e = rc + ry;
+            const double u = pmx * 2.0 / d, v = pmy * 2.0 / e;
+            pmx = u * 0.5 * d;
+            pmy = v * 0.5 * e;
+        }
+        const double nu = first ? pmx - sx + dtau * lx : pmx - sx + dtau * frx + dtau * lx;
+        const double nv = first ? pmy - sy_ + dtau * ly : pmy - sy_ + dtau * fry + dtau * ly;
         if (j <= ny - 1) {
-            double pm = prev.xmom[q];
-            if (rt) {
-                double d = prho[q] + prho[q - 1];
-                double u = pm * 2.0 / d;
-                pm = u * 0.5 * d;
-            }
-            double new_drho_u;
-            if (first) {
-                new_drho_u = pm - stage.xmom[q] + dtau * slow_rhs.xmom[q];
-            } else {
-                double gpx = (extrap[q] - extrap[q - 1]) * dxi;
-                if (moist) gpx /= (1.0 + face_q(pq1, pq2, q, q - 1));   // :215-219
-                double pi_c = 0.5 * (pi_stage[q - 1] + pi_stage[q]);
-                double fast_rhs_rho_u = gr * pi_c * gpx;
-                new_drho_u = pm - stage.xmom[q] + dtau * fast_rhs_rho_u + dtau * slow_rhs.xmom[q];
-            }
-            scratch.xmom[q] += facinv * new_drho_u;
-            data.xmom[q] = stage.xmom[q] + new_drho_u;
+            axm[q] = ax + facinv * nu;
+            dxm[q] = sx + nu;
         }
         if (i <= nx - 1) {
-            double pm = prev.ymom[q];
-            if (rt) {
-                double d = prho[q] + prho[q - sy];
-                double v = pm * 2.0 / d;
-                pm = v * 0.5 * d;
-            }
-            double new_drho_v;
-            if (first) {
-                new_drho_v = pm - stage.ymom[q] + dtau * slow_rhs.ymom[q];
-            } else {
-                double gpy = (extrap[q] - extrap[q - sy]) * dyi;
-                if (moist) gpy /= (1.0 + face_q(pq1, pq2, q, q - sy));  // :238-242
-                double pi_c = 0.5 * (pi_stage[q - sy] + pi_stage[q]);
-                double fast_rhs_rho_v = gr * pi_c * gpy;
-                new_drho_v = pm - stage.ymom[q] + dtau * fast_rhs_rho_v + dtau * slow_rhs.ymom[q];
-            }
-            scratch.ymom[q] += facinv * new_drho_v;
-            data.ymom[q] = stage.ymom[q] + new_drho_v;
+            aym[q] = ay + facinv * nv;
+            dym[q] = sy_ + nv;
         }
     });
+    // the lagged increment's ghost layer, which the next substep reads unless it
+    // reads the periodic images
+    if (!ch.active) lagged_shell(P, prt, srt, lagged, nullptr, nullptr, s);
 
     // K3 + K4 + K5 fused per column (:328-357, :374-453, :518-536, :566-592).
     // One lane per (i, j) column.  Forward sweep: horizontal divergence of the
@@ -241,7 +283,6 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     const double* st0 = stage.cons;
     double* cc0 = data.cons;
     double* cc1 = data.cons + ne;
-    const bool gw = ch.ghost_writes;
     const double ch_w_lo = ch.w_lo, ch_w_hi = ch.w_hi;
     auto column = [=] __device__(int i, int j, auto depth) {
         const long q0 = L.ix(i, j, 0);
@@ -298,6 +339,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         tr1[q0] = t1_km1;
         double drho_km1 = cur.pr - cur.st;
         double drt_km1 = cur.prt_ - cur.srt_;
+        lagged[q0] = drt_km1;
         double s0_km1 = cur.s0, s1_km1 = cur.s1;
         double p_km2 = prim[q0 - sz], p_km1 = cur.pc, p_k = cur.pkp1;
         double q1_km1 = cur.q1, q2_km1 = cur.q2;
@@ -324,6 +366,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 double Om_kp1 = w_above(c, k + 1) - c.szz;
                 double drho_k = c.pr - c.st;
                 double drt_k = c.prt_ - c.srt_;
+                lagged[q] = drt_k;
                 double coeff_P = c.P, coeff_Q = c.Q;
                 if (moist) {   // :379-384
                     double qf = 0.5 * (c.q1 + q1_km1 + c.q2 + q2_km1);
@@ -396,27 +439,6 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 double rt_new = bc.c1 + dtau * (bc.s1 - t1);
                 cc0[q] = r_new;
                 cc1[q] = rt_new;
-                if (gw) {
-                    // ghost layer 1 as the skipped apply_bcs would leave it: the
-                    // periodic images of this cell, and at k = 0 / nz-1 the
-                    // foextrap rows below / above, images included
-                    const int ia[2] = {i, i == 0 ? nx : (i == nx - 1 ? -1 : i)};
-                    const int ja[2] = {j, j == 0 ? ny : (j == ny - 1 ? -1 : j)};
-                    const int nk = (k == 0 ? 1 : 0) + (k == nz - 1 ? 1 : 0);
-                    const int ka[3] = {k, k == 0 ? -1 : nz, nz};
-                    for (int a = 0; a < 2; ++a) {
-                        if (a == 1 && ia[1] == i) continue;
-                        for (int b = 0; b < 2; ++b) {
-                            if (b == 1 && ja[1] == j) continue;
-                            for (int c3 = 0; c3 <= nk; ++c3) {
-                                if (a == 0 && b == 0 && c3 == 0) continue;
-                                long g = L.ix(ia[a], ja[b], ka[c3]);
-                                cc0[g] = r_new;
-                                cc1[g] = rt_new;
-                            }
-                        }
-                    }
-                }
                 sol_next = sol;
                 drw_next = drw_k;
                 p_next = pcq;
@@ -514,6 +536,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 Om_km1 = om_face(kc);
                 Om_k = om_face(kc + 1);
                 if (ka == 0) {      // face 0: the bottom row (:423-432)
+                    lagged[q0] = drt_km1;
                     X[lane] = Om_km1 + dtau * c.ws;
                     Z[lane] = iB[q0];
                     t0r[0] = t0_km1; t1r[0] = t1_km1; omr[0] = Om_km1;
@@ -533,6 +556,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 double Om_kp1 = om_face(k + 1);
                 double drho_k = c.pr - c.st;
                 double drt_k = c.prt_ - c.srt_;
+                lagged[q] = drt_k;
                 double coeff_P = c.P, coeff_Q = c.Q;
                 if (moist) {   // :379-384
                     double qf = 0.5 * (c.q1 + q1_km1 + c.q2 + q2_km1);
@@ -620,24 +644,6 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 double rt_new = c1 + dtau * (s1 - t1);
                 cc0[q] = r_new;
                 cc1[q] = rt_new;
-                if (gw) {
-                    const int ia[2] = {i, i == 0 ? nx : (i == nx - 1 ? -1 : i)};
-                    const int ja[2] = {j, j == 0 ? ny : (j == ny - 1 ? -1 : j)};
-                    const int nk = (k == 0 ? 1 : 0) + (k == nz - 1 ? 1 : 0);
-                    const int ka3[3] = {k, k == 0 ? -1 : nz, nz};
-                    for (int a = 0; a < 2; ++a) {
-                        if (a == 1 && ia[1] == i) continue;
-                        for (int b = 0; b < 2; ++b) {
-                            if (b == 1 && ja[1] == j) continue;
-                            for (int c3 = 0; c3 <= nk; ++c3) {
-                                if (a == 0 && b == 0 && c3 == 0) continue;
-                                long g = L.ix(ia[a], ja[b], ka3[c3]);
-                                cc0[g] = r_new;
-                                cc1[g] = rt_new;
-                            }
-                        }
-                    }
-                }
                 tile_level_fence();
             }
         }
@@ -724,13 +730,13 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
 // ---- erf_fast_rhs_N with no device allocation ---------------------------------
 // For callers that cannot allocate device memory (code under stream / graph
 // capture, tight serving loops, harnesses that forbid hipMalloc): the work
-// fields of the substep (theta extrapolated, the rho*w increment, the two
-// horizontal divergences and the tridiagonal solution: 5 fields of the
-// layout) live in one static device array instead of a context's workspace.
+// fields of the substep (the rho*w increment, the two horizontal divergences
+// and the tridiagonal solution) and one field in reserve, 5 of the layout, live
+// in one static device array instead of a context's workspace.
 // Each GPU holds its own copy of the array until the process ends; calls on
 // one GPU share it, so two calls that overlap on one GPU race.  No element of
 // it needs to start at zero: every launch of the substep writes each element
-// it reads (K1 the grown box of theta, the column kernel its own column)
+// it reads (the column kernel its own column)
 // before reading it, so whatever a previous call left there is never seen.
 namespace erfx {
 namespace noalloc {
@@ -800,7 +806,6 @@ extern "C" int erfx_fast_rhs_N_noalloc(const erfx_config* cfg, void* stream, int
     Params P;
     make_params(*cfg, lay, P);
     FastWork W;
-    W.extrap = base;
     W.drw = base + ne;
     W.trhs = base + 2 * ne;      // two components
     W.soln = base + 4 * ne;

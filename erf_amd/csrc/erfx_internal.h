@@ -47,7 +47,6 @@ void views_release(const erfx_ctx* c);
 
 // erfx_fast.hip
 struct FastWork {
-    double* extrap;   // theta extrapolated forward, cells grown by 1
     double* drw;      // delta rho*w at the previous substep, z-faces grown by 1 laterally
     double* trhs;     // 2 comps: flux divergence of rho and rho*theta increments, cells
     double* soln;     // tridiagonal solution on z-faces
@@ -57,17 +56,20 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
                       hipStream_t s);
 // Options of the sim driver's substep chain; all off for the C-ABI hook.
 struct FastChain {
+    bool active = false;   // the substeps of a stage are chained
     // prev is S_sum of the previous substep without its apply_bcs: apply the
-    // momentum -> velocity -> momentum round trip of that apply_bcs on read
+    // momentum -> velocity -> momentum round trip of that apply_bcs on read and
+    // read ghost cells at their images (periodic, foextrap rows)
     bool rt_prev = false;
-    // write ghost layer 1 of rho and rho*theta (periodic images, foextrap rows)
-    bool ghost_writes = false;
+    bool last = true;      // the stage's last substep
     double w_lo = 0.0, w_hi = 0.0;   // Dirichlet w on the bottom and top faces
 };
 void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erfx_state& slow_rhs,
                 const erfx_state& prev, const erfx_state& stage, const double* prim, const double* pi_stage,
                 const double* fc, const erfx_state& data, const erfx_state& scratch, double dtau,
                 double beta_s, double facinv, hipStream_t s, const FastChain& ch = FastChain());
+void lagged_shell(const Params& P, const double* prt, const double* srt, double* lagged, double* cons,
+                  const double* from, hipStream_t s);
 bool fast_bcs_fusable(const Params& P);
 // no_substep_fun (substepping_type None): S_sum = S_old + slow_dt * F_slow for
 // rho, rho*theta and the momenta

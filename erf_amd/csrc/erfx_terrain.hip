@@ -1,9 +1,9 @@
 // erfx_terrain.hip -- terrain-following grid: the metrics of the node heights
 // and the acoustic substep erf_fast_rhs_T (static terrain, unit map factors).
 //
-// The substep runs as three phases: theta extrapolation and the horizontal
-// momentum increments on the grown box; the new horizontal momenta; and one
-// lane per column that forms Omega of the old increments and the horizontal
+// The substep runs as two phases: theta extrapolation, the horizontal momentum
+// increments and the new horizontal momenta on the faces; and one lane per
+// column that forms Omega of the old increments and the horizontal
 // divergence of the new ones as it sweeps up, solves the implicit vertical
 // system and updates rho, rho*theta and rho*w on the way down.  Every
 // expression keeps the reference's operation order (FP contraction is off),
@@ -86,7 +86,6 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
     double* du = T.du; double* dv = T.dv;
     double* nu = T.nu; double* nv = T.nv; double* om = T.om;
     double* wtop = T.wtop;
-    double* extrap = W.extrap;
     double* trhs0 = W.trhs;
     double* trhs1 = W.trhs + ne;
     double* soln = W.soln;
@@ -100,28 +99,13 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
     // each momentum is put through the momentum -> velocity -> momentum round
     // trip with the face density of its periodic image
     // (ERF_MomentumToVelocity.cpp, ERF_VelocityToMomentum.cpp), so the rounding
-    // is the reference's.
+    // is the reference's.  The horizontal momenta of prev are stage + nu, the sum
+    // the previous substep would have stored: the chain keeps the increments nu,
+    // nv alone and stores the momenta in its last substep.
     const bool rt = ch.rt_prev && step > 0;
     const double* prho = prev.cons;
     auto wrap_c = [=] __device__(int a, int n) { return a < 0 ? a + n : (a > n - 1 ? a - n : a); };
     auto wrap_f = [=] __device__(int a, int n) { return a < 0 ? a + n : (a > n ? a - n : a); };
-    // the cell holding the value of (possibly ghost) cell (i, j, k)
-    auto cimg = [=] __device__(int i, int j, int k) {
-        return L.ix(wrap_c(i, nx), wrap_c(j, ny), k < 0 ? 0 : (k > nz - 1 ? nz - 1 : k));
-    };
-    // round trip of x-momentum on (possibly ghost) face (i, j, k), k valid
-    auto rt_x = [=] __device__(int i, int j, int k) {
-        const int fi = wrap_f(i, nx), cj = wrap_c(j, ny);
-        const double d = prho[L.ix(wrap_c(fi, nx), cj, k)] + prho[L.ix(wrap_c(fi - 1, nx), cj, k)];
-        const double u = pxm[L.ix(fi, cj, k)] * 2.0 / d;
-        return u * 0.5 * d;
-    };
-    auto rt_y = [=] __device__(int i, int j, int k) {
-        const int ci = wrap_c(i, nx), fj = wrap_f(j, ny);
-        const double d = prho[L.ix(ci, wrap_c(fj, ny), k)] + prho[L.ix(ci, wrap_c(fj - 1, ny), k)];
-        const double v = pym[L.ix(ci, fj, k)] * 2.0 / d;
-        return v * 0.5 * d;
-    };
     // rho*w on the top face of column (i, j) as the skipped apply_bcs leaves it
     // (Dirichlet top on a terrain grid, ERF_BoundaryConditions_zvel.cpp:220-257):
     // w = WFromOmega of the top value with u and v as the fill makes them --
@@ -138,7 +122,8 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         }
         const int fi = wrap_f(ii, nx), cj = wrap_c(jj, ny);
         const double d = prho[L.ix(wrap_c(fi, nx), cj, kk)] + prho[L.ix(wrap_c(fi - 1, nx), cj, kk)];
-        return pxm[L.ix(fi, cj, kk)] * 2.0 / d;
+        const long f = L.ix(fi, cj, kk);
+        return (sxm[f] + nu[f]) * 2.0 / d;
     };
     auto v_fill = [=] __device__(int ii, int jj, int kk) -> double {
         if (kk > nz - 1) {
@@ -147,7 +132,8 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         }
         const int ci = wrap_c(ii, nx), fj = wrap_f(jj, ny);
         const double d = prho[L.ix(ci, wrap_c(fj, ny), kk)] + prho[L.ix(ci, wrap_c(fj - 1, ny), kk)];
-        return pym[L.ix(ci, fj, kk)] * 2.0 / d;
+        const long f = L.ix(ci, fj, kk);
+        return (sym[f] + nv[f]) * 2.0 / d;
     };
     auto pw_top = [=] __device__(int i, int j) -> double {
         const double w = met::w_from_omega(i, j, nz, zvh, u_fill, v_fill, z, dxi, dyi);
@@ -155,36 +141,25 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         return w * 0.5 * (r + r);
     };
 
-    // :139-204: rho, rho*theta copied from prev on the grown box (step 0);
-    // theta extrapolated forward and the lagged increment; the horizontal
-    // momentum increments on faces grown by one laterally, kept because the
-    // new momenta overwrite prev when it aliases data (the rho, rho*theta and
-    // rho*w increments are formed where they are used, from prev and stage)
-    launch_box(Box(-1, -1, -1, nx + 1, ny, nz - 1), s, [=] __device__(int i, int j, int k) {
-        const long q = L.ix(i, j, k);
-        if (i <= nx) {
-            if (first) { cc0[q] = pc0[q]; cc1[q] = pc1[q]; }
-            double dt_ = (rt ? cc1[cimg(i, j, k)] : cc1[q]) - sc1[q];
-            extrap[q] = first ? dt_ : dt_ + beta_d * (dt_ - lagged1[q]);
-            lagged1[q] = dt_;
-        }
-        if (k >= 0) du[q] = (rt ? rt_x(i, j, k) : pxm[q]) - sxm[q];
-        if (k >= 0 && i <= nx) dv[q] = (rt ? rt_y(i, j, k) : pym[q]) - sym[q];
-    });
-    // the top layer of cells (k = nz); in the chain also rho*w of the top face
-    // of every column (read by the column kernel, after the horizontal
-    // momenta and the densities of prev are overwritten)
-    launch_box(Box(-1, -1, nz, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
-        const long q = L.ix(i, j, k);
-        if (first) { cc0[q] = pc0[q]; cc1[q] = pc1[q]; }
-        double dt_ = (rt ? cc1[cimg(i, j, k)] : cc1[q]) - sc1[q];
-        extrap[q] = first ? dt_ : dt_ + beta_d * (dt_ - lagged1[q]);
-        lagged1[q] = dt_;
-        if (rt && i >= 0 && i <= nx - 1 && j >= 0 && j <= ny - 1) wtop[L.ix(i, j, -L.ng)] = pw_top(i, j);
-    });
+    // in the chain: rho*w of the top face of every column (read by the column
+    // kernel), before the increments and the densities of prev are overwritten
+    if (rt) {
+        launch_box(Box(0, 0, 0, nx - 1, ny - 1, 0), s,
+                   [=] __device__(int i, int j, int) { wtop[L.ix(i, j, -L.ng)] = pw_top(i, j); });
+    }
 
-
-    // :262-331 horizontal momenta with the terrain-corrected pressure gradient
+    // :139-331 in one launch: theta extrapolated forward, the horizontal momentum
+    // increments of prev (kept in du, dv for the column kernel, because the new
+    // momenta overwrite prev when it aliases data) and the horizontal momenta with
+    // the terrain-corrected pressure gradient.
+    // HBM bound: 17 fields read and 6 (8 in a stage's last substep) written, where
+    // increments and momenta in launches of their own moved 34 (512 x 512 x 96: 1418
+    // us for the two, 1130 us as one).  Each lane marches
+    // up a chunk of KC levels of its (i, j) and forms the extrapolated increment
+    // of its own column and of the columns at i-1 and j-1, kept for levels k-1, k
+    // and k+1 in registers, so every level is read once per chunk (the box order
+    // would put the levels of the gradient's stencil a whole plane of tiles
+    // apart); the columns shared by neighbouring lanes are L2 hits.
     const double* pq1 = prim + PRIM_Q1 * ne;
     const double* pq2 = prim + PRIM_Q2 * ne;
     const double* srx = slow_rhs.xmom;
@@ -195,68 +170,97 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
     double* dym = data.ymom;
     const double* mrx = P.mrx;
     const double* mry = P.mry;
-    // Each lane marches up a chunk of KC levels of its (i, j) and keeps extrap
-    // of its own column and of the columns at i-1 and j-1 for levels k-1, k
-    // and k+1 in registers, so every extrap value is read once per chunk
-    // instead of at three levels (the box order would put the levels of the
-    // gradient's stencil a whole plane of tiles apart).
-    constexpr int KC = 24;
+    const double* drt = first ? pc1 : cc1;
+    const bool store_mom = !ch.active || ch.last;
+    constexpr int KC = 12;   // 512 x 512 x 96: 1147 us at 24 levels, 1130 at 12, 1142 at 8
     const int nch = (nz + KC - 1) / KC;
     launch_box(Box(0, 0, 0, nx, ny, nch - 1), s, [=] __device__(int i, int j, int c) {
         const int k0 = c * KC, k1 = k0 + KC < nz ? k0 + KC : nz;
         const bool xf = j <= ny - 1, yf = i <= nx - 1;
         long q = L.ix(i, j, k0);
-        // c: column (i, j); x: (i-1, j); y: (i, j-1); m / 0 / p: levels k-1 / k / k+1
+        // the cells of the faces as offsets from q: c (i, j), x (i-1, j), y (i, j-1);
+        // in the chain ghost cells are their periodic images
+        const long oc = rt ? (i == nx ? -(long)nx : 0) + (j == ny ? -(long)ny * sy : 0) : 0;
+        const long ox = (rt && i == 0) ? nx - 1 : -1;
+        const long oy = (rt && j == 0) ? (long)(ny - 1) * sy : -sy;
+        auto ext = [&](long a) {
+            const double d = drt[a] - sc1[a];
+            return first ? d : d + beta_d * (d - lagged1[a]);
+        };
+        // m / 0 / p: levels k-1 / k / k+1
         double ecm = 0.0, exm = 0.0, eym = 0.0;
         if (k0 > 0) {
-            ecm = extrap[q - sz];
-            if (xf) exm = extrap[q - 1 - sz];
-            if (yf) eym = extrap[q - sy - sz];
+            ecm = ext(q + oc - sz);
+            if (xf) exm = ext(q + ox - sz);
+            if (yf) eym = ext(q + oy - sz);
         }
-        double ec0 = extrap[q];
-        double ex0 = xf ? extrap[q - 1] : 0.0;
-        double ey0 = yf ? extrap[q - sy] : 0.0;
+        double ec0 = ext(q + oc);
+        double ex0 = xf ? ext(q + ox) : 0.0;
+        double ey0 = yf ? ext(q + oy) : 0.0;
         for (int k = k0; k < k1; ++k, q += sz) {
-            const double ecp = extrap[q + sz];
-            const double exp_ = xf ? extrap[q - 1 + sz] : 0.0;
-            const double eyp = yf ? extrap[q - sy + sz] : 0.0;
+            // the level above the top is a copy of the top one in the chain
+            const long up = (rt && k == nz - 1) ? 0 : sz;
+            const double ecp = ext(q + oc + up);
+            const double exp_ = xf ? ext(q + ox + up) : 0.0;
+            const double eyp = yf ? ext(q + oy + up) : 0.0;
+            // all loads of the level before its first store, which may alias them
+            // as far as the compiler knows (a face outside its box reads inside
+            // the layout; only its stores are guarded)
+            const double sx = sxm[q], sy_ = sym[q], lx = srx[q], ly = sry[q], ax = axm[q], ay = aym[q];
+            const double mx = mrx[q], my = mry[q];
+            const double pc = pi_stage[q], px = pi_stage[q - 1], py = pi_stage[q - sy];
+            double pmx, pmy, rc = 0.0, rx = 0.0, ry = 0.0;
+            if (rt) {
+                pmx = sx + nu[q];
+                pmy = sy_ + nv[q];
+                rc = prho[q + oc]; rx = prho[q + ox]; ry = prho[q + oy];
+            } else {
+                pmx = pxm[q];
+                pmy = pym[q];
+            }
+            const double gp_xi = (ec0 - ex0) * dxi;
+            const double gp_zeta_on_iface = (k == 0)
+                ? 0.5 * dzi * (exp_ + ecp - ex0 - ec0)
+                : 0.25 * dzi * (exp_ + ecp - exm - ecm);
+            double gpx = gp_xi - mx * gp_zeta_on_iface;   // (h_xi / h_zeta) made once
+            const double gp_eta = (ec0 - ey0) * dyi;
+            const double gp_zeta_on_jface = (k == 0)
+                ? 0.5 * dzi * (ecp + eyp - ec0 - ey0)
+                : 0.25 * dzi * (ecp + eyp - ecm - eym);
+            double gpy = gp_eta - my * gp_zeta_on_jface;   // (h_eta / h_zeta) made once
+            if (moist) {
+                gpx /= (1.0 + face_q(pq1, pq2, q, q - 1));
+                gpy /= (1.0 + face_q(pq1, pq2, q, q - sy));
+            }
+            if (rt) {
+                const double d = rc + rx, e = rc + ry;
+                const double u = pmx * 2.0 / d, v = pmy * 2.0 / e;
+                pmx = u * 0.5 * d;
+                pmy = v * 0.5 * e;
+            }
+            const double ix = pmx - sx, iy = pmy - sy_;
+            const double nx_ = ix + dtau * (-Gamma * R_d * (0.5 * (px + pc)) * gpx) + dtau * lx;
+            const double ny_ = iy + dtau * (-Gamma * R_d * (0.5 * (py + pc)) * gpy) + dtau * ly;
             if (xf) {
-                double gp_xi = (ec0 - ex0) * dxi;
-                double gp_zeta_on_iface = (k == 0)
-                    ? 0.5 * dzi * (exp_ + ecp - ex0 - ec0)
-                    : 0.25 * dzi * (exp_ + ecp - exm - ecm);
-                double gpx = gp_xi - mrx[q] * gp_zeta_on_iface;   // (h_xi / h_zeta) made once
-                gpx *= 1.0;
-                if (moist) gpx /= (1.0 + face_q(pq1, pq2, q, q - 1));
-                double pi_c = 0.5 * (pi_stage[q - 1] + pi_stage[q]);
-                double fast_rhs_rho_u = -Gamma * R_d * pi_c * gpx;
-                double n_ = du[q] + dtau * fast_rhs_rho_u + dtau * srx[q];
-                nu[q] = n_;
-                if (k == nz - 1) nu[q + sz] = n_;
-                axm[q] += facinv * n_;
-                dxm[q] = sxm[q] + n_;
+                du[q] = ix;
+                nu[q] = nx_;
+                axm[q] = ax + facinv * nx_;
+                if (store_mom) dxm[q] = sx + nx_;
             }
             if (yf) {
-                double gp_eta = (ec0 - ey0) * dyi;
-                double gp_zeta_on_jface = (k == 0)
-                    ? 0.5 * dzi * (ecp + eyp - ec0 - ey0)
-                    : 0.25 * dzi * (ecp + eyp - ecm - eym);
-                double gpy = gp_eta - mry[q] * gp_zeta_on_jface;   // (h_eta / h_zeta) made once
-                gpy *= 1.0;
-                if (moist) gpy /= (1.0 + face_q(pq1, pq2, q, q - sy));
-                double pi_c = 0.5 * (pi_stage[q - sy] + pi_stage[q]);
-                double fast_rhs_rho_v = -Gamma * R_d * pi_c * gpy;
-                double n_ = dv[q] + dtau * fast_rhs_rho_v + dtau * sry[q];
-                nv[q] = n_;
-                if (k == nz - 1) nv[q + sz] = n_;
-                aym[q] += facinv * n_;
-                dym[q] = sym[q] + n_;
+                dv[q] = iy;
+                nv[q] = ny_;
+                aym[q] = ay + facinv * ny_;
+                if (store_mom) dym[q] = sy_ + ny_;
             }
             ecm = ec0; ec0 = ecp;
             exm = ex0; ex0 = exp_;
             eym = ey0; ey0 = eyp;
         }
     });
+    // the ghost layer of the lagged increment and, in the first substep, of rho
+    // and rho*theta (:139-152), which the chain reads at the images instead
+    if (!ch.active) lagged_shell(P, drt, sc1, lagged1, first ? cc0 : nullptr, pc0, s);
 
     // :414-669, one lane per (i, j) column.  The forward sweep makes, level by
     // level, Omega of the old increments (:460-484) on the face above, the
@@ -267,6 +271,8 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
     // WFromOmega on the interior faces (faces 0 and nz keep the stage value,
     // :620-633), the time-averaged Omega and the rho, rho*theta update (:640-669).
     const Fld fdu{du, L}, fdv{dv, L}, fnu{nu, L}, fnv{nv, L};
+    const double* cr0 = first ? pc0 : cc0;   // rho, rho*theta at the substep's start
+    const double* cr1 = first ? pc1 : cc1;
     const double halfg = fabs(0.5 * (-P.gravity));
     const double* sr0 = slow_rhs.cons;
     const double* sr1 = slow_rhs.cons + ne;
@@ -336,12 +342,13 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
             const long qc = q0 + (long)kc * sz;
             double t0_km1, t1_km1;
             trhs_at(kc, t0_km1, t1_km1);
-            double drho_km1 = cc0[qc] - sc0[qc], drt_km1 = cc1[qc] - sc1[qc];
+            double drho_km1 = cr0[qc] - sc0[qc], drt_km1 = cr1[qc] - sc1[qc];
             double J_km1 = J[qc], s0_km1 = sr0[qc], s1_km1 = sr1[qc];
             double p_km2 = prim[qc - sz], p_km1 = prim[qc];
             double q1_km1 = moist ? pq1[qc] : 0.0, q2_km1 = moist ? pq2[qc] : 0.0;
             double om_km1 = omega_old(kc), om_k = omega_old(kc + 1);
             if (ka == 0) {        // face 0 and cell 0
+                lagged1[q0] = drt_km1;
                 X[lane] = dtau * srz[q0];
                 Z[lane] = fB[q0];
                 omr[0] = om_km1;
@@ -354,7 +361,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
                 if (k > kb) break;
                 const long q = q0 + (long)k * sz;
                 const double Jk = J[q], s0_k = sr0[q], s1_k = sr1[q], p_k = prim[q], p_kp1 = prim[q + sz];
-                const double drho_k = cc0[q] - sc0[q], drt_k = cc1[q] - sc1[q];
+                const double drho_k = cr0[q] - sc0[q], drt_k = cr1[q] - sc1[q];
                 const double q1_k = moist ? pq1[q] : 0.0, q2_k = moist ? pq2[q] : 0.0;
                 const double fP_k = fP[q], fQ_k = fQ[q], srz_k = srz[q], fA_k = fA[q], fB_k = fB[q];
                 const double dw_k = pw(k) - szm[q];
@@ -393,6 +400,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
                 Z[k * 64 + lane] = fB_k;
                 omr[m] = om_k;
                 t0r[m] = t0_k; t1r[m] = t1_k;
+                lagged1[q] = drt_k;
                 tile_level_fence();
                 om_km1 = om_k; om_k = om_kp1;
                 t0_km1 = t0_k; t1_km1 = t1_k;
@@ -447,7 +455,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
                 const double om_lo = Z[k * 64 + lane], om_hi = Z[(k + 1) * 64 + lane];
                 const double szm_k = szm[q], azm_k = azm[q];
                 const double Jq = J[q], pq = prim[q], p_lo = prim[q - sz], p_hi = prim[q + sz];
-                const double sr0_k = sr0[q], sr1_k = sr1[q], cc0_k = cc0[q], cc1_k = cc1[q];
+                const double sr0_k = sr0[q], sr1_k = sr1[q], cc0_k = cr0[q], cc1_k = cr1[q];
                 const double cz_k = (k >= 1) ? szm_k + ((sol + pxr[m]) + pyr[m]) : szm_k;
                 double zflux_lo = beta_2 * sol + beta_1 * om_lo;
                 double zflux_hi = beta_2 * sol_hi + beta_1 * om_hi;
@@ -525,7 +533,8 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         trhs_at(0, t0_km1, t1_km1);
         trhs0[q0] = t0_km1;
         trhs1[q0] = t1_km1;
-        double drho_km1 = cc0[q0] - sc0[q0], drt_km1 = cc1[q0] - sc1[q0];
+        double drho_km1 = cr0[q0] - sc0[q0], drt_km1 = cr1[q0] - sc1[q0];
+        lagged1[q0] = drt_km1;
         double J_km1 = J[q0], s0_km1 = sr0[q0], s1_km1 = sr1[q0];
         double p_km2 = prim[q0 - sz], p_km1 = prim[q0];
         double q1_km1 = moist ? pq1[q0] : 0.0, q2_km1 = moist ? pq2[q0] : 0.0;
@@ -535,7 +544,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         for (int k = 1; k <= nz - 1; ++k) {
             const long q = q0 + (long)k * sz;
             const double Jk = J[q], s0_k = sr0[q], s1_k = sr1[q], p_k = prim[q], p_kp1 = prim[q + sz];
-            const double drho_k = cc0[q] - sc0[q], drt_k = cc1[q] - sc1[q];
+            const double drho_k = cr0[q] - sc0[q], drt_k = cr1[q] - sc1[q];
             const double q1_k = moist ? pq1[q] : 0.0, q2_k = moist ? pq2[q] : 0.0;
             const double fP_k = fP[q], fQ_k = fQ[q], fA_k = fA[q], fB_k = fB[q], srz_k = srz[q];
             const double dw_k = pw(k) - szm[q];
@@ -568,6 +577,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
             trhs0[q] = t0_k;
             trhs1[q] = t1_k;
             soln[q] = s_prev;
+            lagged1[q] = drt_k;
             om_km1 = om_k; om_k = om_kp1;
             t0_km1 = t0_k; t1_km1 = t1_k;
             drho_km1 = drho_k; drt_km1 = drt_k;
@@ -587,7 +597,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
             // loads first, as in the forward sweep
             const double soln_k = soln[q], fCB = fC[q] * fB[q], szm_k = szm[q], om_lo = om[q], azm_k = azm[q];
             const double Jq = J[q], pq = prim[q], p_lo = prim[q - sz], tr0 = trhs0[q], tr1 = trhs1[q];
-            const double sr0_k = sr0[q], sr1_k = sr1[q], cc0_k = cc0[q], cc1_k = cc1[q];
+            const double sr0_k = sr0[q], sr1_k = sr1[q], cc0_k = cr0[q], cc1_k = cr1[q];
             const double sol = soln_k - fCB * sol_hi;
             const double cz_k = (k >= 1) ? szm_k + met::w_from_omega(i, j, k, sol, fnu, fnv, z, dxi, dyi) : szm_k;
             double zflux_lo = beta_2 * sol + beta_1 * om_lo;

@@ -1071,6 +1071,7 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             ch.active = chain;
             ch.rt_prev = chain && ks > 0;
             ch.last = ks == nsub - 1;
+            ch.own_coeffs = true;
             ch.w_lo = P.vel_extdir[2][2];
             ch.w_hi = P.vel_extdir[2][5];
             if (ks == 0) make_fast_coeffs(P, s->fast_coeffs, Sn, s->prim, s->pi_stage, s->r0, s->pi0, dtau, beta_s, st);

@@ -354,30 +354,12 @@ inline void launch_cols(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f, 
     hipLaunchKernelGGL(col_kernel<F>, dim3(gx * gy), dim3((unsigned)width, 1, 1), 0, s, ilo, ihi, jlo, jhi, gx, f);
 }
 
-// ---- column tiles: one work-group of NW waves per 64 columns -------------
+// ---- column tiles: one work-group of 8 waves per 32 or 16 columns ----------
 // For column solves whose per-level work is independent except for a
-// tridiagonal recurrence: the waves split the levels into chunks and form the
-// per-level terms of their chunk in parallel, one wave runs the recurrence
-// over the tile's 64 columns from LDS, and the waves finish their chunks in
-// parallel again.  Lane l of every wave holds column tile * 64 + l of the
-// (i, j) range flattened i fastest (a box narrower than 64 fills the lanes
-// with the next rows), so every level's access of a wave is one contiguous
-// row segment.  The functor is called on all lanes, `valid` false past the
-// range's end, so that every lane reaches the work-group barriers inside it;
-// `lds` holds three arrays of tile_rows<CM, NW>() rows of 64
-// doubles, one value per level and column.
-template <int CM, int NW>
-constexpr int tile_rows() { return NW * CM + 1; }
-template <int CM, int NW, int TC = 64>
-constexpr int tile_lds_doubles() { return 3 * tile_rows<CM, NW>() * TC; }
-// levels per wave chunk for nz levels, and the smallest instantiated CM >= it
-// at 8 waves (0: nz above 96, no tile form: three arrays of 97 rows are
-// 149 KB of the CU's 160 KB of LDS)
-__host__ __device__ inline int tile_chunk(int nz, int nw) { return (nz + nw - 1) / nw; }
-inline int tile_cm8(int nz) {
-    const int c = tile_chunk(nz, 8);
-    return c <= 4 ? 4 : c <= 8 ? 8 : c <= 12 ? 12 : 0;
-}
+// tridiagonal recurrence: the lanes of a column split its levels into chunks,
+// form the per-level terms of their chunk in parallel, pass the recurrence
+// from chunk to chunk and finish their chunks in parallel again.
+__host__ __device__ inline int tile_chunk(int nz, int chunks) { return (nz + chunks - 1) / chunks; }
 // Ends one level of a wave's chunk: keeps the compiler from hoisting the next
 // levels' loads above it (one level of loads per wave covers the latency with
 // the tile's waves in flight, while hoisting several levels exceeds a lane's
@@ -441,124 +423,181 @@ __device__ __forceinline__ void tile_backward(double* X, const double* Y, int nz
     }
 }
 
-// TW = 64: a tile is 64 consecutive columns of the flattened range; TW = 32,
-// 16, 8: a tile is a TW x (64 / TW) block of columns (tiles ordered x
-// fastest), whose lanes then find their j-neighbours in the same tile.  (The
-// column kernels of the substep measure fastest with TW = 64 on 512 x 512 x 96:
-// 2.18 ms against 2.76 ms at 32 x 2 and 2.86 ms at 16 x 4, which fetch 4% and
-// 10% more -- a row segment of TW < 64 doubles spans a cache line more, in
-// proportion, than a whole row does.)
-template <int CM, int NW, int TW, class F>
-__global__ void __launch_bounds__(64 * NW) tile_kernel(int ilo, int ihi, int jlo, int jhi, unsigned nxr,
-                                                       unsigned ncols, unsigned gx, F f) {
-    __shared__ double lds[tile_lds_doubles<CM, NW>()];
-    const unsigned t = xcd_remap(blockIdx.x, gridDim.x);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int i, j;
-    bool valid;
-    if (TW == 64) {
-        const unsigned c = t * 64u + (unsigned)lane;
-        valid = c < ncols;
-        i = ilo + (int)(c % nxr);
-        j = jlo + (int)(c / nxr);
-    } else {
-        i = ilo + (int)((t % gx) * TW) + (lane % TW);
-        j = jlo + (int)((t / gx) * (64 / TW)) + (lane / TW);
-        valid = i <= ihi && j <= jhi;
-    }
-    [[clang::always_inline]] f(i, j, valid, lane, wave, lds);
-}
 template <class F>
 struct TileItem {
     BHdr h;
     F f;
 };
-template <int CM, int NW, class F>
-__global__ void __launch_bounds__(64 * NW) tile_kernel_batch(const TileItem<F>* __restrict__ it,
-                                                             const unsigned* __restrict__ starts, int n) {
-    __shared__ double lds[tile_lds_doubles<CM, NW>()];
+// Relay tiles: a work-group of 8 waves takes TC (32 or 16) consecutive columns
+// of the flattened range and splits their levels into 512 / TC chunks; thread t
+// works on column t % TC in chunk t / TC.  The functor is called on all lanes,
+// `valid` false past the range's end, so that every lane reaches the work-group
+// barriers inside it.  `lds` holds NA arrays of CM values per thread, NX
+// exchange rows of a value per thread, and two carry rows or (CM <= 4) four
+// arrays of a value per face and column.
+template <int CM, int TC>
+constexpr int relay_rows() { return 512 / TC * CM + 1; }
+template <int CM, int TC, int NA, int NX>
+constexpr int relay_lds_doubles() { return (NA * CM + NX) * 512 + (CM <= 4 ? 4 * relay_rows<CM, TC>() : 2) * TC; }
+
+// The tridiagonal solve of a relay tile: rhs, a_k, 1/b_k and c_k of the lane's
+// chunk of `chl` levels in registers; on return rhs holds the solution, x_hi the
+// one on the chunk's upper face and s_top that of face nz (the lanes of the top
+// chunk; r_top, a_top, b_top are its row).  Forward: s_0 = r_0 b_0,
+// s_k = (r_k - a_k s_{k-1}) b_k; backward: x_nz = s_nz,
+// x_k = s_k - (c_k b_k) x_{k+1}: the operation order of a per-column Thomas
+// sweep, so the values are the same.  The elimination is relayed up the chunks
+// and the substitution down them, each lane running its levels and handing one
+// value on (a shuffle within a wave, LDS and a barrier between waves).  Chunks
+// of up to 4 levels stage their rows in LDS instead, where the first chunk's
+// lanes sweep them: a hand-over costs more than a short chunk's levels (64 x 64
+// x 64, two levels per chunk: 18.0 us per launch relayed, 14.4 staged).
+// Every lane of the work-group calls it; `carry` is the LDS after the arrays.
+template <int CM, int TC>
+__device__ __forceinline__ void relay_solve(double* carry, int nz, int chl, int col, bool valid, double (&rhs)[CM],
+                                            const double (&av)[CM], const double (&bv)[CM], double (&cv)[CM],
+                                            double r_top, double a_top, double b_top, double& s_top, double& x_hi) {
+    constexpr int CPW = 64 / TC;               // chunks per wave
+    const int tid = (int)threadIdx.x, wave = tid >> 6, sub = (tid & 63) / TC, chunk = tid / TC;
+    const int ka = chunk * chl;
+    const int kb = (ka + chl < nz ? ka + chl : nz) - 1;
+    const bool has = ka <= kb, top = has && kb == nz - 1;
+    if constexpr (CM <= 4) {
+        double* X = carry;
+        double* Y = X + relay_rows<CM, TC>() * TC;
+        double* Z = Y + relay_rows<CM, TC>() * TC;
+        double* W = Z + relay_rows<CM, TC>() * TC;
+        if (has) {
+#pragma unroll
+            for (int m = 0; m < CM; ++m) {
+                if (ka + m > kb) break;
+                const int r = (ka + m) * TC + col;
+                X[r] = rhs[m]; Y[r] = av[m]; Z[r] = bv[m]; W[r] = cv[m] * bv[m];
+            }
+            if (top) { X[nz * TC + col] = r_top; Y[nz * TC + col] = a_top; Z[nz * TC + col] = b_top; }
+        }
+        __syncthreads();
+        if (chunk == 0 && valid) {
+            tile_forward<TC>(X, Y, Z, nz, col);
+            tile_backward<TC>(X, W, nz, col);
+        }
+        __syncthreads();
+        if (has) {
+#pragma unroll
+            for (int m = 0; m < CM; ++m)
+                if (ka + m <= kb) rhs[m] = X[(ka + m) * TC + col];
+            x_hi = X[(kb + 1) * TC + col];
+            s_top = x_hi;
+        }
+    } else {
+        const int waves = ((nz + chl - 1) / chl + CPW - 1) / CPW;   // waves with levels
+        double s = 0.0;
+        for (int w = 0; w < waves; ++w) {
+            if (wave == w) {
+#pragma unroll
+                for (int u = 0; u < CPW; ++u) {
+                    double in = u == 0 ? (w == 0 ? 0.0 : carry[col]) : __shfl(s, (tid & 63) - TC);
+                    if (sub == u) {
+                        s = in;
+#pragma unroll
+                        for (int m = 0; m < CM; ++m) {
+                            if (ka + m > kb) break;
+                            s = ka + m == 0 ? rhs[m] * bv[m] : (rhs[m] - av[m] * s) * bv[m];
+                            rhs[m] = s;
+                            cv[m] = cv[m] * bv[m];
+                        }
+                        if (top) s_top = (r_top - a_top * s) * b_top;
+                    }
+                }
+                if (sub == CPW - 1) carry[col] = s;
+            }
+            __syncthreads();
+        }
+        x_hi = s_top;
+        for (int w = waves - 1; w >= 0; --w) {
+            if (wave == w) {
+#pragma unroll
+                for (int u = CPW - 1; u >= 0; --u) {
+                    double in = u == CPW - 1 ? carry[TC + col] : __shfl(s, ((tid & 63) + TC) & 63);
+                    if (sub == u && has) {
+                        if (!top) x_hi = in;
+                        s = x_hi;
+#pragma unroll
+                        for (int m = CM - 1; m >= 0; --m) {
+                            if (ka + m > kb) continue;
+                            s = rhs[m] - cv[m] * s;
+                            rhs[m] = s;
+                        }
+                    }
+                }
+                if (sub == 0) carry[TC + col] = s;
+            }
+            __syncthreads();
+        }
+    }
+}
+
+template <int CM, int TC, int NA, int NX, class F>
+__global__ void __launch_bounds__(512) relay_kernel(int ilo, int jlo, unsigned nxr, unsigned ncols, F f) {
+    __shared__ double lds[relay_lds_doubles<CM, TC, NA, NX>()];
+    const unsigned t = xcd_remap(blockIdx.x, gridDim.x);
+    const int col = (int)threadIdx.x % TC, chunk = (int)threadIdx.x / TC;
+    const unsigned c = t * (unsigned)TC + (unsigned)col;
+    const bool valid = c < ncols;
+    const int i = ilo + (int)(c % nxr), j = jlo + (int)(c / nxr);
+    [[clang::always_inline]] f(i, j, valid, col, chunk, lds);
+}
+template <int CM, int TC, int NA, int NX, class F>
+__global__ void __launch_bounds__(512) relay_kernel_batch(const TileItem<F>* __restrict__ it,
+                                                          const unsigned* __restrict__ starts, int n) {
+    __shared__ double lds[relay_lds_doubles<CM, TC, NA, NX>()];
     const unsigned t = xcd_remap(blockIdx.x, gridDim.x);
     const TileItem<F>& m = batch_member(it, starts, n, t);
     const BHdr h = m.h;
     const F& f = m.f;
     const unsigned nxr = (unsigned)(h.hi[0] - h.lo[0] + 1);
     const unsigned ncols = nxr * (unsigned)(h.hi[1] - h.lo[1] + 1);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const unsigned c = (t - h.t0) * 64u + (unsigned)lane;
+    const int col = (int)threadIdx.x % TC, chunk = (int)threadIdx.x / TC;
+    const unsigned c = (t - h.t0) * (unsigned)TC + (unsigned)col;
     const bool valid = c < ncols;
     const int i = h.lo[0] + (int)(c % nxr), j = h.lo[1] + (int)(c / nxr);
-    [[clang::always_inline]] f(i, j, valid, lane, wave, lds);
+    [[clang::always_inline]] f(i, j, valid, col, chunk, lds);
 }
-template <int CM, int NW, class F>
-void launch_tiles_batch(const void* items, const unsigned* starts, int n, unsigned total, unsigned width,
+template <int CM, int TC, int NA, int NX, class F>
+void launch_relay_batch(const void* items, const unsigned* starts, int n, unsigned total, unsigned width,
                         hipStream_t s) {
     (void)width;
-    hipLaunchKernelGGL((tile_kernel_batch<CM, NW, F>), dim3(total), dim3(64 * NW), 0, s,
+    hipLaunchKernelGGL((relay_kernel_batch<CM, TC, NA, NX, F>), dim3(total), dim3(512), 0, s,
                        static_cast<const TileItem<F>*>(items), starts, n);
 }
-// Tiles over the columns (ilo..ihi) x (jlo..jhi); CM >= tile_chunk(nz, NW) of
-// the functor's box.  A recorded (batched) launch always uses flattened tiles.
-template <int CM, int NW, int TW = 64, class F>
-inline void launch_tiles(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f) {
-    static_assert(TW == 64 || TW == 32 || TW == 16 || TW == 8, "tile width");
+template <int CM, int TC, int NA, int NX, class F>
+inline void launch_relay(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f) {
+    static_assert(TC == 16 || TC == 32, "relay tile width");
     const bool ok = ilo <= ihi && jlo <= jhi;
     const unsigned nxr = ok ? (unsigned)(ihi - ilo + 1) : 1u;
-    const unsigned nyr = ok ? (unsigned)(jhi - jlo + 1) : 1u;
-    const unsigned ncols = ok ? nxr * nyr : 0u;
+    const unsigned ncols = ok ? nxr * (unsigned)(jhi - jlo + 1) : 0u;
+    const unsigned tiles = (ncols + TC - 1) / TC;
     if (g_rec) {
-        const unsigned tiles = (ncols + 63u) / 64u;
         TileItem<F> it{{{ilo, jlo, 0}, {ihi, jhi, 0}, 1u, 1u, 0u, tiles}, f};
-        rec_push(&launch_tiles_batch<CM, NW, F>, (unsigned)(64 * NW), it);
+        rec_push(&launch_relay_batch<CM, TC, NA, NX, F>, 512u, it);
         return;
     }
     if (!ok) return;
-    const unsigned gx = (nxr + TW - 1) / TW;
-    const unsigned tiles = TW == 64 ? (ncols + 63u) / 64u : gx * ((nyr + 64 / TW - 1) / (64 / TW));
-    hipLaunchKernelGGL((tile_kernel<CM, NW, TW, F>), dim3(tiles), dim3(64 * NW), 0, s, ilo, ihi, jlo, jhi, nxr,
-                       ncols, gx, f);
+    hipLaunchKernelGGL((relay_kernel<CM, TC, NA, NX, F>), dim3(tiles), dim3(512), 0, s, ilo, jlo, nxr, ncols, f);
 }
-
-// Narrow tiles for boxes of few columns: a work-group of 8 waves takes TC
-// (16 or 32) consecutive columns of the flattened range and splits their
-// levels into 512 / TC chunks; thread t works on column t % TC in chunk
-// t / TC, so the functor sees `lane` = the column within the tile and `wave`
-// = the chunk (chunk 0, the first TC threads, runs the serial sweeps).  The
-// 4,096 columns of a 64 x 64 box make 256 tiles of 16 instead of 64 of 64.
-template <int CM, int TC, class F>
-__global__ void __launch_bounds__(512) tile_kernel_n(int ilo, int jlo, unsigned nxr, unsigned ncols, F f) {
-    __shared__ double lds[tile_lds_doubles<CM, 512 / TC, TC>()];
-    const unsigned t = xcd_remap(blockIdx.x, gridDim.x);
-    const int lane = (int)threadIdx.x % TC, chunk = (int)threadIdx.x / TC;
-    const unsigned c = t * (unsigned)TC + (unsigned)lane;
-    const bool valid = c < ncols;
-    const int i = ilo + (int)(c % nxr), j = jlo + (int)(c / nxr);
-    [[clang::always_inline]] f(i, j, valid, lane, chunk, lds);
-}
-template <int CM, int TC, class F>
-inline void launch_tiles_n(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f) {
-    static_assert(TC == 16 || TC == 32, "narrow tile width");
-    if (ilo > ihi || jlo > jhi) return;
-    const unsigned nxr = (unsigned)(ihi - ilo + 1);
-    const unsigned ncols = nxr * (unsigned)(jhi - jlo + 1);
-    hipLaunchKernelGGL((tile_kernel_n<CM, TC, F>), dim3((ncols + TC - 1) / TC), dim3(512), 0, s, ilo, jlo, nxr, ncols,
-                       f);
-}
-// columns per tile for a box of ncols columns: 64 while that gives every CU a
-// tile, else 32 or 16
+// columns per relay tile for a box of ncols columns: 32 while that gives every
+// CU a tile, else 16 (the 4,096 columns of a 64 x 64 box make 256 tiles of 16)
 inline int tile_columns(long ncols) {
     constexpr long CUS = 256;
-    if ((ncols + 63) / 64 >= CUS) return 64;
-    if ((ncols + 31) / 32 >= CUS) return 32;
-    return 16;
+    return (ncols + 31) / 32 >= CUS ? 32 : 16;
 }
 
 // Variants of the acoustic column kernel (erf_fast_rhs_N): levels of loads
 // kept in flight per lane and work-group width.  Every variant computes the
 // same values; the sim's autotuner times them on the first launches of a run
 // and keeps the fastest.
-// Variant COL_TILE is the tile form (launch_tiles; launch_tiles_n for boxes
-// of few columns, which may have up to 128 levels); COL_FALLBACK for boxes
-// the tile form does not take.
+// Variant COL_TILE is the tile form (launch_relay, up to 128 levels);
+// COL_FALLBACK for boxes the tile form does not take.
 constexpr int COL_NV = ERFX_COL_VARIANTS;
 constexpr int COL_DEPTH[COL_NV] = {2, 3, 4, 2, 3, 4, 2, 3, 4, 0};
 constexpr int COL_WIDTH[COL_NV] = {64, 64, 64, 128, 128, 128, 256, 256, 256, 0};

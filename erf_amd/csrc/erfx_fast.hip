@@ -445,206 +445,218 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
             }
         }
     };
-    // The same column work as a tile of 64 columns per work-group of 8 waves
-    // (launch_tiles), for boxes of up to 96 levels:
-    //  1. each wave takes a chunk of faces k = ka..kb of its 64 columns and forms,
-    //     level by level as the column kernel does, the horizontal divergences of
-    //     cell k and Omega of face k (kept in the lane's registers) and the
-    //     tridiagonal right-hand side of face k, staged in LDS with the face's
-    //     a_k and 1/b_k;
-    //  2. wave 0 runs the elimination up the 64 columns in LDS; the waves then
-    //     stage c_k / b_k and Omega in LDS in place of a_k and 1/b_k, and wave 0
-    //     runs the substitution down the columns;
-    //  3. each wave updates rho*w, the averaged rho*w, rho and rho*theta of its
-    //     chunk's cells from the solution in LDS.
+    // The same column work as a tile of TC (32 or 16) columns per work-group of 8
+    // waves, the levels of a column split into 512 / TC chunks of at most CM, one
+    // lane per chunk and column (launch_relay), for boxes of up to 128 levels:
+    //  1. each lane reads its chunk's levels once and forms, as the column kernel
+    //     does, the horizontal divergences of cell k, Omega of face k + 1 and the
+    //     tridiagonal row of face k; the row of a chunk's first face, which needs
+    //     the cell below, is finished after the chunks have passed each other
+    //     their top cell in LDS;
+    //  2. the elimination is relayed up the chunks and the substitution down them:
+    //     each lane runs its own levels from registers and hands one value to the
+    //     next chunk (chunks of up to 4 levels stage their rows in LDS instead,
+    //     where the first chunk's lanes sweep them);
+    //  3. each lane updates rho*w, the averaged rho*w, rho and rho*theta of its
+    //     cells from what it still holds.
     // Every value is computed by the same expression as in the column kernel, so
-    // the results are bit-identical; the sweep's intermediates never reach HBM,
-    // the per-level loads of a column are spread over 8 waves, and the serial
-    // sweeps read only LDS.
-    const bool implicit_ = implicit;
-    auto tile = [=] __device__(int i, int j, bool valid, int lane, int wave, double* lds, auto cmc, auto tcc) {
+    // the results are bit-identical.  The kernel is HBM bound.  Everything a level
+    // needs later stays in the lane (registers, and four arrays in its own LDS
+    // slots), so each field is read once: the form this replaced (64 columns, 12
+    // levels per wave, rows staged in LDS and swept by one wave, operands read
+    // again for the update) moved 36 fields on 256 x 256 x 80 and took 331 us where
+    // this takes 280; the per-lane form moved 41 on 256 x 256 x 128 and took 503 us
+    // against 394.  With the coefficients of make_fast_coeffs itself
+    // (own_coeffs) a_k and c_k are formed again from P, Q and theta, by the
+    // expressions that made them, instead of being read.
+    const bool own = ch.own_coeffs;
+    const double Dc = dtau * dtau * beta_2 * beta_2 * dzi;
+    auto relay = [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds, auto cmc, auto tcc) {
         constexpr int CM = decltype(cmc)::value;
         constexpr int TC = decltype(tcc)::value;   // columns per tile
-        constexpr int NW = 512 / TC;               // chunks of levels
-        const int ch = tile_chunk(nz, NW);
-        const int ka = wave * ch;
-        const int kb = (ka + ch < nz ? ka + ch : nz) - 1;
-        const bool work = valid && ka <= kb;
+        constexpr int NCH = 512 / TC;              // chunks of levels
+        const int tid = (int)threadIdx.x;
+        const int chl = tile_chunk(nz, NCH);
+        const int ka = chunk * chl;
+        const int kb = (ka + chl < nz ? ka + chl : nz) - 1;
+        const bool has = ka <= kb;
+        const bool work = valid && has;
+        const bool top = has && kb == nz - 1;
         const long q0 = valid ? L.ix(i, j, 0) : 0;
-        constexpr int R = tile_rows<CM, NW>() * TC;
-        double* X = lds;            // right-hand side, then the solution, per face
-        double* Y = lds + R;        // a_k, then c_k / b_k
-        double* Z = lds + 2 * R;    // 1 / b_k, then Omega
-        struct Fw {
-            double P, Q, ws, pkp1, pr, st, prt_, srt_, s0, s1;
-            double dxl, dxh, sxl, sxh, dyl, dyh, syl, syh, pc, pxm, pxp, pym, pyp;
-            double q1, q2;
-        };
-        auto fload = [&](long q, Fw& v) {
-            v.P = Pc[q]; v.Q = Qc[q]; v.ws = slow_rhs.zmom[q];
-            v.pkp1 = prim[q + sz];
-            v.pr = pr0[q];
-            v.st = st0[q]; v.prt_ = prt[q]; v.srt_ = srt[q]; v.s0 = sr0[q]; v.s1 = sr1[q];
-            v.dxl = data.xmom[q]; v.dxh = data.xmom[q + 1]; v.sxl = stage.xmom[q]; v.sxh = stage.xmom[q + 1];
-            v.dyl = data.ymom[q]; v.dyh = data.ymom[q + sy]; v.syl = stage.ymom[q]; v.syh = stage.ymom[q + sy];
-            v.pc = prim[q]; v.pxm = prim[q - 1]; v.pxp = prim[q + 1]; v.pym = prim[q - sy]; v.pyp = prim[q + sy];
-            if (moist) { v.q1 = pq1[q]; v.q2 = pq2[q]; } else { v.q1 = 0.0; v.q2 = 0.0; }
-        };
-        auto hdiv = [&](const Fw& v, double& t0, double& t1) {
-            double xflux_lo = v.dxl - v.sxl;
-            double xflux_hi = v.dxh - v.sxh;
-            double yflux_lo = v.dyl - v.syl;
-            double yflux_hi = v.dyh - v.syh;
-            double pc = v.pc;
-            t0 = (xflux_hi - xflux_lo) * dxi + (yflux_hi - yflux_lo) * dyi;
-            t1 = ((xflux_hi * (pc + v.pxp) - xflux_lo * (pc + v.pxm)) * dxi +
-                  (yflux_hi * (pc + v.pyp) - yflux_lo * (pc + v.pym)) * dyi) * 0.5;
-        };
-        // Omega of the old increments on face kf: prev rho*w (after the round
-        // trip in the substep chain) minus the stage's
-        auto om_face = [&](int kf) -> double {
-            const long qf = q0 + (long)kf * sz;
-            double pzv;
-            if (kf == 0) {
-                pzv = rt ? ch_w_lo * 0.5 * (pr0[q0] + pr0[q0]) : prev.zmom[q0];
-            } else if (!rt) {
-                pzv = prev.zmom[qf];
-            } else if (kf >= nz) {
-                pzv = ch_w_hi * 0.5 * (pr0[qf - sz] + pr0[qf - sz]);
-            } else {
-                double d = pr0[qf] + pr0[qf - sz];
-                double w = prev.zmom[qf] * 2.0 / d;
-                pzv = w * 0.5 * d;
+        // the lane's own LDS slots (array a, level m) and the exchange rows
+        auto slot = [&](int a, int m) -> double& { return lds[(a * CM + m) * 512 + tid]; };
+        auto below = [&](int a) -> double { return lds[(a * CM + chl - 1) * 512 + tid - TC]; };
+        double* xch = lds + 4 * CM * 512;
+        double* carry = xch + 5 * 512;
+        enum { T0 = 0, T1, S0, S1 };
+        double rhs[CM], av[CM], bv[CM], cv[CM], om[CM + 1], prr[CM], ptr_[CM], pp[CM], sz_[CM];
+        double r_top = 0.0, a_top = 0.0, b_top = 0.0, s_top = 0.0;
+        // of the chunk's first cell, until its face's row is finished
+        double f_cP = 0.0, f_cQ = 0.0, f_ws = 0.0, f_drho = 0.0, f_drt = 0.0, f_q1 = 0.0, f_q2 = 0.0;
+        double f_pm2 = 0.0, f_pm1 = 0.0, f_pp1 = 0.0;
+        struct Cell { double drho, drt, s0, s1, t0, t1, q1, q2, om; };   // om: of the cell's lower face
+        // row k of the system: cell k is `c`, the cell below `b`; om_p: Omega of face k + 1
+        auto row = [&](double cP, double cQ, double ws, const Cell& c, const Cell& b, double om_p, double p_km2,
+                       double p_km1, double p_k, double p_kp1, double& a, double& cc) -> double {
+            if (moist) {   // :379-384
+                double qf = 0.5 * (c.q1 + b.q1 + c.q2 + b.q2);
+                cP /= (1.0 + qf);
+                cQ /= (1.0 + qf);
             }
-            return pzv - stage.zmom[qf];
+            double theta_t_lo = 0.5 * (p_km2 + p_km1);
+            double theta_t_mid = 0.5 * (p_km1 + p_k);
+            double theta_t_hi = 0.5 * (p_k + p_kp1);
+            double R0_tmp = cP * c.drt + cQ * b.drt - halfg * (c.drho + b.drho);
+            double R1_tmp = halfg * (-c.s0 - b.s0 + c.t0 + b.t0) +
+                            (cP * (c.s1 - c.t1) + cQ * (b.s1 - b.t1));
+            R1_tmp += beta_1 * dzi * ((om_p - b.om) * halfg
+                                      - (om_p * theta_t_hi - c.om * theta_t_mid) * cP
+                                      - (c.om * theta_t_mid - b.om * theta_t_lo) * cQ);
+            if (own) {
+                a = Dc * (halfg - cQ * theta_t_lo);
+                cc = Dc * (-halfg + cP * theta_t_hi);
+            }
+            return c.om + dtau * (ws + R0_tmp + dtau * beta_2 * R1_tmp);
         };
-        double t0r[CM], t1r[CM], omr[CM + 1];
-        // ---- phase 1: right-hand sides of the chunk's faces ----
+        // ---- phase 1: one reading of the chunk's levels ----
         if (work) {
-            double t0_km1, t1_km1, drho_km1, drt_km1, s0_km1, s1_km1, p_km2, p_km1, p_k, q1_km1, q2_km1;
-            double Om_km1, Om_k;
+            const long qa = q0 + (long)ka * sz;
+            double p_m2 = ka > 1 ? prim[qa - 2 * sz] : prim[q0 - sz], p_m1 = prim[qa - sz], p_k = prim[qa];
+            double pr_k = pr0[qa];
+            double sz_k = stage.zmom[qa];
+            double om_k;
             {
-                const int kc = ka == 0 ? 0 : ka - 1;      // the cell below the chunk's first face
-                Fw c;
-                fload(q0 + (long)kc * sz, c);
-                hdiv(c, t0_km1, t1_km1);
-                drho_km1 = c.pr - c.st;
-                drt_km1 = c.prt_ - c.srt_;
-                s0_km1 = c.s0; s1_km1 = c.s1;
-                p_km2 = prim[q0 + (long)(kc - 1) * sz]; p_km1 = c.pc; p_k = c.pkp1;
-                q1_km1 = c.q1; q2_km1 = c.q2;
-                Om_km1 = om_face(kc);
-                Om_k = om_face(kc + 1);
-                if (ka == 0) {      // face 0: the bottom row (:423-432)
-                    lagged[q0] = drt_km1;
-                    X[lane] = Om_km1 + dtau * c.ws;
-                    Z[lane] = iB[q0];
-                    t0r[0] = t0_km1; t1r[0] = t1_km1; omr[0] = Om_km1;
+                double pz = prev.zmom[qa];
+                if (rt) {
+                    if (ka == 0) {
+                        pz = ch_w_lo * 0.5 * (pr_k + pr_k);
+                    } else {
+                        double d = pr_k + pr0[qa - sz];
+                        double w = pz * 2.0 / d;
+                        pz = w * 0.5 * d;
+                    }
                 }
+                om_k = pz - sz_k;
             }
+            Cell b{};
 #pragma unroll
             for (int m = 0; m < CM; ++m) {
                 const int k = ka + m;
-                if (k == 0) continue;
                 if (k > kb) break;
                 const long q = q0 + (long)k * sz;
-                Fw c;
-                fload(q, c);
-                const double a_k = A[q], b_k = iB[q];
-                double t0_k, t1_k;
-                hdiv(c, t0_k, t1_k);
-                double Om_kp1 = om_face(k + 1);
-                double drho_k = c.pr - c.st;
-                double drt_k = c.prt_ - c.srt_;
-                lagged[q] = drt_k;
-                double coeff_P = c.P, coeff_Q = c.Q;
-                if (moist) {   // :379-384
-                    double qf = 0.5 * (c.q1 + q1_km1 + c.q2 + q2_km1);
-                    coeff_P /= (1.0 + qf);
-                    coeff_Q /= (1.0 + qf);
+                const double ws = slow_rhs.zmom[q], cP = Pc[q], cQ = Qc[q];
+                bv[m] = iB[q];
+                if (!own) { av[m] = A[q]; cv[m] = Cc[q]; }
+                const double p_p = prim[q + sz], pr_p = pr0[q + sz], sz_p = stage.zmom[q + sz];
+                double pz = prev.zmom[q + sz];
+                const double st = st0[q], pt = prt[q], srt_ = srt[q];
+                Cell c;
+                c.s0 = sr0[q]; c.s1 = sr1[q];
+                const double dxl = data.xmom[q], dxh = data.xmom[q + 1], sxl = stage.xmom[q], sxh = stage.xmom[q + 1];
+                const double dyl = data.ymom[q], dyh = data.ymom[q + sy], syl = stage.ymom[q], syh = stage.ymom[q + sy];
+                const double pxm = prim[q - 1], pxp = prim[q + 1], pym = prim[q - sy], pyp = prim[q + sy];
+                c.q1 = 0.0; c.q2 = 0.0;
+                if (moist) { c.q1 = pq1[q]; c.q2 = pq2[q]; }
+                // horizontal flux divergence of the increments (K3)
+                double xflux_lo = dxl - sxl;
+                double xflux_hi = dxh - sxh;
+                double yflux_lo = dyl - syl;
+                double yflux_hi = dyh - syh;
+                c.t0 = (xflux_hi - xflux_lo) * dxi + (yflux_hi - yflux_lo) * dyi;
+                c.t1 = ((xflux_hi * (p_k + pxp) - xflux_lo * (p_k + pxm)) * dxi +
+                        (yflux_hi * (p_k + pyp) - yflux_lo * (p_k + pym)) * dyi) * 0.5;
+                // Omega of the face above
+                if (rt) {
+                    if (k == nz - 1) {
+                        pz = ch_w_hi * 0.5 * (pr_k + pr_k);
+                    } else {
+                        double d = pr_p + pr_k;
+                        double w = pz * 2.0 / d;
+                        pz = w * 0.5 * d;
+                    }
                 }
-                double theta_t_lo = 0.5 * (p_km2 + p_km1);
-                double theta_t_mid = 0.5 * (p_km1 + p_k);
-                double theta_t_hi = 0.5 * (p_k + c.pkp1);
-                double R0_tmp = coeff_P * drt_k + coeff_Q * drt_km1 - halfg * (drho_k + drho_km1);
-                double R1_tmp = halfg * (-c.s0 - s0_km1 + t0_k + t0_km1) +
-                                (coeff_P * (c.s1 - t1_k) + coeff_Q * (s1_km1 - t1_km1));
-                R1_tmp += beta_1 * dzi * ((Om_kp1 - Om_km1) * halfg
-                                          - (Om_kp1 * theta_t_hi - Om_k * theta_t_mid) * coeff_P
-                                          - (Om_k * theta_t_mid - Om_km1 * theta_t_lo) * coeff_Q);
-                X[k * TC + lane] = Om_k + dtau * (c.ws + R0_tmp + dtau * beta_2 * R1_tmp);
-                Y[k * TC + lane] = a_k;
-                Z[k * TC + lane] = b_k;
-                t0r[m] = t0_k; t1r[m] = t1_k; omr[m] = Om_k;
+                const double om_p = pz - sz_p;
+                c.om = om_k;
+                c.drho = pr_k - st;
+                c.drt = pt - srt_;
+                lagged[q] = c.drt;
+                if (m > 0) {
+                    rhs[m] = row(cP, cQ, ws, c, b, om_p, p_m2, p_m1, p_k, p_p, av[m], cv[m]);
+                } else if (k == 0) {   // face 0: the bottom row (:423-432)
+                    rhs[m] = om_k + dtau * ws;
+                    if (own) { av[m] = 0.0; cv[m] = 0.0; }
+                } else {
+                    f_cP = cP; f_cQ = cQ; f_ws = ws; f_drho = c.drho; f_drt = c.drt; f_q1 = c.q1; f_q2 = c.q2;
+                    f_pm2 = p_m2; f_pm1 = p_m1; f_pp1 = p_p;
+                }
+                slot(T0, m) = c.t0; slot(T1, m) = c.t1; slot(S0, m) = c.s0; slot(S1, m) = c.s1;
+                om[m] = om_k; om[m + 1] = om_p;
+                prr[m] = pr_k; ptr_[m] = pt; pp[m] = p_k; sz_[m] = sz_k;
                 tile_level_fence();
-                p_km2 = p_km1; p_km1 = p_k; p_k = c.pkp1;
-                q1_km1 = c.q1; q2_km1 = c.q2;
-                Om_km1 = Om_k; Om_k = Om_kp1;
-                drho_km1 = drho_k; drt_km1 = drt_k;
-                s0_km1 = c.s0; s1_km1 = c.s1;
-                t0_km1 = t0_k; t1_km1 = t1_k;
+                b = c;
+                p_m2 = p_m1; p_m1 = p_k; p_k = p_p;
+                pr_k = pr_p; sz_k = sz_p; om_k = om_p;
             }
-#pragma unroll
-            for (int m = 0; m <= CM; ++m)      // Omega of the face above the chunk
-                if (m == kb - ka + 1) omr[m] = Om_k;
-            if (kb == nz - 1) {                // the top face's row (:423-432)
+            // the top cell, for the chunk above
+            xch[tid] = b.drho; xch[512 + tid] = b.drt; xch[2 * 512 + tid] = b.om;
+            if (moist) { xch[3 * 512 + tid] = b.q1; xch[4 * 512 + tid] = b.q2; }
+            if (top) {                         // the top face's row (:423-432)
                 const long qt = q0 + (long)nz * sz;
-                X[nz * TC + lane] = Om_k + dtau * slow_rhs.zmom[qt];
-                Y[nz * TC + lane] = A[qt];
-                Z[nz * TC + lane] = iB[qt];
+                r_top = om_k + dtau * slow_rhs.zmom[qt];
+                a_top = A[qt];
+                b_top = iB[qt];
             }
         }
         __syncthreads();
-        // ---- phase 2: elimination (wave 0), c_k / b_k and Omega staged, substitution (wave 0) ----
-        if (wave == 0 && valid && implicit_) tile_forward<TC>(X, Y, Z, nz, lane);
-        __syncthreads();
-        if (wave == 0 && valid) {
-            const long qt = q0 + (long)nz * sz;
-            data.zmom[qt] = stage.zmom[qt] + X[nz * TC + lane];
+        if (work && ka > 0) {
+            Cell c, b;
+            b.drho = xch[tid - TC]; b.drt = xch[512 + tid - TC]; b.om = xch[2 * 512 + tid - TC];
+            b.q1 = 0.0; b.q2 = 0.0;
+            if (moist) { b.q1 = xch[3 * 512 + tid - TC]; b.q2 = xch[4 * 512 + tid - TC]; }
+            b.t0 = below(T0); b.t1 = below(T1); b.s0 = below(S0); b.s1 = below(S1);
+            c.drho = f_drho; c.drt = f_drt; c.q1 = f_q1; c.q2 = f_q2; c.om = om[0];
+            c.t0 = slot(T0, 0); c.t1 = slot(T1, 0); c.s0 = slot(S0, 0); c.s1 = slot(S1, 0);
+            rhs[0] = row(f_cP, f_cQ, f_ws, c, b, om[1], f_pm2, f_pm1, pp[0], f_pp1, av[0], cv[0]);
         }
-        if (work) {
+        // what phase 3 reads for the first time, in flight during the sweeps where
+        // the registers allow it: the averaged rho*w, and theta above and below
+        double az[CM], p_top = 0.0, p_bot = 0.0;
+        auto load3 = [&]() {
+            p_top = prim[q0 + (long)(kb + 1) * sz];
+            p_bot = prim[q0 + (long)(ka - 1) * sz];
 #pragma unroll
-            for (int m = 0; m < CM; ++m) {
-                const int k = ka + m;
-                if (k > kb) break;
-                if (implicit_) Y[k * TC + lane] = Cc[q0 + (long)k * sz] * Z[k * TC + lane];
-                Z[k * TC + lane] = omr[m];
-            }
-            if (kb == nz - 1) {
-#pragma unroll
-                for (int m = 0; m <= CM; ++m)
-                    if (m == kb - ka + 1) Z[nz * TC + lane] = omr[m];
-            }
-        }
-        __syncthreads();
-        if (wave == 0 && valid && implicit_) tile_backward<TC>(X, Y, nz, lane);
-        __syncthreads();
+            for (int m = 0; m < CM; ++m)
+                if (ka + m <= kb) az[m] = scratch.zmom[q0 + (long)(ka + m) * sz];
+        };
+        if (CM <= 6 && work) load3();
+        // ---- phase 2: the sweeps ----
+        double x_hi = 0.0;       // the solution on the chunk's upper face
+        relay_solve<CM, TC>(carry, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
         // ---- phase 3: the chunk's cells ----
         if (work) {
+            if (CM > 6) load3();
+            if (top) {
+                const long qt = q0 + (long)nz * sz;
+                data.zmom[qt] = stage.zmom[qt] + s_top;
+            }
 #pragma unroll
             for (int m = 0; m < CM; ++m) {
                 const int k = ka + m;
                 if (k > kb) break;
                 const long q = q0 + (long)k * sz;
-                const double sol = X[k * TC + lane], sol_next = X[(k + 1) * TC + lane];
-                const double szz = stage.zmom[q], azm = scratch.zmom[q];
-                const double pcq = prim[q], p_next = prim[q + sz], pm = prim[q - sz];
-                const double s0 = sr0[q], s1 = sr1[q];
-                const double c0 = step == 0 ? prev.cons[q] : cc0[q];
-                const double c1 = step == 0 ? prev.cons[q + ne] : cc1[q];
-                double drw_k = Z[k * TC + lane], drw_next = Z[(k + 1) * TC + lane];
-                data.zmom[q] = szz + sol;
-                double zflux_lo = beta_2 * sol + beta_1 * drw_k;
-                double zflux_hi = beta_2 * sol_next + beta_1 * drw_next;
-                scratch.zmom[q] = azm + facinv * zflux_lo / (1.0 * 1.0);
+                const bool last = k == kb;
+                const double sol = rhs[m], sol_next = last ? x_hi : rhs[m + 1 < CM ? m + 1 : m];
+                const double pcq = pp[m], p_next = last ? p_top : pp[m + 1 < CM ? m + 1 : m];
+                const double pm = m == 0 ? p_bot : pp[m > 0 ? m - 1 : 0];
+                double zflux_lo = beta_2 * sol + beta_1 * om[m];
+                double zflux_hi = beta_2 * sol_next + beta_1 * om[m + 1];
+                double t0 = slot(T0, m) + dzi * (zflux_hi - zflux_lo);
+                double t1 = slot(T1, m) + 0.5 * dzi * (zflux_hi * (pcq + p_next) - zflux_lo * (pcq + pm));
+                data.zmom[q] = sz_[m] + sol;
+                scratch.zmom[q] = az[m] + facinv * zflux_lo / (1.0 * 1.0);
                 if (k == nz - 1) scratch.zmom[q + sz] += facinv * zflux_hi / (1.0 * 1.0);
-                double t0 = t0r[m] + dzi * (zflux_hi - zflux_lo);
-                double t1 = t1r[m] + 0.5 * dzi * (zflux_hi * (pcq + p_next) - zflux_lo * (pcq + pm));
-                double r_new = c0 + dtau * (s0 - t0);
-                double rt_new = c1 + dtau * (s1 - t1);
-                cc0[q] = r_new;
-                cc1[q] = rt_new;
-                tile_level_fence();
+                cc0[q] = prr[m] + dtau * (slot(S0, m) - t0);
+                cc1[q] = ptr_[m] + dtau * (slot(S1, m) - t1);
             }
         }
     };
@@ -656,48 +668,30 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         var = tag % COL_NV;
         (void)hipEventRecord(P.tuner->ev[2 * tag], s);
     }
-    // the tile form needs nz <= 96; a recorded (batched) launch takes the
-    // largest chunk, so every member of a batch records the same kernel
-    const int cm = tile_cm8(nz) == 0 ? 0 : (g_rec ? 12 : tile_cm8(nz));
-    // 97..128 levels on a box of few columns: the tile form in 32- or
-    // 16-column tiles (three arrays of 129 rows x 32 columns are 99 KB of LDS;
-    // 64 columns would not fit).  A box of many columns keeps the per-lane
-    // form: on the 256 x 256 x 128 CBL the autotuner prefers it to 32-column
-    // tiles.
-    const bool deep = cm == 0 && !g_rec && nz <= 128 && tile_columns((long)nx * ny) < 64;
-    if (var == COL_TILE && cm == 0 && !deep) var = COL_FALLBACK;
+    // The tile form takes up to 128 levels; a recorded (batched) launch up to 96,
+    // always in 32-column tiles of 6 levels per chunk, so every member of a batch
+    // records the same kernel.  It needs the state it updates to be the one it
+    // reads (every substep but a hook's with step > 0 and separate buffers) and
+    // the implicit solve.
+    const bool tiled = implicit && (step == 0 || prev.cons == data.cons) && nz <= (g_rec ? 96 : 128);
+    if (var == COL_TILE && !tiled) var = COL_FALLBACK;
     kt_start(P.timer, KT_FAST_COLUMN, s);
     if (var == COL_TILE) {
-        auto launch = [&](auto cmc) {
-            launch_tiles<decltype(cmc)::value, 8>(0, nx - 1, 0, ny - 1, s,
-                [=] __device__(int i, int j, bool valid, int lane, int wave, double* lds) {
-                    tile(i, j, valid, lane, wave, lds, cmc, std::integral_constant<int, 64>{});
+        auto launch = [&](auto cmc, auto tcc) {
+            launch_relay<decltype(cmc)::value, decltype(tcc)::value, 4, 5>(0, nx - 1, 0, ny - 1, s,
+                [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds) {
+                    relay(i, j, valid, col, chunk, lds, cmc, tcc);
                 });
         };
-        auto launch_n = [&](auto cmc, auto tcc) {
-            launch_tiles_n<decltype(cmc)::value, decltype(tcc)::value>(0, nx - 1, 0, ny - 1, s,
-                [=] __device__(int i, int j, bool valid, int lane, int wave, double* lds) {
-                    tile(i, j, valid, lane, wave, lds, cmc, tcc);
-                });
-        };
+        using IC16 = std::integral_constant<int, 16>;
+        using IC32 = std::integral_constant<int, 32>;
         using IC4 = std::integral_constant<int, 4>;
+        using IC6 = std::integral_constant<int, 6>;
         using IC8 = std::integral_constant<int, 8>;
-        // a box of few columns or of more than 96 levels (a recorded launch
-        // excepted) takes narrow tiles
-        int tc = g_rec ? 64 : tile_columns((long)nx * ny);
-        if (deep && tc > 32) tc = 32;
-        if (tc == 16) {   // 32 chunks: at most 4 levels each up to 128 levels
-            launch_n(IC4{}, std::integral_constant<int, 16>{});
-        } else if (tc == 32) {   // 16 chunks: at most 8 levels each up to 128 levels
-            if (tile_chunk(nz, 16) <= 4) launch_n(IC4{}, std::integral_constant<int, 32>{});
-            else launch_n(IC8{}, std::integral_constant<int, 32>{});
-        } else {
-            switch (cm) {
-                case 4: launch(IC4{}); break;
-                case 8: launch(IC8{}); break;
-                default: launch(std::integral_constant<int, 12>{}); break;
-            }
-        }
+        if (!g_rec && tile_columns((long)nx * ny) == 16) launch(IC4{}, IC16{});   // 32 chunks: at most 4 levels each
+        else if (!g_rec && tile_chunk(nz, 16) <= 4) launch(IC4{}, IC32{});
+        else if (tile_chunk(nz, 16) <= 6) launch(IC6{}, IC32{});
+        else launch(IC8{}, IC32{});
     } else {
         const int width = COL_WIDTH[var];
         switch (COL_DEPTH[var]) {

@@ -62,6 +62,8 @@ struct FastChain {
     // read ghost cells at their images (periodic, foextrap rows)
     bool rt_prev = false;
     bool last = true;      // the stage's last substep
+    // fc is what make_fast_coeffs made for this stage, dtau and beta_s
+    bool own_coeffs = false;
     double w_lo = 0.0, w_hi = 0.0;   // Dirichlet w on the bottom and top faces
 };
 void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erfx_state& slow_rhs,

@@ -285,207 +285,270 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
     double* cz = data.zmom;
     double* azm = scratch.zmom;
     kt_start(P.timer, KT_FAST_COLUMN, s);
-    // The tile form (launch_tiles; the default for boxes of up to 96 levels):
-    // the 8 waves of a 64-column tile form the right-hand sides of their
-    // chunks of faces in parallel and stage them in LDS with a_k and 1/b_k
-    // (Omega and the horizontal divergences stay in registers), wave 0 runs the
-    // elimination in LDS, the waves stage c_k / b_k and Omega, wave 0 runs the
-    // substitution and writes the top face, and the waves update their chunks'
-    // cells.  Every value is the column kernel's expression, so the results are
-    // bit-identical; the serial sweeps read only LDS.
-    auto tile = [=] __device__(int i, int j, bool valid, int lane, int wave, double* lds, auto cmc) {
+    // The tile form (launch_relay; the default for boxes of up to 96 levels), as
+    // the flat grid's: 32 (or 16) columns per work-group of 8 waves, one lane per
+    // column and chunk of levels.  Each lane reads its levels once -- node
+    // heights, increments and theta of a level serve the level above from
+    // registers -- and forms the divergences, Omega, the slope terms and the
+    // tridiagonal rows; the chunks hand their top cell up through LDS; the sweeps
+    // run from registers (short chunks from LDS); and each lane updates its cells
+    // from what it holds.  Every value is the column kernel's expression, so the
+    // results are bit-identical.  HBM bound: the form this replaced (64 columns,
+    // rows swept in LDS, operands read again for the update) moved 49 fields on
+    // 512 x 512 x 96 and took 2105 us where this takes 1464 (1692 with 16-column
+    // tiles, whose rows are one cache line).
+    const bool own = ch.own_coeffs;
+    const double Dc = dtau * dtau * beta_2 * beta_2 * dzi;
+    auto relay = [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds, auto cmc, auto tcc) {
         constexpr int CM = decltype(cmc)::value;
-        constexpr int NW = 8;
-        const int ch = tile_chunk(nz, NW);
-        const int ka = wave * ch;
-        const int kb = (ka + ch < nz ? ka + ch : nz) - 1;
-        const bool work = valid && ka <= kb;
+        constexpr int TC = decltype(tcc)::value;
+        constexpr int NCH = 512 / TC;
+        constexpr int NA = CM > 4 ? 5 : 4;         // arrays in the lane's own LDS slots
+        const int tid = (int)threadIdx.x;
+        const int chl = tile_chunk(nz, NCH);
+        const int ka = chunk * chl;
+        const int kb = (ka + chl < nz ? ka + chl : nz) - 1;
+        const bool has = ka <= kb;
+        const bool work = valid && has;
+        const bool top = has && kb == nz - 1;
         const long q0 = valid ? L.ix(i, j, 0) : 0;
-        constexpr int R = tile_rows<CM, NW>() * 64;
-        double* X = lds;            // right-hand side, then the solution, per face
-        double* Y = lds + R;        // a_k, then c_k / b_k
-        double* Z = lds + 2 * R;    // 1 / b_k, then Omega
-        auto pw = [&](int kf) -> double {
-            const long q = q0 + (long)kf * sz;
+        auto slot = [&](int a, int m) -> double& { return lds[(a * CM + m) * 512 + tid]; };
+        auto below = [&](int a) -> double { return lds[(a * CM + chl - 1) * 512 + tid - TC]; };
+        double* xch = lds + NA * CM * 512;
+        constexpr int NX = NA == 5 ? 9 : 6;        // exchange rows; 6..8 hold this lane's own first cell
+        double* carry = xch + NX * 512;
+        enum { T0 = 0, T1, S0, S1, PX };
+        double rhs[CM], av[CM], bv[CM], cv[CM], om[CM + 1], c0r[CM], c1r[CM], pp[CM], sz_[CM], Jr[CM], pyr[CM];
+        double pxr[NA == 5 ? 1 : CM];
+        double r_top = 0.0, a_top = 0.0, b_top = 0.0, s_top = 0.0;
+        // of the chunk's first cell, until its face's row is finished
+        double f_cP = 0.0, f_cQ = 0.0, f_ws = 0.0, f_dw = 0.0, f_drho = 0.0, f_drt = 0.0, f_q1 = 0.0, f_q2 = 0.0;
+        double f_pm2 = 0.0, f_pm1 = 0.0, f_pp1 = 0.0;
+        struct Cell { double drho, drt, s0, s1, t0, t1, q1, q2, om, J; };   // om: of the cell's lower face
+        // row k of the system (:499-552): cell k is `c`, the cell below `b`; dw the
+        // old rho*w increment, px, py the slope terms of the new increments
+        auto row = [&](double cP, double cQ, double ws, double dw, double px, double py, const Cell& c, const Cell& b,
+                       double om_p, double p_km2, double p_km1, double p_k, double p_kp1, double& a,
+                       double& cc) -> double {
+            const double ofw = (0. - px) - py;
+            double detJ_on_kface = 0.5 * (c.J + b.J);
+            if (moist) {
+                double qf = 0.5 * (c.q1 + b.q1 + c.q2 + b.q2);
+                cP /= (1.0 + qf);
+                cQ /= (1.0 + qf);
+            }
+            double theta_t_lo = 0.5 * (p_km2 + p_km1);
+            double theta_t_mid = 0.5 * (p_km1 + p_k);
+            double theta_t_hi = 0.5 * (p_k + p_kp1);
+            double R0_tmp = (-halfg * c.drho + cP * c.drt) * c.J
+                          + (-halfg * b.drho + cQ * b.drt) * b.J;
+            double R1_tmp = -halfg * (c.s0 * c.J + b.s0 * b.J)
+                          + (cP * c.s1 * c.J + cQ * b.s1 * b.J);
+            R1_tmp += (halfg) * (beta_1 * dzi * (om_p - b.om) + c.t0 + b.t0);
+            R1_tmp += -(cP * (beta_1 * dzi * (om_p * theta_t_hi - c.om * theta_t_mid) + c.t1) +
+                        cQ * (beta_1 * dzi * (c.om * theta_t_mid - b.om * theta_t_lo) + b.t1));
+            if (own) {
+                a = Dc * (halfg - cQ * theta_t_lo);
+                cc = Dc * (-halfg + cP * theta_t_hi);
+            }
+            double r = detJ_on_kface * dw + dtau * (detJ_on_kface * ws + R0_tmp + dtau * beta_2 * R1_tmp);
+            r += detJ_on_kface * ofw;
+            return r;
+        };
+        // nodes of a level: z(i, j), z(i+1, j), z(i, j+1), z(i+1, j+1)
+        struct Nodes { double a, b, c, d; };
+        auto nodes = [&](long q) -> Nodes { return {z.z[q], z.z[q + 1], z.z[q + sy], z.z[q + 1 + sy]}; };
+        auto slope_x = [&](const Nodes& n) { return 0.5 * dxi * (n.d + n.b - n.c - n.a); };   // met::zlo_xi
+        auto slope_y = [&](const Nodes& n) { return 0.5 * dyi * (n.d + n.c - n.b - n.a); };   // met::zlo_eta
+        // prev rho*w on face kf (q its index), with the densities above and below
+        auto pw = [&](int kf, long q, double r_hi, double r_lo) -> double {
             if (!rt) return pzm[q];
             if (kf >= nz) return wtop[L.ix(i, j, -L.ng)];
-            const double d = prho[q] + prho[q - sz];
+            const double d = r_hi + r_lo;
             const double w = pzm[q] * 2.0 / d;
             return w * 0.5 * d;
         };
-        auto omega_old = [&](int kf) -> double {
-            const long q = q0 + (long)kf * sz;
-            if (kf == 0) return 0.;
-            const double dwk = pw(kf) - szm[q];
-            if (kf == nz) return dwk;
-            return met::omega_from_w(i, j, kf, dwk, fdu, fdv, z, dxi, dyi);
-        };
-        auto trhs_at = [&](int k, double& t0, double& t1) {
-            const long q = q0 + (long)k * sz;
-            double h_zeta_cc_xface_hi = 0.5 * dzi * (z(i + 1, j, k + 1) + z(i + 1, j + 1, k + 1) - z(i + 1, j, k) - z(i + 1, j + 1, k));
-            double h_zeta_cc_xface_lo = 0.5 * dzi * (z(i, j, k + 1) + z(i, j + 1, k + 1) - z(i, j, k) - z(i, j + 1, k));
-            double h_zeta_cc_yface_hi = 0.5 * dzi * (z(i, j + 1, k + 1) + z(i + 1, j + 1, k + 1) - z(i, j + 1, k) - z(i + 1, j + 1, k));
-            double h_zeta_cc_yface_lo = 0.5 * dzi * (z(i, j, k + 1) + z(i + 1, j, k + 1) - z(i, j, k) - z(i + 1, j, k));
-            double xflux_lo = nu[q] * h_zeta_cc_xface_lo / 1.0;
-            double xflux_hi = nu[q + 1] * h_zeta_cc_xface_hi / 1.0;
-            double yflux_lo = nv[q] * h_zeta_cc_yface_lo / 1.0;
-            double yflux_hi = nv[q + sy] * h_zeta_cc_yface_hi / 1.0;
-            double mfsq = 1.0 * 1.0;
-            t0 = (xflux_hi - xflux_lo) * dxi * mfsq + (yflux_hi - yflux_lo) * dyi * mfsq;
-            t1 = ((xflux_hi * (prim[q] + prim[q + 1]) - xflux_lo * (prim[q] + prim[q - 1])) * dxi * mfsq +
-                  (yflux_hi * (prim[q] + prim[q + sy]) - yflux_lo * (prim[q] + prim[q - sy])) * dyi * mfsq) * 0.5;
-        };
-        double t0r[CM], t1r[CM], omr[CM + 1], pxr[CM] = {}, pyr[CM] = {};
-        // ---- phase 1: right-hand sides of the chunk's faces ----
+        // ---- phase 1: one reading of the chunk's levels ----
         if (work) {
-            const int kc = ka == 0 ? 0 : ka - 1;      // the cell below the chunk's first face
-            const long qc = q0 + (long)kc * sz;
-            double t0_km1, t1_km1;
-            trhs_at(kc, t0_km1, t1_km1);
-            double drho_km1 = cr0[qc] - sc0[qc], drt_km1 = cr1[qc] - sc1[qc];
-            double J_km1 = J[qc], s0_km1 = sr0[qc], s1_km1 = sr1[qc];
-            double p_km2 = prim[qc - sz], p_km1 = prim[qc];
-            double q1_km1 = moist ? pq1[qc] : 0.0, q2_km1 = moist ? pq2[qc] : 0.0;
-            double om_km1 = omega_old(kc), om_k = omega_old(kc + 1);
-            if (ka == 0) {        // face 0 and cell 0
-                lagged1[q0] = drt_km1;
-                X[lane] = dtau * srz[q0];
-                Z[lane] = fB[q0];
-                omr[0] = om_km1;
-                t0r[0] = t0_km1; t1r[0] = t1_km1;
+            const long qa = q0 + (long)ka * sz;
+            double p_m2 = ka > 1 ? prim[qa - 2 * sz] : prim[q0 - sz], p_m1 = prim[qa - sz], p_k = prim[qa];
+            double c0_k = cr0[qa], sz_k = szm[qa];
+            Nodes zk = nodes(qa);
+            double du0 = du[qa], du1 = du[qa + 1], dv0 = dv[qa], dv1 = dv[qa + sy];
+            double nu0 = 0.0, nu1 = 0.0, nv0 = 0.0, nv1 = 0.0;      // of the level below
+            double dw_k = 0.0, om_k = 0.0;
+            if (ka > 0) {
+                const long ql = qa - sz;
+                nu0 = nu[ql]; nu1 = nu[ql + 1]; nv0 = nv[ql]; nv1 = nv[ql + sy];
+                dw_k = pw(ka, qa, c0_k, rt ? prho[ql] : 0.0) - sz_k;
+                const double uu = 0.25 * (du[ql] + du[ql + 1] + du0 + du1);
+                const double vv = 0.25 * (dv[ql] + dv[ql + sy] + dv0 + dv1);
+                om_k = dw_k - slope_x(zk) * uu - slope_y(zk) * vv;
             }
+            Cell b{};
+            double o_top = 0.0, J_top = 0.0;
 #pragma unroll
             for (int m = 0; m < CM; ++m) {
                 const int k = ka + m;
-                if (k == 0) continue;
                 if (k > kb) break;
                 const long q = q0 + (long)k * sz;
-                const double Jk = J[q], s0_k = sr0[q], s1_k = sr1[q], p_k = prim[q], p_kp1 = prim[q + sz];
-                const double drho_k = cr0[q] - sc0[q], drt_k = cr1[q] - sc1[q];
-                const double q1_k = moist ? pq1[q] : 0.0, q2_k = moist ? pq2[q] : 0.0;
-                const double fP_k = fP[q], fQ_k = fQ[q], srz_k = srz[q], fA_k = fA[q], fB_k = fB[q];
-                const double dw_k = pw(k) - szm[q];
-                const double om_kp1 = omega_old(k + 1);
-                double t0_k, t1_k;
-                trhs_at(k, t0_k, t1_k);
-                // the slope terms of face k with the new increments: Omega of
-                // them here, rho*w from the solution in phase 3 (kept, so the
-                // increments and node heights are read once)
-                double px_k, py_k;
-                met::zface_slope_terms(i, j, k, fnu, fnv, z, dxi, dyi, px_k, py_k);
-                const double ofw = (0. - px_k) - py_k;
-                pxr[m] = px_k; pyr[m] = py_k;
-                double detJ_on_kface = 0.5 * (Jk + J_km1);
-                double coeff_P = fP_k;
-                double coeff_Q = fQ_k;
-                if (moist) {
-                    double qf = 0.5 * (q1_k + q1_km1 + q2_k + q2_km1);
-                    coeff_P /= (1.0 + qf);
-                    coeff_Q /= (1.0 + qf);
+                const double ws = srz[q], cP = fP[q], cQ = fQ[q];
+                bv[m] = fB[q];
+                if (!own) { av[m] = fA[q]; cv[m] = fC[q]; }
+                const double p_p = prim[q + sz], c0_p = cr0[q + sz], sz_p = szm[q + sz];
+                const Nodes zn = nodes(q + sz);
+                const double eu0 = du[q + sz], eu1 = du[q + sz + 1], ev0 = dv[q + sz], ev1 = dv[q + sz + sy];
+                const double mu0 = nu[q], mu1 = nu[q + 1], mv0 = nv[q], mv1 = nv[q + sy];
+                const double c1_k = cr1[q], st0 = sc0[q], st1 = sc1[q];
+                const double pxm = prim[q - 1], pxp = prim[q + 1], pym = prim[q - sy], pyp = prim[q + sy];
+                Cell c;
+                c.s0 = sr0[q]; c.s1 = sr1[q]; c.J = J[q];
+                c.q1 = 0.0; c.q2 = 0.0;
+                if (moist) { c.q1 = pq1[q]; c.q2 = pq2[q]; }
+                const double dw_p = pw(k + 1, q + sz, c0_p, c0_k) - sz_p;
+                // horizontal divergence of the area-weighted new increments (:414-457)
+                double h_xhi = 0.5 * dzi * (zn.b + zn.d - zk.b - zk.d);
+                double h_xlo = 0.5 * dzi * (zn.a + zn.c - zk.a - zk.c);
+                double h_yhi = 0.5 * dzi * (zn.c + zn.d - zk.c - zk.d);
+                double h_ylo = 0.5 * dzi * (zn.a + zn.b - zk.a - zk.b);
+                double xflux_lo = mu0 * h_xlo, xflux_hi = mu1 * h_xhi;
+                double yflux_lo = mv0 * h_ylo, yflux_hi = mv1 * h_yhi;
+                c.t0 = (xflux_hi - xflux_lo) * dxi + (yflux_hi - yflux_lo) * dyi;
+                c.t1 = ((xflux_hi * (p_k + pxp) - xflux_lo * (p_k + pxm)) * dxi +
+                        (yflux_hi * (p_k + pyp) - yflux_lo * (p_k + pym)) * dyi) * 0.5;
+                // Omega of the old increments on the face above (:460-484)
+                double om_p = dw_p;
+                if (k < nz - 1) {
+                    const double uu = 0.25 * (du0 + du1 + eu0 + eu1);
+                    const double vv = 0.25 * (dv0 + dv1 + ev0 + ev1);
+                    om_p = dw_p - slope_x(zn) * uu - slope_y(zn) * vv;
                 }
-                double theta_t_lo = 0.5 * (p_km2 + p_km1);
-                double theta_t_mid = 0.5 * (p_km1 + p_k);
-                double theta_t_hi = 0.5 * (p_k + p_kp1);
-                double R0_tmp = (-halfg * drho_k + coeff_P * drt_k) * Jk
-                              + (-halfg * drho_km1 + coeff_Q * drt_km1) * J_km1;
-                double R1_tmp = -halfg * (s0_k * Jk + s0_km1 * J_km1)
-                              + (coeff_P * s1_k * Jk + coeff_Q * s1_km1 * J_km1);
-                R1_tmp += (halfg) * (beta_1 * dzi * (om_kp1 - om_km1) + t0_k + t0_km1);
-                R1_tmp += -(coeff_P * (beta_1 * dzi * (om_kp1 * theta_t_hi - om_k * theta_t_mid) + t1_k) +
-                            coeff_Q * (beta_1 * dzi * (om_k * theta_t_mid - om_km1 * theta_t_lo) + t1_km1));
-                double rhs = detJ_on_kface * dw_k + dtau * (detJ_on_kface * srz_k + R0_tmp + dtau * beta_2 * R1_tmp);
-                rhs += detJ_on_kface * ofw;
-                X[k * 64 + lane] = rhs;
-                Y[k * 64 + lane] = fA_k;
-                Z[k * 64 + lane] = fB_k;
-                omr[m] = om_k;
-                t0r[m] = t0_k; t1r[m] = t1_k;
-                lagged1[q] = drt_k;
+                c.om = om_k;
+                c.drho = c0_k - st0;
+                c.drt = c1_k - st1;
+                lagged1[q] = c.drt;
+                // the slope terms of the lower face with the new increments
+                double px = 0.0, py = 0.0;
+                if (k > 0) {
+                    px = slope_x(zk) * (0.25 * (nu0 + nu1 + mu0 + mu1));
+                    py = slope_y(zk) * (0.25 * (nv0 + nv1 + mv0 + mv1));
+                }
+                if (m > 0) {
+                    const int l = m > 0 ? m - 1 : 0;
+                    b.t0 = slot(T0, l); b.t1 = slot(T1, l); b.s0 = slot(S0, l); b.s1 = slot(S1, l);
+                    b.om = om[l]; b.J = Jr[l];
+                    rhs[m] = row(cP, cQ, ws, dw_k, px, py, c, b, om_p, p_m2, p_m1, p_k, p_p, av[m], cv[m]);
+                } else if (k == 0) {      // face 0
+                    rhs[m] = dtau * ws;
+                    if (own) { av[m] = 0.0; cv[m] = 0.0; }
+                } else {
+                    if constexpr (NA == 5) {
+                        xch[6 * 512 + tid] = cP; xch[7 * 512 + tid] = cQ; xch[8 * 512 + tid] = ws;
+                    } else {
+                        f_cP = cP; f_cQ = cQ; f_ws = ws;
+                    }
+                    f_dw = dw_k; f_drho = c.drho; f_drt = c.drt;
+                    f_q1 = c.q1; f_q2 = c.q2; f_pm2 = p_m2; f_pm1 = p_m1; f_pp1 = p_p;
+                }
+                slot(T0, m) = c.t0; slot(T1, m) = c.t1; slot(S0, m) = c.s0; slot(S1, m) = c.s1;
+                if constexpr (NA == 5) slot(PX, m) = px; else pxr[m] = px;
+                pyr[m] = py; Jr[m] = c.J;
+                om[m] = om_k; om[m + 1] = om_p;
+                o_top = om_k; J_top = c.J;
+                c0r[m] = c0_k; c1r[m] = c1_k; pp[m] = p_k; sz_[m] = sz_k;
                 tile_level_fence();
-                om_km1 = om_k; om_k = om_kp1;
-                t0_km1 = t0_k; t1_km1 = t1_k;
-                drho_km1 = drho_k; drt_km1 = drt_k;
-                J_km1 = Jk; s0_km1 = s0_k; s1_km1 = s1_k;
-                p_km2 = p_km1; p_km1 = p_k;
-                q1_km1 = q1_k; q2_km1 = q2_k;
+                b.drho = c.drho; b.drt = c.drt; b.q1 = c.q1; b.q2 = c.q2;
+                p_m2 = p_m1; p_m1 = p_k; p_k = p_p;
+                c0_k = c0_p; sz_k = sz_p; om_k = om_p; dw_k = dw_p;
+                zk = zn;
+                du0 = eu0; du1 = eu1; dv0 = ev0; dv1 = ev1;
+                nu0 = mu0; nu1 = mu1; nv0 = mv0; nv1 = mv1;
             }
-#pragma unroll
-            for (int m = 0; m <= CM; ++m)      // Omega of the face above the chunk
-                if (m == kb - ka + 1) omr[m] = om_k;
-            if (kb == nz - 1) {   // the top face: the right-hand side of its elimination step
+            // the top cell, for the chunk above
+            xch[tid] = b.drho; xch[512 + tid] = b.drt; xch[2 * 512 + tid] = o_top; xch[3 * 512 + tid] = J_top;
+            if (moist) { xch[4 * 512 + tid] = b.q1; xch[5 * 512 + tid] = b.q2; }
+            if (top) {   // the top face: the right-hand side of its elimination step
                 const long qt = q0 + (long)nz * sz;
-                X[nz * 64 + lane] = dtau * srz[qt];
-                Y[nz * 64 + lane] = fA[qt];
-                Z[nz * 64 + lane] = fB[qt];
+                r_top = dtau * srz[qt];
+                a_top = fA[qt];
+                b_top = fB[qt];
             }
         }
         __syncthreads();
-        // ---- phase 2: elimination (wave 0), c_k / b_k and Omega staged, substitution (wave 0) ----
-        if (wave == 0 && valid) {
-            tile_forward(X, Y, Z, nz, lane);
-            const long qt = q0 + (long)nz * sz;
-            cz[qt] = szm[qt];
-        }
-        __syncthreads();
-        if (work) {
-#pragma unroll
-            for (int m = 0; m < CM; ++m) {
-                const int k = ka + m;
-                if (k > kb) break;
-                Y[k * 64 + lane] = fC[q0 + (long)k * sz] * Z[k * 64 + lane];
-                Z[k * 64 + lane] = omr[m];
+        if (work && ka > 0) {
+            Cell c, b;
+            b.drho = xch[tid - TC]; b.drt = xch[512 + tid - TC]; b.om = xch[2 * 512 + tid - TC];
+            b.J = xch[3 * 512 + tid - TC];
+            b.q1 = 0.0; b.q2 = 0.0;
+            if (moist) { b.q1 = xch[4 * 512 + tid - TC]; b.q2 = xch[5 * 512 + tid - TC]; }
+            b.t0 = below(T0); b.t1 = below(T1); b.s0 = below(S0); b.s1 = below(S1);
+            c.drho = f_drho; c.drt = f_drt; c.q1 = f_q1; c.q2 = f_q2; c.om = om[0]; c.J = Jr[0];
+            c.t0 = slot(T0, 0); c.t1 = slot(T1, 0); c.s0 = slot(S0, 0); c.s1 = slot(S1, 0);
+            double px;
+            if constexpr (NA == 5) {
+                px = slot(PX, 0);
+                f_cP = xch[6 * 512 + tid]; f_cQ = xch[7 * 512 + tid]; f_ws = xch[8 * 512 + tid];
+            } else {
+                px = pxr[0];
             }
-            if (kb == nz - 1) {
-#pragma unroll
-                for (int m = 0; m <= CM; ++m)
-                    if (m == kb - ka + 1) Z[nz * 64 + lane] = omr[m];
-            }
+            rhs[0] = row(f_cP, f_cQ, f_ws, f_dw, px, pyr[0], c, b, om[1], f_pm2, f_pm1, pp[0], f_pp1, av[0], cv[0]);
         }
-        __syncthreads();
-        if (wave == 0 && valid) tile_backward(X, Y, nz, lane);
-        __syncthreads();
+        // ---- phase 2 ----
+        double x_hi = 0.0;       // the solution on the chunk's upper face
+        relay_solve<CM, TC>(carry, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
         // ---- phase 3: rho*w, the averaged Omega, rho and rho*theta of the chunk ----
         if (work) {
+            if (top) {
+                const long qt = q0 + (long)nz * sz;
+                cz[qt] = szm[qt];
+            }
+            const double p_top = prim[q0 + (long)(kb + 1) * sz], p_bot = prim[q0 + (long)(ka - 1) * sz];
+            double az[CM];
+#pragma unroll
+            for (int m = 0; m < CM; ++m)
+                if (ka + m <= kb) az[m] = azm[q0 + (long)(ka + m) * sz];
 #pragma unroll
             for (int m = 0; m < CM; ++m) {
                 const int k = ka + m;
                 if (k > kb) break;
                 const long q = q0 + (long)k * sz;
-                const double sol = X[k * 64 + lane], sol_hi = X[(k + 1) * 64 + lane];
-                const double om_lo = Z[k * 64 + lane], om_hi = Z[(k + 1) * 64 + lane];
-                const double szm_k = szm[q], azm_k = azm[q];
-                const double Jq = J[q], pq = prim[q], p_lo = prim[q - sz], p_hi = prim[q + sz];
-                const double sr0_k = sr0[q], sr1_k = sr1[q], cc0_k = cr0[q], cc1_k = cr1[q];
-                const double cz_k = (k >= 1) ? szm_k + ((sol + pxr[m]) + pyr[m]) : szm_k;
-                double zflux_lo = beta_2 * sol + beta_1 * om_lo;
-                double zflux_hi = beta_2 * sol_hi + beta_1 * om_hi;
-                double fast_rhs_rho = -(t0r[m] + (zflux_hi - zflux_lo) * dzi) / Jq;
-                double fast_rhs_rhotheta = -(t1r[m] + 0.5 * (zflux_hi * (pq + p_hi) -
-                                                             zflux_lo * (pq + p_lo)) * dzi) / Jq;
+                const bool last = k == kb;
+                const double sol = rhs[m], sol_hi = last ? x_hi : rhs[m + 1 < CM ? m + 1 : m];
+                const double pq = pp[m], p_hi = last ? p_top : pp[m + 1 < CM ? m + 1 : m];
+                const double p_lo = m == 0 ? p_bot : pp[m > 0 ? m - 1 : 0];
+                double px;
+                if constexpr (NA == 5) px = slot(PX, m); else px = pxr[m];
+                const double cz_k = (k >= 1) ? sz_[m] + ((sol + px) + pyr[m]) : sz_[m];
+                double zflux_lo = beta_2 * sol + beta_1 * om[m];
+                double zflux_hi = beta_2 * sol_hi + beta_1 * om[m + 1];
+                double fast_rhs_rho = -(slot(T0, m) + (zflux_hi - zflux_lo) * dzi) / Jr[m];
+                double fast_rhs_rhotheta = -(slot(T1, m) + 0.5 * (zflux_hi * (pq + p_hi) -
+                                                                  zflux_lo * (pq + p_lo)) * dzi) / Jr[m];
                 cz[q] = cz_k;
-                azm[q] = azm_k + facinv * zflux_lo / (1.0 * 1.0);
+                azm[q] = az[m] + facinv * zflux_lo / (1.0 * 1.0);
                 if (k == nz - 1) azm[q + sz] += facinv * zflux_hi / (1.0 * 1.0);
-                cc0[q] = cc0_k + dtau * (sr0_k + fast_rhs_rho);
-                cc1[q] = cc1_k + dtau * (sr1_k + fast_rhs_rhotheta);
-                tile_level_fence();
+                cc0[q] = c0r[m] + dtau * (slot(S0, m) + fast_rhs_rho);
+                cc1[q] = c1r[m] + dtau * (slot(S1, m) + fast_rhs_rhotheta);
             }
         }
     };
-    // a recorded (batched) launch takes the largest chunk, so every member of a
-    // batch records the same kernel
-    const int cm = tile_cm8(nz) == 0 ? 0 : (g_rec ? 12 : tile_cm8(nz));
-    if (cm != 0 && P.col_variant == COL_TILE) {
-        auto launch = [&](auto cmc) {
-            launch_tiles<decltype(cmc)::value, 8>(0, nx - 1, 0, ny - 1, s,
-                [=] __device__(int i, int j, bool valid, int lane, int wave, double* lds) {
-                    tile(i, j, valid, lane, wave, lds, cmc);
+    // a recorded (batched) launch takes chunks of 6 levels in 32-column tiles, so
+    // every member of a batch records the same kernel
+    if (nz <= 96 && P.col_variant == COL_TILE) {
+        auto launch = [&](auto cmc, auto tcc) {
+            constexpr int CM = decltype(cmc)::value;
+            launch_relay<CM, decltype(tcc)::value, (CM > 4 ? 5 : 4), (CM > 4 ? 9 : 6)>(0, nx - 1, 0, ny - 1, s,
+                [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds) {
+                    relay(i, j, valid, col, chunk, lds, cmc, tcc);
                 });
         };
-        switch (cm) {
-            case 4: launch(std::integral_constant<int, 4>{}); break;
-            case 8: launch(std::integral_constant<int, 8>{}); break;
-            default: launch(std::integral_constant<int, 12>{}); break;
-        }
+        using IC16 = std::integral_constant<int, 16>;
+        using IC32 = std::integral_constant<int, 32>;
+        using IC4 = std::integral_constant<int, 4>;
+        using IC6 = std::integral_constant<int, 6>;
+        if (!g_rec && tile_columns((long)nx * ny) == 16) launch(IC4{}, IC16{});   // 32 chunks: at most 3 levels each
+        else if (!g_rec && tile_chunk(nz, 16) <= 4) launch(IC4{}, IC32{});
+        else launch(IC6{}, IC32{});
     } else
     launch_cols(0, nx - 1, 0, ny - 1, s, [=] __device__(int i, int j) {
         const long q0 = L.ix(i, j, 0);

@@ -125,3 +125,24 @@ def test_tile_form_matches_column_form(case):
     assert _same(a, b) == []
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("moist", [False, True])
+@pytest.mark.parametrize("shape", [(24, 20, 9), (24, 20, 33), (41, 23, 128), (96, 96, 16), (97, 95, 65), (96, 96, 97),
+                                   (96, 96, 128)])
+def test_tile_form_chunk_edges(shape, moist):
+    """The tile form where its chunks of levels change: one level per chunk (9
+    and 16 levels), one level past a full set of chunks (33 = 32 + 1 in 16-column
+    tiles, 65 = 16 x 4 + 1 and 97 = 16 x 6 + 1 in 32-column tiles), the largest
+    it takes (128), and a column count that leaves the last tile partial (41 x
+    23, 97 x 95): bit-identical with one lane per column."""
+    case = P.moist_bubble if moist else P.rising_thermal
+    cfg, f = case(*shape, seed=31, adv=C.ADV_UPWIND3)
+    a, b = _pair(cfg, f)
+    a.set_graph(False)
+    a.set_column_variant(7)          # one lane per column
+    a.step(0.0, 0.5, 2)
+    b.step(0.0, 0.5, 2)
+    assert _same(a, b) == []
+    a.close()
+    b.close()

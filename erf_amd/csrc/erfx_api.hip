@@ -678,10 +678,7 @@ int erfx_mlp_create(int capacity, erfx_mlp** out) {
         {(void**)&N.P.w, NPARAM * 4}, {(void**)&N.P.m, NPARAM * 4}, {(void**)&N.P.v, NPARAM * 4},
         {(void**)&N.P.w1b, NI * NH * 2}, {(void**)&N.P.w2b, NH * NH * 2}, {(void**)&N.P.w2tb, NH * NH * 2},
         {(void**)&N.P.w3b, NH * NO * 2},
-        {(void**)&N.T.z1, cap * NH * 4}, {(void**)&N.T.h1, cap * NH * 2}, {(void**)&N.T.z2, cap * NH * 4},
-        {(void**)&N.T.h2, cap * NH * 2}, {(void**)&N.T.dz2, cap * NH * 2}, {(void**)&N.T.dz1, cap * NH * 4},
-        {(void**)&N.T.dy, cap * NO * 4}, {(void**)&N.T.loss, cap * 4},
-        {(void**)&N.ybuf, cap * NO * 4}, {(void**)&N.partial, nblk * NPARAM * 4}, {(void**)&N.loss_dev, 4},
+        {(void**)&N.loss, cap * 4}, {(void**)&N.partial, nblk * NPARAM * 4}, {(void**)&N.loss_dev, 4},
     };
     for (auto& r : req) {
         int rc = balloc(m->allocs, r.p, r.bytes);
@@ -751,7 +748,7 @@ static int mlp_pass(erfx_mlp* m, const float* x, const float* t, int n, bool upd
     // the summed gradient is staged in the partial buffer's last block, past
     // every block a pass of n <= cap samples uses
     float* gstage = grad_host ? N.partial + (size_t)((N.cap + 63) / 64) * mlp::NPARAM : nullptr;
-    mlp_train_pass(N, x, t, n, update, (float)lr, gstage, nullptr);
+    mlp_train_pass(N, x, t, n, update, (float)lr, gstage, loss != nullptr, nullptr);
     int rc = launch_status();
     if (rc) return rc;
     if (grad_host || loss) {

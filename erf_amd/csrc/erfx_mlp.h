@@ -22,8 +22,8 @@ static_assert(NPARAM == 18180, "8-128-128-4 parameter count");
 struct Weights {
     const __bf16* w1;    // [k][u]
     const float* b1;
-    const __bf16* w2;    // [k][u]
-    const __bf16* w2t;   // [u][k]
+    const __bf16* w2;    // rows k, K along u, in operand order (frag)
+    const __bf16* w2t;   // rows u, K along k, in operand order (frag)
     const float* b2;
     const __bf16* w3;    // [u][o]
     const float* b3;
@@ -40,30 +40,26 @@ struct Params_ {
     __bf16* w3b;
 };
 
+// Place of element (row, c) of a 128 x 128 operand stored so that one load of a
+// wave, 16 bytes per lane, is 1 KB on end: tile row / 32 of K-step c / 16 at
+// ((c / 16) * 4 + row / 32) * 512, lane row % 32 + 32 * (c / 8 % 2), element c % 8.
+// (Stored by rows, the 64 lanes of a load touch 64 cache lines.)
+__host__ __device__ __forceinline__ int frag(int row, int c) {
+    return ((c / 16 * 4 + row / 32) * 64 + row % 32 + 32 * (c / 8 % 2)) * 8 + c % 8;
+}
+
 __device__ __forceinline__ void write_bf16_copy(const Params_& pm, int p, float w) {
     const __bf16 b = (__bf16)w;
     if (p < OFF_B1) {
         pm.w1b[p - OFF_W1] = b;
     } else if (p >= OFF_W2 && p < OFF_B2) {
         const int e = p - OFF_W2, k = e / NH, u = e % NH;
-        pm.w2b[e] = b;
-        pm.w2tb[u * NH + k] = b;
+        pm.w2b[frag(k, u)] = b;
+        pm.w2tb[frag(u, k)] = b;
     } else if (p >= OFF_W3 && p < OFF_B3) {
         pm.w3b[p - OFF_W3] = b;
     }
 }
-
-// activations the backward pass reads, per sample
-struct TrainBuf {
-    float* z1;      // [s][NH] pre-activation of layer 1
-    __bf16* h1;     // [s][NH]
-    float* z2;      // [s][NH]
-    __bf16* h2;     // [s][NH]
-    __bf16* dz2;    // [s][NH]
-    float* dz1;     // [s][NH]
-    float* dy;      // [s][NO]
-    float* loss;    // [s] squared error
-};
 
 }  // namespace mlp
 
@@ -71,8 +67,7 @@ struct TrainBuf {
 struct Net {
     mlp::Weights W;
     mlp::Params_ P;
-    mlp::TrainBuf T;
-    float* ybuf = nullptr;      // [cap][NO]
+    float* loss = nullptr;      // [cap] squared error per sample of the last pass
     float* partial = nullptr;   // [(cap + 63) / 64 + 1][NPARAM]
     float* loss_dev = nullptr;  // [1]
     int cap = 0;                // samples per training pass
@@ -87,7 +82,7 @@ struct MlpScaling {
 void mlp_forward(const Net& N, const float* x, float* y, int n, hipStream_t s);
 void mlp_refresh(const Net& N, hipStream_t s);
 void mlp_train_pass(Net& N, const float* x, const float* tgt, int n, bool update, float lr, float* grad_out,
-                    hipStream_t s);
+                    bool want_loss, hipStream_t s);
 
 // erfx_kessler.hip: Kessler's local tendencies as training rows, and the
 // microphysics step with the network (see there)

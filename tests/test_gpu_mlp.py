@@ -142,3 +142,39 @@ def test_forward_throughput_against_matrix_core_peak():
         assert np.linalg.norm(y - yr) / np.linalg.norm(yr) <= 5e-3
         assert tf > 0.0
         net.close()
+
+
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 65, 129, 131073])
+def test_forward_and_gradient_at_tile_edges(n):
+    """Batches at the edges of the 32-sample wave tile and the 64-sample block of
+    the training pass (and, for the forward, just past the batch from which it
+    runs four waves a block): the numpy restatement rounds to BF16 where the GPU
+    does, so what is left is FP32 sums in another order, which flip single BF16
+    roundings of hidden units (half a unit in 2^-8 of one unit in some hundred):
+    the bounds of the tests above."""
+    torch = _torch()
+    from erf_amd.lib import MLP
+    rng = np.random.default_rng(n)
+    p = _params(11)
+    x = (2.0 * rng.normal(0, 1, (n, M.NI))).astype(np.float32)
+    t = rng.normal(0, 1, (n, M.NO)).astype(np.float32)
+    net = MLP(n)
+    net.set_params(p)
+    xd, td = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    yd = torch.full((n + 1, M.NO), 7.0, dtype=torch.float32, device="cuda")
+    net.forward(xd.data_ptr(), yd.data_ptr(), n)
+    torch.cuda.synchronize()
+    y = yd.cpu().numpy().astype(np.float64)
+    assert np.all(y[n] == 7.0)           # nothing past the batch
+    k = min(n, 500)
+    for part in (slice(0, k), slice(n - k, n)):
+        yr, _ = M.forward(p, x[part].astype(np.float64), bf=True)
+        assert np.linalg.norm(y[:n][part] - yr) <= 5e-3 * np.linalg.norm(yr)
+    if n <= 1000:
+        loss, g = net.gradient(xd.data_ptr(), td.data_ptr(), n)
+        lr_, gr = M.loss_and_grad(p, x.astype(np.float64), t.astype(np.float64), bf=True)
+        assert abs(loss - lr_) <= 1e-3 * lr_
+        for a, b in ((M.OFF_W1, M.OFF_B1), (M.OFF_B1, M.OFF_W2), (M.OFF_W2, M.OFF_B2), (M.OFF_B2, M.OFF_W3),
+                     (M.OFF_W3, M.OFF_B3), (M.OFF_B3, M.NPARAM)):
+            assert np.linalg.norm(g[a:b] - gr[a:b]) <= 2e-2 * np.linalg.norm(gr[a:b])
+    net.close()

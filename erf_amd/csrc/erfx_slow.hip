@@ -1512,7 +1512,7 @@ struct PostOp {
     bool dxlo, dxhi, dylo, dyhi;
     const double* mu_h;
     const double* mu_v;
-    int n0, ncons;
+    int n0, ncons, upd_lo, upd_hi;
     const double *ax, *ay, *az;
     double* cur;
     double* nc;
@@ -1538,7 +1538,8 @@ struct PostOp {
         const long q = L.ix(i, j, k);
         const long ne = L.ne, sy = L.sy, sz = L.sz;
         if (copy_slow)
-            for (int c = 2; c < ncons; ++c) cur[q + c * ne] = nc[q + c * ne];
+            for (int c = 2; c < ncons; ++c)
+                if (!(c >= upd_lo && c < upd_hi)) cur[q + c * ne] = nc[q + c * ne];
         for (int m = 0; m < NF; ++m) {
             const int n = n0 + m;
             const double* ps = prim + (n - 1) * ne;
@@ -1569,7 +1570,9 @@ struct PostOp {
 // One block of slow scalars of erf_slow_rhs_post (ERF_slow_rhs_post.cpp:364-497):
 // advection with the time-averaged momenta (AdvectionSrcForScalars), diffusion
 // (DiffusionSrcForState_N), then cur = old + dt * rhs, clipped at 0 for the
-// moisture species.  copy_slow: first copy every slow comp of S_new into cur.
+// moisture species.  copy_slow: first copy the slow comps of S_new into cur that
+// no block updates (those in [upd_lo, upd_hi) are written by their block: copying
+// them too moved 8 fields per stage of a moist step for nothing).
 struct ScalarBlock {
     int n0, ncomp;            // cons comps [n0, n0 + ncomp)
     int ht, vt;               // advection types (a WENO horizontal type also in z)
@@ -1599,6 +1602,7 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
     const double* mu_h = eddy ? eddy + B.mu_h * ne : nullptr;
     const double* mu_v = eddy ? eddy + B.mu_v * ne : nullptr;
     const int n0 = B.n0, nc_b = B.ncomp;
+    const int upd_lo = ERFX_RHOSCALAR, upd_hi = P.moist ? ERFX_RHOQ1 + P.n_qstate : ERFX_RHOSCALAR + 1;
     const bool clip = B.clip;
     const double* ax = scratch.xmom;
     const double* ay = scratch.ymom;
@@ -1630,6 +1634,7 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
             op.copy_slow = copy_slow && m == 0; op.ae = ae; op.slow_dt = slow_dt;
             op.dxlo = dxlo; op.dxhi = dxhi; op.dylo = dylo; op.dyhi = dyhi;
             op.mu_h = mu_h; op.mu_v = mu_v; op.n0 = n0 + m; op.ncons = ncons;
+            op.upd_lo = upd_lo; op.upd_hi = upd_hi;
             op.ax = ax; op.ay = ay; op.az = az; op.cur = cur; op.nc = nc; op.oc = oc; op.crb = crb; op.prim = prim;
             op.dstate = dst;
             launch_march(op, nx, ny, nz, s);
@@ -1657,7 +1662,8 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
         constexpr bool mixed = decltype(mc)::value;
         const long q = L.ix(i, j, k);
         if (copy_slow)
-            for (int c = 2; c < ncons; ++c) cur[q + c * ne] = nc[q + c * ne];
+            for (int c = 2; c < ncons; ++c)
+                if (!(c >= upd_lo && c < upd_hi)) cur[q + c * ne] = nc[q + c * ne];
         double fx0 = ax[q], fx1 = ax[q + 1], fy0 = ay[q], fy1 = ay[q + sy], fz0 = az[q], fz1 = az[q + sz];
         for (int m = 0; m < nc_b; ++m) {
             const int n = n0 + m;

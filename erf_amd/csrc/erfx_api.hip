@@ -1017,7 +1017,7 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
         cl.add(un, uo, (long)ne); cl.add(vn, vo, (long)ne); cl.add(wn, wo, (long)ne);
         copy_fields(cl, st);
     }
-    apply_bcs(P, So, un, vn, wn, P.ng_cons, P.ng_vel, false, true, st);
+    apply_bcs(P, So, un, vn, wn, P.ng_cons, P.ng_vel, false, true, st, true);
     cons_to_prim(P, So.cons, s->prim, s->pi_stage, P.ng_cons, st);
     // MRI: S_new <- S_old (ERF_MRI.H:225-230)
     {

@@ -295,40 +295,288 @@ void velocity_to_momentum(const Params& P, const double* xv, const double* yv, c
     });
 }
 
-// apply_bcs with unsynced momenta on a box periodic in x and y with wall /
-// outflow z faces, in two launches instead of the ~30 of the generic sequence
-// below.  It writes exactly the values that sequence leaves behind
-// (FillIntermediatePatch for rho first, then M2V on the valid faces, the cons
-// fills of the remaining components, the velocity fills, V2M on the box grown
-// by 1 and FillBoundary of the momenta), point for point:
-//   KA  cons ghosts and every velocity the sequence defines, each computed
-//       from valid data (periodic images, same-column values), so no lane
-//       reads a ghost another lane writes;
-//   KB  momenta: V2M where the sequence applies it, the periodic image's V2M
-//       on the FillBoundary layers.
-// Points the sequence does not touch are not written.
-bool fast_bcs_fusable(const Params& P) {
-    if (!P.periodic[0] || !P.periodic[1]) return false;
+// The fused fills: every ghost value the generic sequences below leave behind,
+// computed from valid data alone, so no lane reads a ghost another lane writes
+// and one launch replaces the stages.  What a ghost point holds after
+// FillBoundary, the lateral x fill, the lateral y fill and the vertical fill
+// follows by resolving them in reverse: the vertical row takes the point's value
+// on the nearest level, a point beyond a y face what the y rule reads (its
+// periodic image on a periodic axis), that point's x position likewise.
+bool bcs_fusable(const Params& P) {
+    if (!P.periodic[0] && !P.periodic[1]) return false;
     const int G = P.ng_cons > P.ng_vel ? P.ng_cons : P.ng_vel;
     if (P.L.nx < G + 1 || P.L.ny < G + 1 || P.L.nz < 2 * G) return false;
     for (int v = 0; v < 2; ++v)
         for (int o : {2, 5})
             if (P.bck[v][o] != EXT_DIR && P.bck[v][o] != FOEXTRAP) return false;
     if (P.bck[2][5] != EXT_DIR && P.bck[2][5] != NEUMANN_INT) return false;
+    for (int d = 0; d < 2; ++d) {
+        if (P.periodic[d]) continue;
+        if (P.terrain) return false;
+        for (int o : {d, d + 3})
+            for (int f = 0; f < 4; ++f) {
+                const int t = P.bck[f][o];
+                if (t != EXT_DIR && t != FOEXTRAP && t != REFLECT_EVEN && !(f < 3 && t == REFLECT_ODD) &&
+                    !(f == d && t == NEUMANN_INT))
+                    return false;
+            }
+    }
     return P.cfg.ncons <= 8;
 }
+// periodic in x and y besides: the substeps of a stage can be chained
+bool fast_bcs_fusable(const Params& P) { return P.periodic[0] && P.periodic[1] && bcs_fusable(P); }
 
 struct ConsRows {
-    int r[8];   // foextrap rows filled below and above, per component (lateral reach the same)
+    int r[8];   // ghost cells filled by the lateral rules and the vertical rows, per component
 };
 
-void apply_bcs_periodic(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, int ngc,
-                        int ngv, bool fast_only, hipStream_t s) {
+// Lateral resolution of one box: the rules of each field on the four lateral
+// faces.  Each `*_at` returns the value of a point of valid k at any lateral
+// index, from `base` at valid points.  PER: both axes periodic (the rules drop
+// out at compile time).
+template <bool PER>
+struct LatFill {
+    int nx, ny;
+    bool px, py;
+    int kind[4][6];                          // x-, y-, z-velocity, cons
+    double vel[3][6];
+    double ext[ERFX_NCONS_MOIST][6];
+    static __device__ __forceinline__ int wrap(int a, int n, int hi) { return a < 0 ? a + n : (a > hi ? a - n : a); }
+    // cell-centred along an axis of n cells: moves `a` to the source index, false
+    // for a Dirichlet ghost; `neg` flips the sign (odd reflection)
+    static __device__ __forceinline__ bool cell(int& a, int n, int tl, int th, bool per, bool& neg) {
+        if (PER || per) { a = wrap(a, n, n - 1); return true; }
+        if (a >= 0 && a <= n - 1) return true;
+        const bool lo = a < 0;
+        const int t = lo ? tl : th;
+        if (t == EXT_DIR) return false;
+        if (t == FOEXTRAP) a = lo ? 0 : n - 1;
+        else { a = lo ? -1 - a : 2 * (n - 1) + 1 - a; neg ^= (t == REFLECT_ODD); }
+        return true;
+    }
+    template <class B>
+    __device__ __forceinline__ double cons_at(int n, int i, int j, const B& base) const {
+        bool neg = false;
+        int a = i, b = j;
+        if (!cell(b, ny, kind[3][1], kind[3][4], py, neg)) return j < 0 ? ext[n][1] : ext[n][4];
+        if (!cell(a, nx, kind[3][0], kind[3][3], px, neg)) return i < 0 ? ext[n][0] : ext[n][3];
+        return base(a, b);
+    }
+    // a velocity component along its own axis (faces 0..n) from base(face), which
+    // is evaluated in one place (and once more for the Neumann rule), as it is the
+    // kernel's largest expression; `rules` false: periodic images alone
+    template <class B>
+    static __device__ __forceinline__ double normal(int m, int n, int tl, int th, double vl, double vh, bool per,
+                                                    bool rules, const B& base) {
+        if (PER || per) return base(wrap(m, n, n));
+        bool neu = false, odd = false;
+        int a = m;
+        const bool lo = m <= 0;
+        if (rules && (m <= 0 || m >= n)) {
+            const int t = lo ? tl : th;
+            if (t == EXT_DIR) return lo ? vl : vh;
+            if (t == NEUMANN_INT) { neu = true; a = lo ? 1 : n - 1; }
+            else if (m < 0 || m > n) {
+                a = t == FOEXTRAP ? (lo ? 0 : n) : (lo ? -m : 2 * n - m);
+                odd = t == REFLECT_ODD;
+            }
+        }
+        double v = base(a);
+        if (neu) v = (4.0 * v - base(lo ? 2 : n - 2)) / 3.0;
+        return odd ? -v : v;
+    }
+    template <class B>
+    __device__ __forceinline__ double u_at(int i, int j, bool rules, const B& base) const {
+        bool neg = false;
+        int b = j;
+        if (!cell(b, ny, kind[0][1], kind[0][4], py, neg)) return j < 0 ? vel[0][1] : vel[0][4];
+        const double v = normal(i, nx, kind[0][0], kind[0][3], vel[0][0], vel[0][3], px, rules,
+                                [&](int m) __attribute__((always_inline)) { return base(m, b); });
+        return neg ? -v : v;
+    }
+    template <class B>
+    __device__ __forceinline__ double v_at(int i, int j, bool rules, const B& base) const {
+        // one axis is periodic, so the order of the two rules does not matter
+        bool neg = false;
+        int a = i;
+        if (!cell(a, nx, kind[1][0], kind[1][3], px, neg)) return i < 0 ? vel[1][0] : vel[1][3];
+        const double v = normal(j, ny, kind[1][1], kind[1][4], vel[1][1], vel[1][4], py, rules,
+                                [&](int m) __attribute__((always_inline)) { return base(a, m); });
+        return neg ? -v : v;
+    }
+    template <class B>
+    __device__ __forceinline__ double w_at(int i, int j, const B& base) const {
+        bool neg = false;
+        int a = i, b = j;
+        if (!cell(b, ny, kind[2][1], kind[2][4], py, neg)) return j < 0 ? vel[2][1] : vel[2][4];
+        if (!cell(a, nx, kind[2][0], kind[2][3], px, neg)) return i < 0 ? vel[2][0] : vel[2][3];
+        const double v = base(a, b);
+        return neg ? -v : v;
+    }
+    // whether the face m of a component normal to an axis takes a rule there
+    static __device__ __forceinline__ bool face_rule(int m, int n, int tl, int th, bool per) {
+        if (PER || per) return false;
+        const int t = m == 0 ? tl : th;
+        return (m == 0 || m == n) && (t == EXT_DIR || t == NEUMANN_INT);
+    }
+};
+template <bool PER>
+static LatFill<PER> lat_fill(const Params& P) {
+    LatFill<PER> F;
+    F.nx = P.L.nx; F.ny = P.L.ny; F.px = P.periodic[0]; F.py = P.periodic[1];
+    for (int o = 0; o < 6; ++o) {
+        for (int f = 0; f < 4; ++f) F.kind[f][o] = P.bck[f][o];
+        for (int v = 0; v < 3; ++v) F.vel[v][o] = P.vel_extdir[v][o];
+        for (int n = 0; n < ERFX_NCONS_MOIST; ++n) F.ext[n][o] = P.cons_extdir[n][o];
+    }
+    return F;
+}
+
+// Ghost cells of cons and every velocity the fills define, in one launch.
+//   RAW = false: the velocities are MomentumToVelocity of S's momenta on the
+//   valid faces (ERF_MomentumToVelocity.cpp:24-96), ghosts filled from those;
+//   RAW = true: the velocity arrays hold the valid faces already; only ghosts and
+//   the faces a rule sets are written.
+// ngv: ghost width of the rules and vertical rows; periodic images reach
+// P.ng_vel (P.ng_cons for cons).  Points the sequences do not touch are not
+// written.
+template <bool PER, bool RAW>
+static void fill_points(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, const ConsRows& R,
+                        int rmax, int ngv, hipStream_t s) {
     const Lay L = P.L;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const int ngC = P.ng_cons, ngV = P.ng_vel;
     const int G = ngC > ngV ? ngC : ngV;
-    const long ne = L.ne, sy = L.sy, sz = L.sz;
+    const long ne = L.ne;
+    const int nc = P.cfg.ncons;
+    double* c = S.cons;
+    const double* xm = S.xmom;
+    const double* ym = S.ymom;
+    const double* zm = S.zmom;
+    const LatFill<PER> F = lat_fill<PER>(P);
+    const bool px = PER || P.periodic[0], py = PER || P.periodic[1];
+    const int xtl = P.bck[0][2], xth = P.bck[0][5], ytl = P.bck[1][2], yth = P.bck[1][5];
+    const double xvl = P.vel_extdir[0][2], xvh = P.vel_extdir[0][5];
+    const double yvl = P.vel_extdir[1][2], yvh = P.vel_extdir[1][5];
+    const double zvl = P.vel_extdir[2][2], zvh = P.vel_extdir[2][5];
+    const int zth = P.bck[2][5];
+    const int kz = rmax > ngv ? rmax : (ngv > 1 ? ngv : 1);
+    const Box grown(-G, -G, -kz, nx + G, ny + G, nz - 1 + kz);
+    const bool terr = PER && P.terrain;
+    const Zn zt{P.z_nd, L};
+    const double dxi = P.dxInv[0], dyi = P.dxInv[1];
+    launch_box(grown, s, [=] __device__(int i, int j, int k) {
+        // ghost depth along x and y of the cell and of the x- / y-face
+        const int dxc = i < 0 ? -i : (i > nx - 1 ? i - (nx - 1) : 0), dyc = j < 0 ? -j : (j > ny - 1 ? j - (ny - 1) : 0);
+        const int dxf = i < 0 ? -i : (i > nx ? i - nx : 0), dyf = j < 0 ? -j : (j > ny ? j - ny : 0);
+        const long q = L.ix(i, j, k);
+        const bool kval = k >= 0 && k <= nz - 1;
+        const int depth = k < 0 ? -k : (k > nz - 1 ? k - nz + 1 : 0);   // vertical ghost row
+        // within g of the valid box, reached by periodic images alone
+        auto image = [&](int dx, int dy, int g) { return (dx == 0 || px) && (dy == 0 || py) && dx <= g && dy <= g; };
+        // ---- cons ghosts
+        if (kval && (dxc > 0 || dyc > 0)) {
+            if (image(dxc, dyc, ngC)) {
+                const long src = L.ix(LatFill<PER>::wrap(i, nx, nx - 1), LatFill<PER>::wrap(j, ny, ny - 1), k);
+                for (int n = 0; n < nc; ++n) c[q + n * ne] = c[src + n * ne];
+            } else if (!PER) {
+                for (int n = 0; n < nc; ++n)
+                    if (dxc <= R.r[n] && dyc <= R.r[n])
+                        c[q + n * ne] = F.cons_at(n, i, j, [&](int a, int b) __attribute__((always_inline)) { return c[L.ix(a, b, k) + n * ne]; });
+            }
+        }
+        if (depth > 0) {
+            const int ks = k < 0 ? 0 : nz - 1;
+            for (int n = 0; n < nc; ++n)
+                if (depth <= R.r[n] && dxc <= R.r[n] && dyc <= R.r[n])
+                    c[q + n * ne] = F.cons_at(n, i, j, [&](int a, int b) __attribute__((always_inline)) { return c[L.ix(a, b, ks) + n * ne]; });
+        }
+        // the velocities on valid faces
+        auto rho = [&](int a, int b, int kk) __attribute__((always_inline)) {
+            return F.cons_at(0, a, b, [&](int e, int f) __attribute__((always_inline)) { return c[L.ix(e, f, kk)]; });
+        };
+        auto u_of = [&](int fi, int jj, int kk) __attribute__((always_inline)) {
+            const long f = L.ix(fi, jj, kk);
+            if constexpr (RAW) return xv[f];
+            else return xm[f] * 2.0 / (rho(fi, jj, kk) + rho(fi - 1, jj, kk));
+        };
+        auto v_of = [&](int ii, int fj, int kk) __attribute__((always_inline)) {
+            const long f = L.ix(ii, fj, kk);
+            if constexpr (RAW) return yv[f];
+            else return ym[f] * 2.0 / (rho(ii, fj, kk) + rho(ii, fj - 1, kk));
+        };
+        auto w_of = [&](int ii, int jj, int fk) __attribute__((always_inline)) {
+            const long f = L.ix(ii, jj, fk);
+            if constexpr (RAW) return zv[f];
+            const int kl = fk - 1 < 0 ? 0 : fk - 1, kh = fk > nz - 1 ? nz - 1 : fk;
+            return zm[f] * 2.0 / (rho(ii, jj, kh) + rho(ii, jj, kl));
+        };
+        auto u_lat = [&](int ii, int jj, int kk, bool rules) __attribute__((always_inline)) {
+            return F.u_at(ii, jj, rules, [&](int a, int b) __attribute__((always_inline)) { return u_of(a, b, kk); });
+        };
+        auto v_lat = [&](int ii, int jj, int kk, bool rules) __attribute__((always_inline)) {
+            return F.v_at(ii, jj, rules, [&](int a, int b) __attribute__((always_inline)) { return v_of(a, b, kk); });
+        };
+        auto w_lat = [&](int ii, int jj, int kk) __attribute__((always_inline)) {
+            return F.w_at(ii, jj, [&](int a, int b) __attribute__((always_inline)) { return w_of(a, b, kk); });
+        };
+        const bool lo = k < 0;
+        const int kv = kval ? k : (lo ? 0 : nz - 1);     // the level a vertical row copies
+        // ---- x-velocity: valid faces, images and rule ghosts, vertical rows
+        const bool un = dxf <= ngv && dyc <= ngv;
+        const bool ukeep = RAW && dxf == 0 && dyc == 0 && !LatFill<PER>::face_rule(i, nx, F.kind[0][0], F.kind[0][3], px);
+        if (kval ? !ukeep && (un || image(dxf, dyc, ngV)) : depth <= ngv && un)
+            xv[q] = !kval && (lo ? xtl : xth) == EXT_DIR ? (lo ? xvl : xvh) : u_lat(i, j, kv, un);
+        // ---- y-velocity
+        const bool vn = dxc <= ngv && dyf <= ngv;
+        const bool vkeep = RAW && dxc == 0 && dyf == 0 && !LatFill<PER>::face_rule(j, ny, F.kind[1][1], F.kind[1][4], py);
+        if (kval ? !vkeep && (vn || image(dxc, dyf, ngV)) : depth <= ngv && vn)
+            yv[q] = !kval && (lo ? ytl : yth) == EXT_DIR ? (lo ? yvl : yvh) : v_lat(i, j, kv, vn);
+        // ---- z-velocity (k = 0 takes the zlo value on the valid box grown by ngv)
+        const bool near = dxc <= ngv && dyc <= ngv;
+        const bool plane = near && (k == 0 || k == nz);
+        if (k >= 0 && k <= nz && (near || image(dxc, dyc, ngV)) && !(RAW && dxc == 0 && dyc == 0 && !plane)) {
+            double w;
+            if (terr && plane && (k == 0 || zth == EXT_DIR)) {
+                // terrain wall: WFromOmega with u, v as this launch leaves them
+                auto uf = [&](int ii, int jj, int kk) __attribute__((always_inline)) {
+                    const bool l = kk < 0, in = kk >= 0 && kk <= nz - 1;
+                    return !in && (l ? xtl : xth) == EXT_DIR ? (l ? xvl : xvh)
+                                                             : u_lat(ii, jj, in ? kk : (l ? 0 : nz - 1), true);
+                };
+                auto vf = [&](int ii, int jj, int kk) __attribute__((always_inline)) {
+                    const bool l = kk < 0, in = kk >= 0 && kk <= nz - 1;
+                    return !in && (l ? ytl : yth) == EXT_DIR ? (l ? yvl : yvh)
+                                                             : v_lat(ii, jj, in ? kk : (l ? 0 : nz - 1), true);
+                };
+                w = met::w_from_omega(i, j, k, k == 0 ? zvl : zvh, uf, vf, zt, dxi, dyi);
+            } else if (plane && k == 0) {
+                w = zvl;
+            } else if (plane && zth == EXT_DIR) {
+                w = zvh;
+            } else {
+                w = w_lat(i, j, plane ? nz - 1 : k);   // (beyond `near` only images, where no rule applies)
+                if (plane) w = (4.0 * w - w_lat(i, j, nz - 2)) / 3.0;
+            }
+            zv[q] = w;
+        }
+    });
+}
+
+// apply_bcs on a box with a periodic lateral axis in two launches instead of the
+// ~30 of the generic sequence below, point for point what that leaves behind:
+// fill_points, then the momenta: V2M where the sequence applies it, the periodic
+// image's V2M on the FillBoundary layers.  `synced`: every component's ghosts
+// take part in the one fill (its rho ghosts are valid on entry, as this forms
+// them again).
+template <bool PER>
+static void apply_bcs_fused(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, int ngc,
+                            int ngv, bool fast_only, bool synced, hipStream_t s) {
+    const Lay L = P.L;
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    const int ngC = P.ng_cons, ngV = P.ng_vel;
+    const int G = ngC > ngV ? ngC : ngV;
+    const long sy = L.sy, sz = L.sz;
     const int nc = P.cfg.ncons;
     // rows per component: rho by the first FillIntermediatePatch, the others by the second
     ConsRows R;
@@ -336,143 +584,38 @@ void apply_bcs_periodic(const Params& P, const erfx_state& S, double* xv, double
     const int ncomp2 = fast_only ? 1 : nc - 1;
     int rmax = 0;
     for (int n = 0; n < 8; ++n) {
-        R.r[n] = n == 0 ? ngu1 : (n < 1 + ncomp2 && n < nc ? ngc : 0);
+        R.r[n] = n == 0 ? ngu1 : (n < 1 + ncomp2 && n < nc ? (synced ? ngu1 : ngc) : 0);
         if (R.r[n] > rmax) rmax = R.r[n];
     }
-    double* c = S.cons;
+    fill_points<PER, false>(P, S, xv, yv, zv, R, rmax, ngv, s);
+    const double* c = S.cons;
     double* xm = S.xmom;
     double* ym = S.ymom;
     double* zm = S.zmom;
-    const int xtl = P.bck[0][2], xth = P.bck[0][5], ytl = P.bck[1][2], yth = P.bck[1][5];
-    const double xvl = P.vel_extdir[0][2], xvh = P.vel_extdir[0][5];
-    const double yvl = P.vel_extdir[1][2], yvh = P.vel_extdir[1][5];
-    const double zvl = P.vel_extdir[2][2], zvh = P.vel_extdir[2][5];
-    const int zth = P.bck[2][5];
-    const int kz = rmax > ngv ? rmax : (ngv > 1 ? ngv : 1);
-    const Box grownA(-G, -G, -kz, nx + G, ny + G, nz - 1 + kz);
-    const bool terr = P.terrain;
-    const Zn zt{P.z_nd, L};
-    const double dxi = P.dxInv[0], dyi = P.dxInv[1];
+    const bool px = PER || P.periodic[0], py = PER || P.periodic[1];
     const Box grownB(-G, -G, -1, nx + G, ny + G, nz);
-
-    launch_box(grownA, s, [=] __device__(int i, int j, int k) {
-        // periodic images: cell-centred and face-centred along x / y
-        const int ic = i < 0 ? i + nx : (i > nx - 1 ? i - nx : i);
-        const int jc = j < 0 ? j + ny : (j > ny - 1 ? j - ny : j);
-        const int if_ = i < 0 ? i + nx : (i > nx ? i - nx : i);
-        const int jf = j < 0 ? j + ny : (j > ny ? j - ny : j);
-        const long q = L.ix(i, j, k);
-        const bool kval = k >= 0 && k <= nz - 1;
-        const int depth = k < 0 ? -k : (k > nz - 1 ? k - nz + 1 : 0);   // vertical ghost row
-        // ---- cons ghosts
-        if (kval && (i < 0 || i > nx - 1 || j < 0 || j > ny - 1) && i >= -ngC && i <= nx - 1 + ngC &&
-            j >= -ngC && j <= ny - 1 + ngC) {
-            const long src = L.ix(ic, jc, k);
-            for (int n = 0; n < nc; ++n) c[q + n * ne] = c[src + n * ne];
-        }
-        if (depth > 0) {
-            const long src = L.ix(ic, jc, k < 0 ? 0 : nz - 1);
-            for (int n = 0; n < nc; ++n) {
-                const int rr = R.r[n];
-                if (depth <= rr && i >= -rr && i <= nx - 1 + rr && j >= -rr && j <= ny - 1 + rr)
-                    c[q + n * ne] = c[src + n * ne];
-            }
-        }
-        // rho after the fills at a cell of valid k (any lateral index)
-        auto rho_v = [&](int ii, int jj, int kk) {
-            int a = ii < 0 ? ii + nx : (ii > nx - 1 ? ii - nx : ii);
-            int b = jj < 0 ? jj + ny : (jj > ny - 1 ? jj - ny : jj);
-            return c[L.ix(a, b, kk)];
-        };
-        // M2V of a valid face (ERF_MomentumToVelocity.cpp:24-96)
-        auto u_of = [&](int fi, int jj, int kk) {
-            long f = L.ix(fi, jj, kk);
-            return xm[f] * 2.0 / (rho_v(fi, jj, kk) + rho_v(fi - 1, jj, kk));
-        };
-        auto v_of = [&](int ii, int fj, int kk) {
-            long f = L.ix(ii, fj, kk);
-            return ym[f] * 2.0 / (rho_v(ii, fj, kk) + rho_v(ii, fj - 1, kk));
-        };
-        auto w_of = [&](int ii, int jj, int fk) {
-            long f = L.ix(ii, jj, fk);
-            int kl = fk - 1 < 0 ? 0 : fk - 1, kh = fk > nz - 1 ? nz - 1 : fk;
-            return zm[f] * 2.0 / (rho_v(ii, jj, kh) + rho_v(ii, jj, kl));
-        };
-        // ---- x-velocity: valid faces, FillBoundary layers, vertical ghost rows
-        if (kval && i >= -ngV && i <= nx + ngV && j >= -ngV && j <= ny - 1 + ngV) {
-            xv[q] = u_of(if_, jc, k);
-        } else if (depth > 0 && depth <= ngv && i >= -ngv && i <= nx + ngv && j >= -ngv && j <= ny - 1 + ngv) {
-            bool lo = k < 0;
-            int t = lo ? xtl : xth;
-            xv[q] = t == EXT_DIR ? (lo ? xvl : xvh) : u_of(if_, jc, lo ? 0 : nz - 1);
-        }
-        // ---- y-velocity
-        if (kval && i >= -ngV && i <= nx - 1 + ngV && j >= -ngV && j <= ny + ngV) {
-            yv[q] = v_of(ic, jf, k);
-        } else if (depth > 0 && depth <= ngv && i >= -ngv && i <= nx - 1 + ngv && j >= -ngv && j <= ny + ngv) {
-            bool lo = k < 0;
-            int t = lo ? ytl : yth;
-            yv[q] = t == EXT_DIR ? (lo ? yvl : yvh) : v_of(ic, jf, lo ? 0 : nz - 1);
-        }
-        // ---- z-velocity (k = 0 takes the zlo value on the valid box grown by ngv)
-        if (k >= 0 && k <= nz && i >= -ngV && i <= nx - 1 + ngV && j >= -ngV && j <= ny - 1 + ngV) {
-            const bool near = i >= -ngv && i <= nx - 1 + ngv && j >= -ngv && j <= ny - 1 + ngv;
-            double w;
-            if (terr && near && (k == 0 || (k == nz && zth == EXT_DIR))) {
-                // terrain wall: WFromOmega with u, v as this launch leaves them
-                // (the x / y branches above, evaluated again here)
-                auto uf = [&](int ii, int jj, int kk) {
-                    const int fi = ii < 0 ? ii + nx : (ii > nx ? ii - nx : ii);
-                    const int cj = jj < 0 ? jj + ny : (jj > ny - 1 ? jj - ny : jj);
-                    if (kk >= 0 && kk <= nz - 1) return u_of(fi, cj, kk);
-                    const bool lo = kk < 0;
-                    return (lo ? xtl : xth) == EXT_DIR ? (lo ? xvl : xvh) : u_of(fi, cj, lo ? 0 : nz - 1);
-                };
-                auto vf = [&](int ii, int jj, int kk) {
-                    const int ci = ii < 0 ? ii + nx : (ii > nx - 1 ? ii - nx : ii);
-                    const int fj = jj < 0 ? jj + ny : (jj > ny ? jj - ny : jj);
-                    if (kk >= 0 && kk <= nz - 1) return v_of(ci, fj, kk);
-                    const bool lo = kk < 0;
-                    return (lo ? ytl : yth) == EXT_DIR ? (lo ? yvl : yvh) : v_of(ci, fj, lo ? 0 : nz - 1);
-                };
-                w = met::w_from_omega(i, j, k, k == 0 ? zvl : zvh, uf, vf, zt, dxi, dyi);
-            } else if (near && k == 0) w = zvl;
-            else if (near && k == nz && zth == EXT_DIR) w = zvh;
-            else if (near && k == nz) w = (4.0 * w_of(ic, jc, nz - 1) - w_of(ic, jc, nz - 2)) / 3.0;
-            else w = w_of(ic, jc, k);
-            zv[q] = w;
-        }
-    });
-
     launch_box(grownB, s, [=] __device__(int i, int j, int k) {
-        const int ic = i < 0 ? i + nx : (i > nx - 1 ? i - nx : i);
-        const int jc = j < 0 ? j + ny : (j > ny - 1 ? j - ny : j);
-        const int if_ = i < 0 ? i + nx : (i > nx ? i - nx : i);
-        const int jf = j < 0 ? j + ny : (j > ny ? j - ny : j);
+        const int dxc = i < 0 ? -i : (i > nx - 1 ? i - (nx - 1) : 0), dyc = j < 0 ? -j : (j > ny - 1 ? j - (ny - 1) : 0);
+        const int dxf = i < 0 ? -i : (i > nx ? i - nx : 0), dyf = j < 0 ? -j : (j > ny ? j - ny : 0);
         const long q = L.ix(i, j, k);
         const bool kval = k >= 0 && k <= nz - 1;
+        const int ic = px ? LatFill<PER>::wrap(i, nx, nx - 1) : i, jc = py ? LatFill<PER>::wrap(j, ny, ny - 1) : j;
+        const int if_ = px ? LatFill<PER>::wrap(i, nx, nx) : i, jf = py ? LatFill<PER>::wrap(j, ny, ny) : j;
+        // a FillBoundary layer: beyond the valid box, reached by periodic images alone
+        auto image = [&](int dx, int dy) {
+            return (dx > 0 || dy > 0) && (dx == 0 || px) && (dy == 0 || py) && dx <= ngV && dy <= ngV;
+        };
         // VelocityToMomentum (ERF_VelocityToMomentum.cpp:24-114) at face index f
         auto xm_at = [&](long f) { return xv[f] * 0.5 * (c[f] + c[f - 1]); };
         auto ym_at = [&](long f) { return yv[f] * 0.5 * (c[f] + c[f - sy]); };
         auto zm_at = [&](long f) { return zv[f] * 0.5 * (c[f] + c[f - sz]); };
-        // x-momentum: FillBoundary layers take the image's V2M
-        if (kval && (i < 0 || i > nx || j < 0 || j > ny - 1) && i >= -ngV && i <= nx + ngV && j >= -ngV &&
-            j <= ny - 1 + ngV) {
-            xm[q] = xm_at(L.ix(if_, jc, k));
-        } else if (i >= -1 && i <= nx + 1 && j >= -1 && j <= ny && k >= -1 && k <= nz) {
-            xm[q] = xm_at(q);
-        }
-        if (kval && (i < 0 || i > nx - 1 || j < 0 || j > ny) && i >= -ngV && i <= nx - 1 + ngV && j >= -ngV &&
-            j <= ny + ngV) {
-            ym[q] = ym_at(L.ix(ic, jf, k));
-        } else if (i >= -1 && i <= nx && j >= -1 && j <= ny + 1 && k >= -1 && k <= nz) {
-            ym[q] = ym_at(q);
-        }
-        if (k >= 0 && k <= nz && (i < 0 || i > nx - 1 || j < 0 || j > ny - 1) && i >= -ngV && i <= nx - 1 + ngV &&
-            j >= -ngV && j <= ny - 1 + ngV) {
-            zm[q] = zm_at(L.ix(ic, jc, k));
-        } else if (i >= -1 && i <= nx && j >= -1 && j <= ny && k >= 0 && k <= nz) {
-            zm[q] = zm_at(q);
+        if (kval && image(dxf, dyc)) xm[q] = xm_at(L.ix(if_, jc, k));
+        else if (dxf <= 1 && dyc <= 1 && k >= -1 && k <= nz) xm[q] = xm_at(q);
+        if (kval && image(dxc, dyf)) ym[q] = ym_at(L.ix(ic, jf, k));
+        else if (dxc <= 1 && dyf <= 1 && k >= -1 && k <= nz) ym[q] = ym_at(q);
+        if (k >= 0 && k <= nz) {
+            if (image(dxc, dyc)) zm[q] = zm_at(L.ix(ic, jc, k));
+            else if (dxc <= 1 && dyc <= 1) zm[q] = zm_at(q);
         }
     });
 }
@@ -496,9 +639,12 @@ void fill_intermediate_patch(const Params& P, const erfx_state& S, double* xv, d
 
 // apply_bcs (Source/TimeIntegration/ERF_TI_utils.H:53-150).
 void apply_bcs(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, int ngc, int ngv,
-               bool fast_only, bool synced, hipStream_t s) {
-    if (!synced && ngc >= 1 && ngv >= 1 && fast_bcs_fusable(P)) {
-        apply_bcs_periodic(P, S, xv, yv, zv, ngc, ngv, fast_only, s);
+               bool fast_only, bool synced, hipStream_t s, bool filled) {
+    // synced: the sequence reads the density ghosts as they are, which the fused
+    // form forms again: the same where the caller says that they are filled
+    if ((!synced || filled) && ngc >= 1 && ngv >= 1 && bcs_fusable(P)) {
+        if (P.periodic[0] && P.periodic[1]) apply_bcs_fused<true>(P, S, xv, yv, zv, ngc, ngv, fast_only, synced, s);
+        else apply_bcs_fused<false>(P, S, xv, yv, zv, ngc, ngv, fast_only, synced, s);
         return;
     }
     int scomp, ncomp, ngu;
@@ -520,6 +666,14 @@ void apply_bcs(const Params& P, const erfx_state& S, double* xv, double* yv, dou
 
 // ERF::FillPatch, level 0 at the old time (ERF_FillPatch.cpp:19-140).
 void fill_patch(const Params& P, double* c, double* u, double* v, double* w, hipStream_t s) {
+    if (bcs_fusable(P)) {
+        const erfx_state S{c, nullptr, nullptr, nullptr};
+        ConsRows R;
+        for (int n = 0; n < 8; ++n) R.r[n] = n < P.cfg.ncons ? P.ng_cons : 0;
+        if (P.periodic[0] && P.periodic[1]) fill_points<true, true>(P, S, u, v, w, R, P.ng_cons, P.ng_vel, s);
+        else fill_points<false, true>(P, S, u, v, w, R, P.ng_cons, P.ng_vel, s);
+        return;
+    }
     fill_cons(P, c, 0, P.cfg.ncons, P.ng_cons, s);
     fill_xvel(P, u, P.ng_vel, s);
     fill_yvel(P, v, P.ng_vel, s);

@@ -20,7 +20,7 @@ void velocity_to_momentum(const Params& P, const double* xv, const double* yv, c
 void fill_intermediate_patch(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv,
                              int ngc, int ngv, bool cons_only, int icomp, int ncomp, hipStream_t s);
 void apply_bcs(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, int ngc, int ngv,
-               bool fast_only, bool synced, hipStream_t s);
+               bool fast_only, bool synced, hipStream_t s, bool filled = false);
 void fill_patch(const Params& P, double* c, double* u, double* v, double* w, hipStream_t s);
 void cons_to_prim(const Params& P, const double* c, double* prim, double* pi_stage, int ng, hipStream_t s);
 

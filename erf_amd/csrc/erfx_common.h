@@ -537,10 +537,21 @@ __device__ __forceinline__ void relay_solve(double* carry, int nz, int chl, int 
     }
 }
 
-template <int CM, int TC, int NA, int NX, class F>
-__global__ void __launch_bounds__(512) relay_kernel(int ilo, int jlo, unsigned nxr, unsigned ncols, F f) {
+// `extra(n)` runs on the lanes of the work-groups past the tiles, n from 0: work
+// of the same launch that touches nothing the tiles read or write.
+struct NoExtra {
+    static constexpr bool ANY = false;
+    __device__ void operator()(unsigned) const {}
+};
+template <int CM, int TC, int NA, int NX, class F, class X>
+__global__ void __launch_bounds__(512) relay_kernel(int ilo, int jlo, unsigned nxr, unsigned ncols, unsigned tiles, F f,
+                                                    X extra) {
     __shared__ double lds[relay_lds_doubles<CM, TC, NA, NX>()];
-    const unsigned t = xcd_remap(blockIdx.x, gridDim.x);
+    if (X::ANY && blockIdx.x >= tiles) {
+        extra((blockIdx.x - tiles) * 512u + threadIdx.x);
+        return;
+    }
+    const unsigned t = xcd_remap(blockIdx.x, tiles);
     const int col = (int)threadIdx.x % TC, chunk = (int)threadIdx.x / TC;
     const unsigned c = t * (unsigned)TC + (unsigned)col;
     const bool valid = c < ncols;
@@ -570,8 +581,8 @@ void launch_relay_batch(const void* items, const unsigned* starts, int n, unsign
     hipLaunchKernelGGL((relay_kernel_batch<CM, TC, NA, NX, F>), dim3(total), dim3(512), 0, s,
                        static_cast<const TileItem<F>*>(items), starts, n);
 }
-template <int CM, int TC, int NA, int NX, class F>
-inline void launch_relay(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f) {
+template <int CM, int TC, int NA, int NX, class F, class X = NoExtra>
+inline void launch_relay(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f, unsigned nextra = 0, X extra = X()) {
     static_assert(TC == 16 || TC == 32, "relay tile width");
     const bool ok = ilo <= ihi && jlo <= jhi;
     const unsigned nxr = ok ? (unsigned)(ihi - ilo + 1) : 1u;
@@ -583,7 +594,8 @@ inline void launch_relay(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f)
         return;
     }
     if (!ok) return;
-    hipLaunchKernelGGL((relay_kernel<CM, TC, NA, NX, F>), dim3(tiles), dim3(512), 0, s, ilo, jlo, nxr, ncols, f);
+    hipLaunchKernelGGL((relay_kernel<CM, TC, NA, NX, F, X>), dim3(tiles + (nextra + 511u) / 512u), dim3(512), 0, s, ilo,
+                       jlo, nxr, ncols, tiles, f, extra);
 }
 // columns per relay tile for a box of ncols columns: 32 while that gives every
 // CU a tile, else 16 (the 4,096 columns of a 64 x 64 box make 256 tiles of 16)

@@ -45,75 +45,159 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
     const double* pq1 = prim + PRIM_Q1 * ne;
     const double* pq2 = prim + PRIM_Q2 * ne;
     const double* J = P.terrain ? P.detJ : nullptr;
+    // cell values of a level, and the coefficients of the face between `lo` and `hi`
+    struct Lv { double r, pib, pis, rt_, q1, q2; };
+    struct Row { double a, b, c, P, Q; };
+    auto load = [=] __device__(long q) {
+        Lv v{r0[q], pi0[q], pi_stage[q], rt[q], 0.0, 0.0};
+        if (moist) { v.q1 = pq1[q]; v.q2 = pq2[q]; }
+        return v;
+    };
+    // theta at levels k-2 .. k+1; detJ on the face (terrain)
+    auto face = [=] __device__(const Lv& lo, const Lv& hi, double pr_km2, double pr_km1, double pr_k, double pr_kp1,
+                               double detJ_on_kface) {
+        double rhobar_lo = lo.r, rhobar_hi = hi.r;
+        double pibar_lo = lo.pib, pibar_hi = hi.pib;
+        double pi_c = 0.5 * (lo.pis + hi.pis);
+        double coeff_P, coeff_Q;
+        if (J) {   // terrain (ERF_make_fast_coeffs.cpp:113-137)
+            double inv_detJ_on_kface = 1. / detJ_on_kface;
+            coeff_P = -Gamma * R_d * dzi * inv_detJ_on_kface + halfg * R_d * rhobar_hi / (c_v * pibar_hi * hi.rt_);
+            coeff_Q = Gamma * R_d * dzi * inv_detJ_on_kface + halfg * R_d * rhobar_lo / (c_v * pibar_lo * lo.rt_);
+        } else {
+            coeff_P = -Gamma * R_d * dzi + halfg * R_d * rhobar_hi / (c_v * pibar_hi * hi.rt_);
+            coeff_Q = Gamma * R_d * dzi + halfg * R_d * rhobar_lo / (c_v * pibar_lo * lo.rt_);
+        }
+        coeff_P *= pi_c;
+        coeff_Q *= pi_c;
+        Row w;
+        w.P = coeff_P;
+        w.Q = coeff_Q;
+        if (moist) {   // ERF_make_fast_coeffs.cpp:183-188
+            double qf = 0.5 * (hi.q1 + lo.q1 + hi.q2 + lo.q2);
+            coeff_P /= (1.0 + qf);
+            coeff_Q /= (1.0 + qf);
+        }
+        double theta_t_lo = 0.5 * (pr_km2 + pr_km1);
+        double theta_t_mid = 0.5 * (pr_km1 + pr_k);
+        double theta_t_hi = 0.5 * (pr_k + pr_kp1);
+        w.a = D * (halfg - coeff_Q * theta_t_lo);
+        w.c = D * (-halfg + coeff_P * theta_t_hi);
+        w.b = (J ? detJ_on_kface : 1.0) + D * (coeff_Q - coeff_P) * theta_t_mid;
+        return w;
+    };
+    const double at = top_outflow ? -1.0 : 0.0;
+    // Boxes of few columns: one lane per column and chunk of levels (launch_relay),
+    // so a lane forms one to four rows instead of a whole column of them in
+    // sequence; the recurrence, whose division per level is the serial part, runs
+    // over LDS on one chunk's lanes and the inverses are taken in parallel again.
+    // 64 x 64 x 64: 24.9 us one lane per column, 10.3 us; 161 x 97 x 63 moist: 39.8
+    // us, 34.2 us.  With more columns, or more than 4 levels per chunk at 8,192 or
+    // more, the lanes of the per-column form fill the chip and it reads each level
+    // once (190 x 150 x 80: 53 us against 86; 5.4 TB/s at 512 x 512 x 96).
+    const long ncols = (long)nx * ny;
+    auto tile = [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds, auto cmc, auto tcc) {
+        constexpr int CM = decltype(cmc)::value;
+        constexpr int TC = decltype(tcc)::value;
+        constexpr int R = relay_rows<CM, TC>() * TC;
+        const int chl = tile_chunk(nz, 512 / TC);
+        const int ka = chunk * chl;
+        const int kb = (ka + chl < nz ? ka + chl : nz) - 1;
+        const bool work = valid && ka <= kb;
+        const long q0 = valid ? L.ix(i, j, 0) : 0;
+        double* X = lds;            // a_k
+        double* Y = lds + R;        // b_k, then the pivot
+        double* Z = lds + 2 * R;    // c_k
+        if (work) {
+#pragma unroll
+            for (int m = 0; m < CM; ++m) {
+                const int k = ka + m;
+                if (k > kb) break;
+                const long q = q0 + (long)k * sz;
+                if (k == 0) { A[q] = 0.0; B[q] = 1.0; Cc[q] = 0.0; continue; }
+                const Row w = face(load(q - sz), load(q), prim[q - 2 * sz], prim[q - sz], prim[q], prim[q + sz],
+                                   J ? 0.5 * (J[q] + J[q - sz]) : 1.0);
+                A[q] = w.a; Cc[q] = w.c; Pc[q] = w.P; Qc[q] = w.Q;
+                X[k * TC + col] = w.a; Y[k * TC + col] = w.b; Z[k * TC + col] = w.c;
+            }
+        }
+        __syncthreads();
+        if (chunk == 0 && valid) {
+            double bet = 1.0, c_prev = 0.0;
+            for (int k = 1; k <= nz - 1; ++k) {
+                double gam = c_prev / bet;
+                bet = Y[k * TC + col] - X[k * TC + col] * gam;
+                Y[k * TC + col] = bet;
+                c_prev = Z[k * TC + col];
+            }
+            const long qt = q0 + (long)nz * sz;     // the top face keeps B itself
+            A[qt] = at; Cc[qt] = 0.0;
+            double gam = c_prev / bet;
+            B[qt] = 1.0 - at * gam;
+        }
+        __syncthreads();
+        if (work) {
+#pragma unroll
+            for (int m = 0; m < CM; ++m) {
+                const int k = ka + m;
+                if (k > kb) break;
+                if (k > 0) B[q0 + (long)k * sz] = 1.0 / Y[k * TC + col];   // interior faces store 1/B (:287-290)
+            }
+        }
+    };
+    if (!g_rec && nz <= 128 && (tile_columns(ncols) == 16 || (nz <= 64 && ncols < 16384))) {
+        auto launch = [&](auto cmc, auto tcc) {
+            constexpr int CM = decltype(cmc)::value, TC = decltype(tcc)::value;
+            launch_relay<CM, TC, 0, 0>(0, nx - 1, 0, ny - 1, s,
+                [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds) {
+                    tile(i, j, valid, col, chunk, lds, cmc, tcc);
+                });
+        };
+        using IC16 = std::integral_constant<int, 16>;
+        using IC32 = std::integral_constant<int, 32>;
+        using IC4 = std::integral_constant<int, 4>;
+        if (tile_columns(ncols) == 16) launch(IC4{}, IC16{});
+        else launch(IC4{}, IC32{});
+        return;
+    }
     launch_cols(0, nx - 1, 0, ny - 1, s, [=] __device__(int i, int j) {
         const long q0 = L.ix(i, j, 0);
         // bottom face, then the interior faces with the recurrence carried along
         A[q0] = 0.0; B[q0] = 1.0; Cc[q0] = 0.0;
         double bet = 1.0;
         double c_prev = 0.0;
-        double r_lo = r0[q0], pib_lo = pi0[q0], pis_lo = pi_stage[q0], rt_lo = rt[q0];
+        Lv lo = load(q0);
         double pr_km2 = prim[q0 - sz], pr_km1 = prim[q0], pr_k = prim[q0 + sz];
-        double q1_lo = moist ? pq1[q0] : 0.0, q2_lo = moist ? pq2[q0] : 0.0;
-        struct Lv { double r, pib, pis, rt_, pkp1, q1, q2; };
-        auto load = [&](long q, Lv& v) {
-            v.r = r0[q]; v.pib = pi0[q]; v.pis = pi_stage[q]; v.rt_ = rt[q]; v.pkp1 = prim[q + sz];
-            if (moist) { v.q1 = pq1[q]; v.q2 = pq2[q]; } else { v.q1 = 0.0; v.q2 = 0.0; }
-        };
         constexpr int RD = 4;
         Lv ring[RD];
+        double pnext[RD];
 #pragma unroll
         for (int d = 0; d < RD; ++d)
-            if (1 + d <= nz - 1) load(q0 + (1 + d) * sz, ring[d]);
+            if (1 + d <= nz - 1) { ring[d] = load(q0 + (1 + d) * sz); pnext[d] = prim[q0 + (2 + d) * sz]; }
         for (int kb = 1; kb <= nz - 1; kb += RD) {
 #pragma unroll
             for (int d = 0; d < RD; ++d) {
                 const int k = kb + d;
                 if (k > nz - 1) break;
                 const long q = q0 + k * sz;
-                Lv v = ring[d];
-                if (k + RD <= nz - 1) load(q + RD * sz, ring[d]);
-                double rhobar_lo = r_lo, rhobar_hi = v.r;
-                double pibar_lo = pib_lo, pibar_hi = v.pib;
-                double pi_c = 0.5 * (pis_lo + v.pis);
-                double coeff_P, coeff_Q, detJ_on_kface = 1.0;
-                if (J) {   // terrain (ERF_make_fast_coeffs.cpp:113-137)
-                    detJ_on_kface = 0.5 * (J[q] + J[q - sz]);
-                    double inv_detJ_on_kface = 1. / detJ_on_kface;
-                    coeff_P = -Gamma * R_d * dzi * inv_detJ_on_kface + halfg * R_d * rhobar_hi / (c_v * pibar_hi * v.rt_);
-                    coeff_Q = Gamma * R_d * dzi * inv_detJ_on_kface + halfg * R_d * rhobar_lo / (c_v * pibar_lo * rt_lo);
-                } else {
-                    coeff_P = -Gamma * R_d * dzi + halfg * R_d * rhobar_hi / (c_v * pibar_hi * v.rt_);
-                    coeff_Q = Gamma * R_d * dzi + halfg * R_d * rhobar_lo / (c_v * pibar_lo * rt_lo);
-                }
-                coeff_P *= pi_c;
-                coeff_Q *= pi_c;
-                Pc[q] = coeff_P;
-                Qc[q] = coeff_Q;
-                if (moist) {   // ERF_make_fast_coeffs.cpp:183-188
-                    double qf = 0.5 * (v.q1 + q1_lo + v.q2 + q2_lo);
-                    coeff_P /= (1.0 + qf);
-                    coeff_Q /= (1.0 + qf);
-                }
-                double theta_t_lo = 0.5 * (pr_km2 + pr_km1);
-                double theta_t_mid = 0.5 * (pr_km1 + pr_k);
-                double theta_t_hi = 0.5 * (pr_k + v.pkp1);
-                double a = D * (halfg - coeff_Q * theta_t_lo);
-                double c = D * (-halfg + coeff_P * theta_t_hi);
-                double b = (J ? detJ_on_kface : 1.0) + D * (coeff_Q - coeff_P) * theta_t_mid;
-                A[q] = a;
-                Cc[q] = c;
+                const Lv v = ring[d];
+                const double pkp1 = pnext[d];
+                if (k + RD <= nz - 1) { ring[d] = load(q + RD * sz); pnext[d] = prim[q + (RD + 1) * sz]; }
+                const Row w = face(lo, v, pr_km2, pr_km1, pr_k, pkp1, J ? 0.5 * (J[q] + J[q - sz]) : 1.0);
+                Pc[q] = w.P;
+                Qc[q] = w.Q;
+                A[q] = w.a;
+                Cc[q] = w.c;
                 double gam = c_prev / bet;
-                bet = b - a * gam;
-                c_prev = c;
+                bet = w.b - w.a * gam;
+                c_prev = w.c;
                 B[q] = 1.0 / bet;                        // interior faces store 1/B (:287-290)
-                r_lo = v.r; pib_lo = v.pib; pis_lo = v.pis; rt_lo = v.rt_;
-                pr_km2 = pr_km1; pr_km1 = pr_k; pr_k = v.pkp1;
-                q1_lo = v.q1; q2_lo = v.q2;
+                lo = v;
+                pr_km2 = pr_km1; pr_km1 = pr_k; pr_k = pkp1;
             }
         }
         // top face keeps B itself
         const long qt = q0 + nz * sz;
-        const double at = top_outflow ? -1.0 : 0.0;
         A[qt] = at; Cc[qt] = 0.0;
         double gam = c_prev / bet;
         B[qt] = 1.0 - at * gam;
@@ -138,35 +222,6 @@ void no_substep(const Params& P, const erfx_state& ssum, const erfx_state& sold,
         if (j <= ny - 1 && k <= nz - 1) ssum.xmom[q] = sold.xmom[q] + slow_dt * fslow.xmom[q];
         if (i <= nx - 1 && k <= nz - 1) ssum.ymom[q] = sold.ymom[q] + slow_dt * fslow.ymom[q];
         if (i <= nx - 1 && j <= ny - 1) ssum.zmom[q] = sold.zmom[q] + slow_dt * fslow.zmom[q];
-    });
-}
-
-// The grown box's ghost layer (one cell all round, edges and corners included)
-// of the lagged increment rt_prev - rt_stage, in one launch: the z rows, the y
-// rows, then the x sides with the lanes along j.  With `cons` and `from`, rho and
-// rho*theta of those cells are copied from `from` as well (the terrain form's
-// first substep).
-void lagged_shell(const Params& P, const double* prt, const double* srt, double* lagged, double* cons,
-                  const double* from, hipStream_t s) {
-    const Lay L = P.L;
-    const int nx = L.nx, ny = L.ny, nz = L.nz;
-    const long ne = L.ne;
-    const int nzr = 2 * (ny + 2), nyr = 2 * nz, w = nx + 2 > ny ? nx + 2 : ny;
-    launch_box(Box(0, 0, 0, w - 1, nzr + 2 * nyr - 1, 0), s, [=] __device__(int t, int r, int) {
-        int i, j, k;
-        if (r < nzr) {
-            if (t > nx + 1) return;
-            i = t - 1; j = r / 2 - 1; k = (r & 1) ? nz : -1;
-        } else if (r < nzr + nyr) {
-            if (t > nx + 1) return;
-            i = t - 1; k = (r - nzr) / 2; j = ((r - nzr) & 1) ? ny : -1;
-        } else {
-            if (t > ny - 1) return;
-            j = t; k = (r - nzr - nyr) / 2; i = ((r - nzr - nyr) & 1) ? nx : -1;
-        }
-        const long q = L.ix(i, j, k);
-        if (cons) { cons[q] = from[q]; cons[q + ne] = from[q + ne]; }
-        lagged[q] = prt[q] - srt[q];
     });
 }
 
@@ -261,8 +316,8 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         }
     });
     // the lagged increment's ghost layer, which the next substep reads unless it
-    // reads the periodic images
-    if (!ch.active) lagged_shell(P, prt, srt, lagged, nullptr, nullptr, s);
+    // reads the periodic images (written with the column launch below)
+    const LaggedShell shell{L, prt, srt, lagged, nullptr, nullptr};
 
     // K3 + K4 + K5 fused per column (:328-357, :374-453, :518-536, :566-592).
     // One lane per (i, j) column.  Forward sweep: horizontal divergence of the
@@ -677,11 +732,12 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     if (var == COL_TILE && !tiled) var = COL_FALLBACK;
     kt_start(P.timer, KT_FAST_COLUMN, s);
     if (var == COL_TILE) {
+        if (!ch.active && g_rec) lagged_shell(shell, s);
         auto launch = [&](auto cmc, auto tcc) {
             launch_relay<decltype(cmc)::value, decltype(tcc)::value, 4, 5>(0, nx - 1, 0, ny - 1, s,
                 [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds) {
                     relay(i, j, valid, col, chunk, lds, cmc, tcc);
-                });
+                }, ch.active ? 0u : shell.lanes(), shell);
         };
         using IC16 = std::integral_constant<int, 16>;
         using IC32 = std::integral_constant<int, 32>;
@@ -693,6 +749,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         else if (tile_chunk(nz, 16) <= 6) launch(IC6{}, IC32{});
         else launch(IC8{}, IC32{});
     } else {
+        if (!ch.active) lagged_shell(shell, s);
         const int width = COL_WIDTH[var];
         switch (COL_DEPTH[var]) {
         case 2:

@@ -70,8 +70,45 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 const erfx_state& prev, const erfx_state& stage, const double* prim, const double* pi_stage,
                 const double* fc, const erfx_state& data, const erfx_state& scratch, double dtau,
                 double beta_s, double facinv, hipStream_t s, const FastChain& ch = FastChain());
-void lagged_shell(const Params& P, const double* prt, const double* srt, double* lagged, double* cons,
-                  const double* from, hipStream_t s);
+// The grown box's ghost layer (one cell all round, edges and corners included)
+// of the lagged increment rt_prev - rt_stage, a point per lane: the z rows, the y
+// rows, then the x sides with the lanes along j.  With `cons` and `from`, rho and
+// rho*theta of those cells are copied from `from` as well (the terrain form's
+// first substep).  It runs as extra work-groups of the column launch, which
+// writes the layer's interior: a launch of its own took 5 to 7 us.
+struct LaggedShell {
+    static constexpr bool ANY = true;
+    Lay L;
+    const double *prt, *srt;
+    double* lagged;
+    double* cons;
+    const double* from;
+    __host__ __device__ int width() const { return L.nx + 2 > L.ny ? L.nx + 2 : L.ny; }
+    unsigned lanes() const { return (unsigned)width() * (unsigned)(2 * (L.ny + 2) + 4 * L.nz); }
+    __device__ __forceinline__ void operator()(unsigned n) const {
+        const int nx = L.nx, ny = L.ny, nz = L.nz;
+        const int nzr = 2 * (ny + 2), nyr = 2 * nz, w = width();
+        const int r = (int)(n / (unsigned)w), t = (int)(n % (unsigned)w);
+        int i, j, k;
+        if (r < nzr) {
+            if (t > nx + 1) return;
+            i = t - 1; j = r / 2 - 1; k = (r & 1) ? nz : -1;
+        } else if (r < nzr + nyr) {
+            if (t > nx + 1) return;
+            i = t - 1; k = (r - nzr) / 2; j = ((r - nzr) & 1) ? ny : -1;
+        } else {
+            if (t > ny - 1 || r >= nzr + 2 * nyr) return;
+            j = t; k = (r - nzr - nyr) / 2; i = ((r - nzr - nyr) & 1) ? nx : -1;
+        }
+        const long q = L.ix(i, j, k);
+        if (cons) { cons[q] = from[q]; cons[q + L.ne] = from[q + L.ne]; }
+        lagged[q] = prt[q] - srt[q];
+    }
+};
+// the same in a launch of its own, for the column forms that take no extra work
+inline void lagged_shell(const LaggedShell& S, hipStream_t s) {
+    launch_grid((S.lanes() + 255u) / 256u, s, [=] __device__(unsigned b) { S(b * 256u + threadIdx.x); });
+}
 bool fast_bcs_fusable(const Params& P);
 // no_substep_fun (substepping_type None): S_sum = S_old + slow_dt * F_slow for
 // rho, rho*theta and the momenta

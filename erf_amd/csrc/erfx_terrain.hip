@@ -259,8 +259,9 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         }
     });
     // the ghost layer of the lagged increment and, in the first substep, of rho
-    // and rho*theta (:139-152), which the chain reads at the images instead
-    if (!ch.active) lagged_shell(P, drt, sc1, lagged1, first ? cc0 : nullptr, pc0, s);
+    // and rho*theta (:139-152), which the chain reads at the images instead (written
+    // with the column launch below)
+    const LaggedShell shell{L, drt, sc1, lagged1, first ? cc0 : nullptr, pc0};
 
     // :414-669, one lane per (i, j) column.  The forward sweep makes, level by
     // level, Omega of the old increments (:460-484) on the face above, the
@@ -535,12 +536,13 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
     // a recorded (batched) launch takes chunks of 6 levels in 32-column tiles, so
     // every member of a batch records the same kernel
     if (nz <= 96 && P.col_variant == COL_TILE) {
+        if (!ch.active && g_rec) lagged_shell(shell, s);
         auto launch = [&](auto cmc, auto tcc) {
             constexpr int CM = decltype(cmc)::value;
             launch_relay<CM, decltype(tcc)::value, (CM > 4 ? 5 : 4), (CM > 4 ? 9 : 6)>(0, nx - 1, 0, ny - 1, s,
                 [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds) {
                     relay(i, j, valid, col, chunk, lds, cmc, tcc);
-                });
+                }, ch.active ? 0u : shell.lanes(), shell);
         };
         using IC16 = std::integral_constant<int, 16>;
         using IC32 = std::integral_constant<int, 32>;
@@ -549,7 +551,8 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         if (!g_rec && tile_columns((long)nx * ny) == 16) launch(IC4{}, IC16{});   // 32 chunks: at most 3 levels each
         else if (!g_rec && tile_chunk(nz, 16) <= 4) launch(IC4{}, IC32{});
         else launch(IC6{}, IC32{});
-    } else
+    } else {
+    if (!ch.active) lagged_shell(shell, s);
     launch_cols(0, nx - 1, 0, ny - 1, s, [=] __device__(int i, int j) {
         const long q0 = L.ix(i, j, 0);
         // Omega of the old increments on face kf (0 at the bottom, the rho*w
@@ -678,6 +681,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
             p_hi = pq;
         }
     });
+    }
     // algorithmic bytes per cell: the fields of the substep this kernel reads
     // (stage rho, rho*theta, rho*u, rho*v, rho*w; the previous rho*u, rho*v,
     // rho*w; the new rho*u, rho*v; the current rho, rho*theta; the slow RHS of

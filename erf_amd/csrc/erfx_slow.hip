@@ -1313,7 +1313,7 @@ constexpr int MARCH_PW = 72;   // LDS row of the level tile: columns i0-3 .. i0+
 
 template <class Op, int MR>
 __global__ void __launch_bounds__(64 * (MR + 1))
-march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, int mk) {
+march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, unsigned per, int mk) {
     constexpr int NF = Op::NF;
     constexpr int PR = MR + 6;                        // rows of the level tile
     constexpr int RPT = (PR + MR) / (MR + 1);         // tile rows loaded per lane (rows ly, ly + MR + 1, ...)
@@ -1321,7 +1321,9 @@ march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, int 
     __shared__ double xs[NF][MR][65];
     __shared__ double ys[NF][MR + 1][64];
     const Lay L = op.L;
-    const unsigned t = xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned ts = xcd_remap(blockIdx.x, gridDim.x);
+    const int ms = (int)(ts / per);                   // the scalar of the block (`per` tiles each)
+    const unsigned t = ts % per;
     const unsigned bx = t % gx, by = (t / gx) % gy, bz = t / (gx * gy);
     const int lx = threadIdx.x, ly = threadIdx.y;
     const int i0 = (int)bx * 64, j0 = (int)by * MR;
@@ -1346,7 +1348,7 @@ march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, int 
             const bool rok = rr < PR && jj >= -ng && jj <= ny + ng;
 #pragma unroll
             for (int m = 0; m < NF; ++m) {
-                const double* ps = op.field(m);
+                const double* ps = op.field(ms + m);
                 rm[m][r] = (rok && cm_ok) ? ps[L.ix(cm, jj, k)] : 0.0;
                 rh[m][r] = (rok && ch_ok) ? ps[L.ix(ch, jj, k)] : 0.0;
             }
@@ -1378,7 +1380,7 @@ march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, int 
     if (cellok) {
 #pragma unroll
         for (int m = 0; m < NF; ++m) {
-            const double* ps = op.field(m);
+            const double* ps = op.field(ms + m);
             const double lo3 = ps[qc + (long)(k0 - 3) * sz];
 #pragma unroll
             for (int d = 0; d < 6; ++d) zr[m][d] = ps[qc + (long)(k0 - 2 + d) * sz];
@@ -1437,7 +1439,7 @@ march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, int 
             load_level(k + 1);
             if (cellok) {
 #pragma unroll
-                for (int m = 0; m < NF; ++m) zn[m] = op.field(m)[qc + (long)(k + 4) * sz];
+                for (int m = 0; m < NF; ++m) zn[m] = op.field(ms + m)[qc + (long)(k + 4) * sz];
             }
         }
         if (cellok) {
@@ -1449,7 +1451,7 @@ march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, int 
                 gy0[m] = ys[m][ly][lx];
                 gy1[m] = ys[m][ly + 1][lx];
             }
-            op.cell(i, j, k, gx0, gx1, gy0, gy1, gzl, gzh);
+            op.cell(ms, i, j, k, gx0, gx1, gy0, gy1, gzl, gzh);
 #pragma unroll
             for (int m = 0; m < NF; ++m) gzl[m] = gzh[m];
         }
@@ -1471,11 +1473,12 @@ march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, int 
 }
 
 template <class Op, int MR>
-inline void launch_march_rows(const Op& op, int nx, int ny, int nz, int mk, hipStream_t s) {
+inline void launch_march_rows(const Op& op, int ns, int nx, int ny, int nz, int mk, hipStream_t s) {
     const unsigned gx = (unsigned)((nx + 63) / 64), gy = (unsigned)((ny + MR - 1) / MR);
     const unsigned gz = (unsigned)((nz + mk - 1) / mk);
-    hipLaunchKernelGGL((march_kernel<Op, MR>), dim3(gx * gy * gz), dim3(64, MR + 1, 1), 0, s, op, nx, ny, nz, gx, gy,
-                       mk);
+    const unsigned per = gx * gy * gz;
+    hipLaunchKernelGGL((march_kernel<Op, MR>), dim3(per * (unsigned)ns), dim3(64, MR + 1, 1), 0, s, op, nx, ny, nz, gx,
+                       gy, per, mk);
 }
 // A box whose default tiling gives fewer work-groups than the GPU has CUs
 // (the 64^3 rising thermal: 24) takes shorter stacks of levels and, if that
@@ -1484,15 +1487,15 @@ inline void launch_march_rows(const Op& op, int nx, int ny, int nz, int mk, hipS
 // change any value.
 constexpr int MARCH_MIN_GROUPS = 256;
 template <class Op>
-inline void launch_march(const Op& op, int nx, int ny, int nz, hipStream_t s) {
+inline void launch_march(const Op& op, int ns, int nx, int ny, int nz, hipStream_t s) {
     constexpr int MR = march_rows<Op::MIXED>();
     auto groups = [&](int mr, int mk) {
-        return ((nx + 63) / 64) * ((ny + mr - 1) / mr) * ((nz + mk - 1) / mk);
+        return ns * ((nx + 63) / 64) * ((ny + mr - 1) / mr) * ((nz + mk - 1) / mk);
     };
     int mk = MARCH_MK;
     while (mk > 4 && groups(MR, mk) < MARCH_MIN_GROUPS) mk = mk / 2 > 4 ? mk / 2 : 4;
-    if (MR != 4 && groups(MR, mk) < MARCH_MIN_GROUPS) launch_march_rows<Op, 4>(op, nx, ny, nz, mk, s);
-    else launch_march_rows<Op, MR>(op, nx, ny, nz, mk, s);
+    if (MR != 4 && groups(MR, mk) < MARCH_MIN_GROUPS) launch_march_rows<Op, 4>(op, ns, nx, ny, nz, mk, s);
+    else launch_march_rows<Op, MR>(op, ns, nx, ny, nz, mk, s);
 }
 
 // The scalar update of erf_slow_rhs_post as a marching operator: NF scalars
@@ -1533,15 +1536,17 @@ struct PostOp {
         if constexpr (TT >= 0) return f * interp_scalar_vals_t<mixed, TT>(t, sp2, sp1, s, sm1, sm2, sm3, f, fr);
         return c2c2 ? f * (0.5 * (s + sm1)) : f * interp_scalar_vals<mixed>(t, sp2, sp1, s, sm1, sm2, sm3, f, fr);
     }
-    __device__ __forceinline__ void cell(int i, int j, int k, const double* gx0, const double* gx1, const double* gy0,
-                                         const double* gy1, const double* gz0, const double* gz1) const {
+    // scalar ms of the block
+    __device__ __forceinline__ void cell(int ms, int i, int j, int k, const double* gx0, const double* gx1,
+                                         const double* gy0, const double* gy1, const double* gz0,
+                                         const double* gz1) const {
         const long q = L.ix(i, j, k);
         const long ne = L.ne, sy = L.sy, sz = L.sz;
-        if (copy_slow)
+        if (copy_slow && ms == 0)
             for (int c = 2; c < ncons; ++c)
                 if (!(c >= upd_lo && c < upd_hi)) cur[q + c * ne] = nc[q + c * ne];
         for (int m = 0; m < NF; ++m) {
-            const int n = n0 + m;
+            const int n = n0 + ms + m;
             const double* ps = prim + (n - 1) * ne;
             double invdetJ = Jc ? ((Jc[q] > 0.) ? 1. / Jc[q] : 1.) : 1.;
             double r = -invdetJ * (1.0 * 1.0) * ((gx1[m] - gx0[m]) * dxi + (gy1[m] - gy0[m]) * dyi + (gz1[m] - gz0[m]) * dzi);
@@ -1619,43 +1624,42 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
     }
     if (!g_rec) {
         // one evaluation per face (the batched ensembles record the per-cell
-        // form below), one launch per scalar of the block: the six-level z
-        // rings and the staged rows of several fields at once would exceed the
-        // registers of four waves per SIMD.  The first launch makes the copy of
-        // the slow components; the later ones read only prim, the face mass
-        // fluxes and the old state, which no launch of the block writes.
-        auto run = [&](auto mc, auto tc, int m) {
+        // form below), a work-group per scalar and tile: the six-level z rings and
+        // the staged rows of several fields at once would exceed the registers of
+        // four waves per SIMD, while the scalars of a block, which read only prim,
+        // the face mass fluxes and the old state, run side by side in one launch
+        // (32 x 32 x 24 moist, three scalars: 36 us in three launches, 13.7 us).
+        // The first scalar's work-groups make the copy of the slow components.
+        auto run = [&](auto mc, auto tc) {
             constexpr bool mixed = decltype(mc)::value;
             PostOp<mixed, 1, decltype(tc)::value> op;
             op.L = L; op.nx = nx; op.ny = ny;
             op.dxi = dxi; op.dyi = dyi; op.dzi = dzi; op.Jc = Jc;
             op.ht = ht; op.vt = vt; op.hf = hf; op.vf = vf;
             op.c2c2 = c2c2; op.use_diff = use_diff; op.consA = consA; op.turb = turb; op.clip = clip;
-            op.copy_slow = copy_slow && m == 0; op.ae = ae; op.slow_dt = slow_dt;
+            op.copy_slow = copy_slow; op.ae = ae; op.slow_dt = slow_dt;
             op.dxlo = dxlo; op.dxhi = dxhi; op.dylo = dylo; op.dyhi = dyhi;
-            op.mu_h = mu_h; op.mu_v = mu_v; op.n0 = n0 + m; op.ncons = ncons;
+            op.mu_h = mu_h; op.mu_v = mu_v; op.n0 = n0; op.ncons = ncons;
             op.upd_lo = upd_lo; op.upd_hi = upd_hi;
             op.ax = ax; op.ay = ay; op.az = az; op.cur = cur; op.nc = nc; op.oc = oc; op.crb = crb; op.prim = prim;
             op.dstate = dst;
-            launch_march(op, nx, ny, nz, s);
+            launch_march(op, nc_b, nx, ny, nz, s);
         };
         // one type in all three directions (WENO5, WENO-Z5, U3, U5): that type
         // fixed at compile time
         const int fixed = (!c2c2 && ht == vt && (ht == ERFX_ADV_WENO5 || ht == ERFX_ADV_WENOZ5 ||
                                                  ht == ERFX_ADV_UPWIND3 || ht == ERFX_ADV_UPWIND5)) ? ht : -1;
-        auto typed = [&](auto mc, int m) {
+        auto typed = [&](auto mc) {
             switch (fixed) {
-                case ERFX_ADV_WENO5: run(mc, std::integral_constant<int, ERFX_ADV_WENO5>{}, m); break;
-                case ERFX_ADV_WENOZ5: run(mc, std::integral_constant<int, ERFX_ADV_WENOZ5>{}, m); break;
-                case ERFX_ADV_UPWIND3: run(mc, std::integral_constant<int, ERFX_ADV_UPWIND3>{}, m); break;
-                case ERFX_ADV_UPWIND5: run(mc, std::integral_constant<int, ERFX_ADV_UPWIND5>{}, m); break;
-                default: run(mc, std::integral_constant<int, -1>{}, m); break;
+                case ERFX_ADV_WENO5: run(mc, std::integral_constant<int, ERFX_ADV_WENO5>{}); break;
+                case ERFX_ADV_WENOZ5: run(mc, std::integral_constant<int, ERFX_ADV_WENOZ5>{}); break;
+                case ERFX_ADV_UPWIND3: run(mc, std::integral_constant<int, ERFX_ADV_UPWIND3>{}); break;
+                case ERFX_ADV_UPWIND5: run(mc, std::integral_constant<int, ERFX_ADV_UPWIND5>{}); break;
+                default: run(mc, std::integral_constant<int, -1>{}); break;
             }
         };
-        for (int m = 0; m < nc_b; ++m) {
-            if (mixed_rt) typed(std::true_type{}, m);
-            else typed(std::false_type{}, m);
-        }
+        if (mixed_rt) typed(std::true_type{});
+        else typed(std::false_type{});
         return;
     }
     launch_box_prec(mixed_rt, Box(0, 0, 0, nx - 1, ny - 1, nz - 1), s, [=] __device__(int i, int j, int k, auto mc) {

@@ -1062,8 +1062,8 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
         for (int ks = 0; ks < (nosub ? 0 : nsub); ++ks) {
             // On a laterally periodic box the apply_bcs between two substeps is
             // folded into the next substep (round trip of the momenta on read,
-            // ghost cells read at their images); the full fill runs after the
-            // stage's last substep.
+            // ghost cells read at their images), the one after the stage's last
+            // substep into slow_rhs_post.
             FastChain ch;
             ch.active = chain;
             ch.rt_prev = chain && ks > 0;
@@ -1078,9 +1078,9 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             else
                 fast_rhs_N(P, c->fw, ks, nrk, Fs, ks == 0 ? So : Ss, Sn, s->prim, s->pi_stage, s->fast_coeffs, Ss, Sc,
                            dtau, beta_s, inv_fac, st, ch);
-            if (!chain || ks == nsub - 1) apply_bcs(P, Ss, un, vn, wn, 1, 1, true, false, st);
+            if (!chain) apply_bcs(P, Ss, un, vn, wn, 1, 1, true, false, st);
         }
-        slow_rhs_post(P, c->sw, nrk, slow_dt, Fs, So, Sn, Ss, s->prim, Sc, s->eddy, st);
+        slow_rhs_post(P, c->sw, nrk, slow_dt, Fs, So, Sn, Ss, s->prim, Sc, s->eddy, st, chain);
         apply_bcs(P, Sn, un, vn, wn, P.ng_cons, P.ng_vel, false, false, st);
     }
     // advance_microphysics on the new state (ERF_Advance.cpp:172-174)

@@ -188,6 +188,6 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
 void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                    const erfx_state& old,
                    const erfx_state& snew, const erfx_state& data, const double* prim,
-                   const erfx_state& scratch, const double* eddy, hipStream_t s);
+                   const erfx_state& scratch, const double* eddy, hipStream_t s, bool round_trip = false);
 
 }  // namespace erfx

@@ -1012,7 +1012,12 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
     velocity_to_momentum(P, uo, vo, wo, P.ng_vel, P.ng_vel, cons_old, So.xmom, So.ymom, So.zmom, st);
     // advance_dycore
     if (P.use_turb) turbulent_viscosity(P, c->sw, cons_old, uo, vo, wo, s->eddy, st);
-    {
+    // With the fused fills every value of the new velocities and of S_new that is
+    // read is written before: the velocities by the next fill, S_new by the first
+    // stage's update and fill, that stage reading S_old in its place.  The generic
+    // sequence leaves the outer ghost layers to the copies.
+    const bool copies = !bcs_fusable(P);
+    if (copies) {
         CopyList cl;
         cl.add(un, uo, (long)ne); cl.add(vn, vo, (long)ne); cl.add(wn, wo, (long)ne);
         copy_fields(cl, st);
@@ -1020,7 +1025,7 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
     apply_bcs(P, So, un, vn, wn, P.ng_cons, P.ng_vel, false, true, st, true);
     cons_to_prim(P, So.cons, s->prim, s->pi_stage, P.ng_cons, st);
     // MRI: S_new <- S_old (ERF_MRI.H:225-230)
-    {
+    if (copies) {
         CopyList cl;
         cl.add(Sn.cons, So.cons, (long)(nc * ne)); cl.add(Sn.xmom, So.xmom, (long)ne);
         cl.add(Sn.ymom, So.ymom, (long)ne); cl.add(Sn.zmom, So.zmom, (long)ne);
@@ -1048,9 +1053,10 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             if (nosub) { nsub = 1; dtau = dt; }
             else { nsub = ratio; dtau = sub_timestep; }
         }
+        const erfx_state& stage = nrk == 0 && !copies ? So : Sn;
         if (nrk > 0) cons_to_prim(P, Sn.cons, s->prim, s->pi_stage, P.ng_cons, st);
         const double slow_dt = sdt[nrk];
-        slow_rhs_pre(P, c->sw, nrk, slow_dt, Fs, Sn, s->prim, Sc, un, vn, wn, s->eddy, s->r0, s->p0, st);
+        slow_rhs_pre(P, c->sw, nrk, slow_dt, Fs, stage, s->prim, Sc, un, vn, wn, s->eddy, s->r0, s->p0, st);
         const double inv_fac = 1.0 / static_cast<double>(nsub);
         if (nosub) {
             // no_substep_fun (ERF_TI_no_substep_fun.H:1-146): the fast
@@ -1071,16 +1077,16 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             ch.own_coeffs = true;
             ch.w_lo = P.vel_extdir[2][2];
             ch.w_hi = P.vel_extdir[2][5];
-            if (ks == 0) make_fast_coeffs(P, s->fast_coeffs, Sn, s->prim, s->pi_stage, s->r0, s->pi0, dtau, beta_s, st);
+            if (ks == 0) make_fast_coeffs(P, s->fast_coeffs, stage, s->prim, s->pi_stage, s->r0, s->pi0, dtau, beta_s, st);
             if (P.terrain)
-                fast_rhs_T(P, c->fw, c->tw, ks, nrk, Fs, ks == 0 ? So : Ss, Sn, s->prim, s->pi_stage, s->fast_coeffs,
+                fast_rhs_T(P, c->fw, c->tw, ks, nrk, Fs, ks == 0 ? So : Ss, stage, s->prim, s->pi_stage, s->fast_coeffs,
                            Ss, Sc, dtau, beta_s, inv_fac, st, ch);
             else
-                fast_rhs_N(P, c->fw, ks, nrk, Fs, ks == 0 ? So : Ss, Sn, s->prim, s->pi_stage, s->fast_coeffs, Ss, Sc,
+                fast_rhs_N(P, c->fw, ks, nrk, Fs, ks == 0 ? So : Ss, stage, s->prim, s->pi_stage, s->fast_coeffs, Ss, Sc,
                            dtau, beta_s, inv_fac, st, ch);
             if (!chain) apply_bcs(P, Ss, un, vn, wn, 1, 1, true, false, st);
         }
-        slow_rhs_post(P, c->sw, nrk, slow_dt, Fs, So, Sn, Ss, s->prim, Sc, s->eddy, st, chain);
+        slow_rhs_post(P, c->sw, nrk, slow_dt, Fs, So, Sn, Ss, s->prim, Sc, s->eddy, st, chain, stage.cons);
         apply_bcs(P, Sn, un, vn, wn, P.ng_cons, P.ng_vel, false, false, st);
     }
     // advance_microphysics on the new state (ERF_Advance.cpp:172-174)

@@ -109,6 +109,7 @@ struct LaggedShell {
 inline void lagged_shell(const LaggedShell& S, hipStream_t s) {
     launch_grid((S.lanes() + 255u) / 256u, s, [=] __device__(unsigned b) { S(b * 256u + threadIdx.x); });
 }
+bool bcs_fusable(const Params& P);
 bool fast_bcs_fusable(const Params& P);
 // no_substep_fun (substepping_type None): S_sum = S_old + slow_dt * F_slow for
 // rho, rho*theta and the momenta
@@ -188,6 +189,7 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
 void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                    const erfx_state& old,
                    const erfx_state& snew, const erfx_state& data, const double* prim,
-                   const erfx_state& scratch, const double* eddy, hipStream_t s, bool round_trip = false);
+                   const erfx_state& scratch, const double* eddy, hipStream_t s, bool round_trip = false,
+                   const double* stage_cons = nullptr);
 
 }  // namespace erfx

@@ -1519,6 +1519,7 @@ struct PostOp {
     const double *ax, *ay, *az;
     double* cur;
     double* nc;
+    const double* rc;         // the stage's cons (nc, or elsewhere in the first stage)
     const double* oc;
     double* crb;
     const double* prim;
@@ -1544,7 +1545,11 @@ struct PostOp {
         const long ne = L.ne, sy = L.sy, sz = L.sz;
         if (copy_slow && ms == 0)
             for (int c = 2; c < ncons; ++c)
-                if (!(c >= upd_lo && c < upd_hi)) cur[q + c * ne] = nc[q + c * ne];
+                if (!(c >= upd_lo && c < upd_hi)) {
+                    const double v = rc[q + c * ne];
+                    cur[q + c * ne] = v;
+                    if (rc != nc) nc[q + c * ne] = v;
+                }
         for (int m = 0; m < NF; ++m) {
             const int n = n0 + ms + m;
             const double* ps = prim + (n - 1) * ne;
@@ -1555,12 +1560,12 @@ struct PostOp {
             } else if (use_diff) {
                 const int dsx0 = (dxlo && i == 0) ? -1 : 0, dsx1 = (dxhi && i == nx - 1) ? 1 : 0;
                 const int dsy0 = (dylo && j == 0) ? -1 : 0, dsy1 = (dyhi && j == ny - 1) ? 1 : 0;
-                double dfx0 = diff_flux_bc(nc, ps, mu_h, q, 1, dxi, ae, consA, turb, dsx0) * 1.0;
-                double dfx1 = diff_flux_bc(nc, ps, mu_h, q + 1, 1, dxi, ae, consA, turb, dsx1) * 1.0;
-                double dfy0 = diff_flux_bc(nc, ps, mu_h, q, sy, dyi, ae, consA, turb, dsy0) * 1.0;
-                double dfy1 = diff_flux_bc(nc, ps, mu_h, q + sy, sy, dyi, ae, consA, turb, dsy1) * 1.0;
-                double dfz0 = diff_flux(nc, ps, mu_v, q, sz, dzi, ae, consA, turb);
-                double dfz1 = diff_flux(nc, ps, mu_v, q + sz, sz, dzi, ae, consA, turb);
+                double dfx0 = diff_flux_bc(rc, ps, mu_h, q, 1, dxi, ae, consA, turb, dsx0) * 1.0;
+                double dfx1 = diff_flux_bc(rc, ps, mu_h, q + 1, 1, dxi, ae, consA, turb, dsx1) * 1.0;
+                double dfy0 = diff_flux_bc(rc, ps, mu_h, q, sy, dyi, ae, consA, turb, dsy0) * 1.0;
+                double dfy1 = diff_flux_bc(rc, ps, mu_h, q + sy, sy, dyi, ae, consA, turb, dsy1) * 1.0;
+                double dfz0 = diff_flux(rc, ps, mu_v, q, sz, dzi, ae, consA, turb);
+                double dfz1 = diff_flux(rc, ps, mu_v, q + sz, sz, dzi, ae, consA, turb);
                 r -= (dfx1 - dfx0) * dxi * 1.0 + (dfy1 - dfy0) * dyi * 1.0 + (dfz1 - dfz0) * dzi;
             }
             crb[q + n * ne] = r;
@@ -1587,7 +1592,8 @@ struct ScalarBlock {
 };
 static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B, bool copy_slow, double slow_dt,
                        const erfx_state& rhs, const erfx_state& old, const erfx_state& snew, const erfx_state& data,
-                       const double* prim, const erfx_state& scratch, const double* eddy, hipStream_t s) {
+                       const double* prim, const erfx_state& scratch, const double* eddy, const double* rc,
+                       hipStream_t s) {
     const Lay L = P.L;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const long ne = L.ne, sy = L.sy, sz = L.sz;
@@ -1619,7 +1625,7 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
     // on a terrain grid the diffusion terms are made beforehand (DiffusionSrcForState_T)
     const double* dst = nullptr;
     if (use_diff && P.terrain) {
-        diffusion_state_T(P, W, n0, nc_b, nc, prim, s);
+        diffusion_state_T(P, W, n0, nc_b, rc, prim, s);
         dst = W.dstate;
     }
     if (!g_rec) {
@@ -1641,8 +1647,8 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
             op.dxlo = dxlo; op.dxhi = dxhi; op.dylo = dylo; op.dyhi = dyhi;
             op.mu_h = mu_h; op.mu_v = mu_v; op.n0 = n0; op.ncons = ncons;
             op.upd_lo = upd_lo; op.upd_hi = upd_hi;
-            op.ax = ax; op.ay = ay; op.az = az; op.cur = cur; op.nc = nc; op.oc = oc; op.crb = crb; op.prim = prim;
-            op.dstate = dst;
+            op.ax = ax; op.ay = ay; op.az = az; op.cur = cur; op.nc = nc; op.rc = rc; op.oc = oc; op.crb = crb;
+            op.prim = prim; op.dstate = dst;
             launch_march(op, nc_b, nx, ny, nz, s);
         };
         // one type in all three directions (WENO5, WENO-Z5, U3, U5): that type
@@ -1667,7 +1673,11 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
         const long q = L.ix(i, j, k);
         if (copy_slow)
             for (int c = 2; c < ncons; ++c)
-                if (!(c >= upd_lo && c < upd_hi)) cur[q + c * ne] = nc[q + c * ne];
+                if (!(c >= upd_lo && c < upd_hi)) {
+                    const double v = rc[q + c * ne];
+                    cur[q + c * ne] = v;
+                    if (rc != nc) nc[q + c * ne] = v;
+                }
         double fx0 = ax[q], fx1 = ax[q + 1], fy0 = ay[q], fy1 = ay[q + sy], fz0 = az[q], fz1 = az[q + sz];
         for (int m = 0; m < nc_b; ++m) {
             const int n = n0 + m;
@@ -1695,12 +1705,12 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
             } else if (use_diff) {
                 const int dsx0 = (dxlo && i == 0) ? -1 : 0, dsx1 = (dxhi && i == nx - 1) ? 1 : 0;
                 const int dsy0 = (dylo && j == 0) ? -1 : 0, dsy1 = (dyhi && j == ny - 1) ? 1 : 0;
-                double dfx0 = diff_flux_bc(nc, ps, mu_h, q, 1, dxi, ae, consA, turb, dsx0) * 1.0;
-                double dfx1 = diff_flux_bc(nc, ps, mu_h, q + 1, 1, dxi, ae, consA, turb, dsx1) * 1.0;
-                double dfy0 = diff_flux_bc(nc, ps, mu_h, q, sy, dyi, ae, consA, turb, dsy0) * 1.0;
-                double dfy1 = diff_flux_bc(nc, ps, mu_h, q + sy, sy, dyi, ae, consA, turb, dsy1) * 1.0;
-                double dfz0 = diff_flux(nc, ps, mu_v, q, sz, dzi, ae, consA, turb);
-                double dfz1 = diff_flux(nc, ps, mu_v, q + sz, sz, dzi, ae, consA, turb);
+                double dfx0 = diff_flux_bc(rc, ps, mu_h, q, 1, dxi, ae, consA, turb, dsx0) * 1.0;
+                double dfx1 = diff_flux_bc(rc, ps, mu_h, q + 1, 1, dxi, ae, consA, turb, dsx1) * 1.0;
+                double dfy0 = diff_flux_bc(rc, ps, mu_h, q, sy, dyi, ae, consA, turb, dsy0) * 1.0;
+                double dfy1 = diff_flux_bc(rc, ps, mu_h, q + sy, sy, dyi, ae, consA, turb, dsy1) * 1.0;
+                double dfz0 = diff_flux(rc, ps, mu_v, q, sz, dzi, ae, consA, turb);
+                double dfz1 = diff_flux(rc, ps, mu_v, q + sz, sz, dzi, ae, consA, turb);
                 r -= (dfx1 - dfx0) * dxi * 1.0 + (dfy1 - dfy0) * dyi * 1.0 + (dfz1 - dfz0) * dzi;
             }
             crb[q + n * ne] = r;
@@ -1715,11 +1725,18 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
 // erf_slow_rhs_post (Source/TimeIntegration/ERF_slow_rhs_post.cpp:49-559): the
 // slow variables are RhoScalar (:168-172) and, with moisture, the n_qstate
 // species as one block with the moist advection types (:173-175, :364-434);
-// then S_new <- S_data.
+// then S_new <- S_data.  round_trip: the momenta are the substep chain's, which
+// leaves the fill's momentum round trip to this copy.  stage_cons: the stage's
+// cons where S_new does not hold it yet (the first stage reads S_old's, so no
+// copy of S_old has to be made: that and the velocities, 14 fields of
+// 512 x 512 x 96, took 1.5 ms a step);
+// null for S_new's.
 void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                    const erfx_state& old, const erfx_state& snew, const erfx_state& data, const double* prim,
-                   const erfx_state& scratch, const double* eddy, hipStream_t s, bool round_trip) {
+                   const erfx_state& scratch, const double* eddy, hipStream_t s, bool round_trip,
+                   const double* stage_cons) {
     (void)nrk;
+    if (!stage_cons) stage_cons = snew.cons;
     const Lay L = P.L;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const long ne = L.ne;
@@ -1727,11 +1744,11 @@ void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, 
     const erfx_config& c = P.cfg;
     ScalarBlock scal{ERFX_RHOSCALAR, 1, c.dryscal_horiz_adv, c.dryscal_vert_adv, c.dryscal_horiz_upw_frac,
                      c.dryscal_vert_upw_frac, 4 /* Scalar_h */, 10 /* Scalar_v */, false};
-    post_block(P, W, scal, true, slow_dt, rhs, old, snew, data, prim, scratch, eddy, s);
+    post_block(P, W, scal, true, slow_dt, rhs, old, snew, data, prim, scratch, eddy, stage_cons, s);
     if (P.moist) {
         ScalarBlock moist{ERFX_RHOQ1, P.n_qstate, c.moistscal_horiz_adv, c.moistscal_vert_adv,
                           c.moistscal_horiz_upw_frac, c.moistscal_vert_upw_frac, 5 /* Q_h */, 11 /* Q_v */, true};
-        post_block(P, W, moist, false, slow_dt, rhs, old, snew, data, prim, scratch, eddy, s);
+        post_block(P, W, moist, false, slow_dt, rhs, old, snew, data, prim, scratch, eddy, stage_cons, s);
     }
     double* cur = data.cons;
     double* nc = snew.cons;

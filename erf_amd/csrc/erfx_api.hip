@@ -1009,23 +1009,24 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
     Sn.cons = s->cons[nw];
     // FillPatch of the old state and V2M on the full velocity ghost width (:98-108)
     fill_patch(P, cons_old, uo, vo, wo, st);
-    velocity_to_momentum(P, uo, vo, wo, P.ng_vel, P.ng_vel, cons_old, So.xmom, So.ymom, So.zmom, st);
+    const bool fused = bcs_fusable(P);
+    if (fused) velocity_round_trip(P, uo, vo, wo, P.ng_vel, P.ng_vel, cons_old, So.xmom, So.ymom, So.zmom, un, vn, wn, st);
+    else velocity_to_momentum(P, uo, vo, wo, P.ng_vel, P.ng_vel, cons_old, So.xmom, So.ymom, So.zmom, st);
     // advance_dycore
     if (P.use_turb) turbulent_viscosity(P, c->sw, cons_old, uo, vo, wo, s->eddy, st);
     // With the fused fills every value of the new velocities and of S_new that is
-    // read is written before: the velocities by the next fill, S_new by the first
-    // stage's update and fill, that stage reading S_old in its place.  The generic
-    // sequence leaves the outer ghost layers to the copies.
-    const bool copies = !bcs_fusable(P);
-    if (copies) {
+    // read is written before: the velocities above and by the next fill, S_new by the
+    // first stage's update and fill, that stage reading S_old in its place.  The
+    // generic sequence leaves the outer ghost layers to the copies.
+    if (!fused) {
         CopyList cl;
         cl.add(un, uo, (long)ne); cl.add(vn, vo, (long)ne); cl.add(wn, wo, (long)ne);
         copy_fields(cl, st);
     }
-    apply_bcs(P, So, un, vn, wn, P.ng_cons, P.ng_vel, false, true, st, true);
+    apply_bcs(P, So, un, vn, wn, P.ng_cons, P.ng_vel, false, true, st, true, fused);
     cons_to_prim(P, So.cons, s->prim, s->pi_stage, P.ng_cons, st);
     // MRI: S_new <- S_old (ERF_MRI.H:225-230)
-    if (copies) {
+    if (!fused) {
         CopyList cl;
         cl.add(Sn.cons, So.cons, (long)(nc * ne)); cl.add(Sn.xmom, So.xmom, (long)ne);
         cl.add(Sn.ymom, So.ymom, (long)ne); cl.add(Sn.zmom, So.zmom, (long)ne);
@@ -1053,7 +1054,7 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             if (nosub) { nsub = 1; dtau = dt; }
             else { nsub = ratio; dtau = sub_timestep; }
         }
-        const erfx_state& stage = nrk == 0 && !copies ? So : Sn;
+        const erfx_state& stage = nrk == 0 && fused ? So : Sn;
         if (nrk > 0) cons_to_prim(P, Sn.cons, s->prim, s->pi_stage, P.ng_cons, st);
         const double slow_dt = sdt[nrk];
         slow_rhs_pre(P, c->sw, nrk, slow_dt, Fs, stage, s->prim, Sc, un, vn, wn, s->eddy, s->r0, s->p0, st);
@@ -1086,8 +1087,9 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
                            dtau, beta_s, inv_fac, st, ch);
             if (!chain) apply_bcs(P, Ss, un, vn, wn, 1, 1, true, false, st);
         }
-        slow_rhs_post(P, c->sw, nrk, slow_dt, Fs, So, Sn, Ss, s->prim, Sc, s->eddy, st, chain, stage.cons);
-        apply_bcs(P, Sn, un, vn, wn, P.ng_cons, P.ng_vel, false, false, st);
+        slow_rhs_post(P, c->sw, nrk, slow_dt, Fs, So, Sn, Ss, s->prim, Sc, s->eddy, st, chain ? s->vel[nw] : nullptr,
+                      stage.cons);
+        apply_bcs(P, Sn, un, vn, wn, P.ng_cons, P.ng_vel, false, false, st, false, chain);
     }
     // advance_microphysics on the new state (ERF_Advance.cpp:172-174)
     if (P.moist) {

@@ -295,6 +295,52 @@ void velocity_to_momentum(const Params& P, const double* xv, const double* yv, c
     });
 }
 
+// The start of a step where the fills are fused: VelocityToMomentum of the old
+// velocities, and on the valid faces the MomentumToVelocity and VelocityToMomentum
+// that apply_bcs on the old state begins with (its new velocities xn, yn, zn).
+// Bound by HBM: 512 x 512 x 96 345 us for the first part alone and 857 for the fill,
+// 507 + 158 so.
+void velocity_round_trip(const Params& P, const double* xv, const double* yv, const double* zv, int gx, int gz_w,
+                         const double* dens, double* xm, double* ym, double* zm, double* xn, double* yn, double* zn,
+                         hipStream_t s) {
+    const Lay L = P.L;
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    launch_box(Box(-gx, -gx, -gx, nx + gx, ny + gx, nz + gx), s, [=] __device__(int i, int j, int k) {
+        const long c = L.ix(i, j, k);
+        const bool in = i >= 0 && j >= 0 && k >= 0 && i <= nx && j <= ny && k <= nz;
+        if (j <= ny - 1 + gx && k <= nz - 1 + gx) {
+            const double d = dens[c] + dens[c - 1];
+            double m = xv[c] * 0.5 * d;
+            if (in && j < ny && k < nz) {
+                const double u = m * 2.0 / d;
+                xn[c] = u;
+                m = u * 0.5 * d;
+            }
+            xm[c] = m;
+        }
+        if (i <= nx - 1 + gx && k <= nz - 1 + gx) {
+            const double d = dens[c] + dens[c - L.sy];
+            double m = yv[c] * 0.5 * d;
+            if (in && i < nx && k < nz) {
+                const double v = m * 2.0 / d;
+                yn[c] = v;
+                m = v * 0.5 * d;
+            }
+            ym[c] = m;
+        }
+        if (i <= nx - 1 + gx && j <= ny - 1 + gx && k >= 0 && k <= nz && k >= -gz_w && k <= nz + gz_w) {
+            const double d = dens[c] + dens[c - L.sz];
+            double m = zv[c] * 0.5 * d;
+            if (in && i < nx && j < ny && k > 0 && k < nz) {
+                const double w = m * 2.0 / d;
+                zn[c] = w;
+                m = w * 0.5 * d;
+            }
+            zm[c] = m;
+        }
+    });
+}
+
 // The fused fills: every ghost value the generic sequences below leave behind,
 // computed from valid data alone, so no lane reads a ghost another lane writes
 // and one launch replaces the stages.  What a ghost point holds after
@@ -354,13 +400,18 @@ struct LatFill {
         else { a = lo ? -1 - a : 2 * (n - 1) + 1 - a; neg ^= (t == REFLECT_ODD); }
         return true;
     }
+    // moves (i, j) to the source of a cons ghost, false where the Dirichlet value v is it
+    __device__ __forceinline__ bool cons_src(int n, int& i, int& j, double& v) const {
+        bool neg = false;
+        const bool jl = j < 0, il = i < 0;
+        if (!cell(j, ny, kind[3][1], kind[3][4], py, neg)) { v = jl ? ext[n][1] : ext[n][4]; return false; }
+        if (!cell(i, nx, kind[3][0], kind[3][3], px, neg)) { v = il ? ext[n][0] : ext[n][3]; return false; }
+        return true;
+    }
     template <class B>
     __device__ __forceinline__ double cons_at(int n, int i, int j, const B& base) const {
-        bool neg = false;
-        int a = i, b = j;
-        if (!cell(b, ny, kind[3][1], kind[3][4], py, neg)) return j < 0 ? ext[n][1] : ext[n][4];
-        if (!cell(a, nx, kind[3][0], kind[3][3], px, neg)) return i < 0 ? ext[n][0] : ext[n][3];
-        return base(a, b);
+        double v = 0.0;
+        return cons_src(n, i, j, v) ? base(i, j) : v;
     }
     // a velocity component along its own axis (faces 0..n) from base(face), which
     // is evaluated in one place (and once more for the Neumann rule), as it is the
@@ -436,7 +487,9 @@ static LatFill<PER> lat_fill(const Params& P) {
 //   RAW = false: the velocities are MomentumToVelocity of S's momenta on the
 //   valid faces (ERF_MomentumToVelocity.cpp:24-96), ghosts filled from those;
 //   RAW = true: the velocity arrays hold the valid faces already; only ghosts and
-//   the faces a rule sets are written.
+//   the faces a rule sets are written, and with S's momenta given (ngv is P.ng_vel
+//   then) VelocityToMomentum of those, where the sequence applies it and on the
+//   periodic images.
 // ngv: ghost width of the rules and vertical rows; periodic images reach
 // P.ng_vel (P.ng_cons for cons).  Points the sequences do not touch are not
 // written.
@@ -450,9 +503,9 @@ static void fill_points(const Params& P, const erfx_state& S, double* xv, double
     const long ne = L.ne;
     const int nc = P.cfg.ncons;
     double* c = S.cons;
-    const double* xm = S.xmom;
-    const double* ym = S.ymom;
-    const double* zm = S.zmom;
+    double* xm = S.xmom;
+    double* ym = S.ymom;
+    double* zm = S.zmom;
     const LatFill<PER> F = lat_fill<PER>(P);
     const bool px = PER || P.periodic[0], py = PER || P.periodic[1];
     const int xtl = P.bck[0][2], xth = P.bck[0][5], ytl = P.bck[1][2], yth = P.bck[1][5];
@@ -525,13 +578,21 @@ static void fill_points(const Params& P, const erfx_state& S, double* xv, double
         // ---- x-velocity: valid faces, images and rule ghosts, vertical rows
         const bool un = dxf <= ngv && dyc <= ngv;
         const bool ukeep = RAW && dxf == 0 && dyc == 0 && !LatFill<PER>::face_rule(i, nx, F.kind[0][0], F.kind[0][3], px);
-        if (kval ? !ukeep && (un || image(dxf, dyc, ngV)) : depth <= ngv && un)
-            xv[q] = !kval && (lo ? xtl : xth) == EXT_DIR ? (lo ? xvl : xvh) : u_lat(i, j, kv, un);
+        if (kval ? !ukeep && (un || image(dxf, dyc, ngV)) : depth <= ngv && un) {
+            const double u = !kval && (lo ? xtl : xth) == EXT_DIR ? (lo ? xvl : xvh) : u_lat(i, j, kv, un);
+            xv[q] = u;
+            if (RAW && xm && (kval && image(dxf, dyc, ngV) || dxf <= 1 && dyc <= 1 && k >= -1 && k <= nz))
+                xm[q] = u * 0.5 * (rho(i, j, kv) + rho(i - 1, j, kv));
+        }
         // ---- y-velocity
         const bool vn = dxc <= ngv && dyf <= ngv;
         const bool vkeep = RAW && dxc == 0 && dyf == 0 && !LatFill<PER>::face_rule(j, ny, F.kind[1][1], F.kind[1][4], py);
-        if (kval ? !vkeep && (vn || image(dxc, dyf, ngV)) : depth <= ngv && vn)
-            yv[q] = !kval && (lo ? ytl : yth) == EXT_DIR ? (lo ? yvl : yvh) : v_lat(i, j, kv, vn);
+        if (kval ? !vkeep && (vn || image(dxc, dyf, ngV)) : depth <= ngv && vn) {
+            const double v = !kval && (lo ? ytl : yth) == EXT_DIR ? (lo ? yvl : yvh) : v_lat(i, j, kv, vn);
+            yv[q] = v;
+            if (RAW && xm && (kval && image(dxc, dyf, ngV) || dxc <= 1 && dyf <= 1 && k >= -1 && k <= nz))
+                ym[q] = v * 0.5 * (rho(i, j, kv) + rho(i, j - 1, kv));
+        }
         // ---- z-velocity (k = 0 takes the zlo value on the valid box grown by ngv)
         const bool near = dxc <= ngv && dyc <= ngv;
         const bool plane = near && (k == 0 || k == nz);
@@ -559,6 +620,8 @@ static void fill_points(const Params& P, const erfx_state& S, double* xv, double
                 if (plane) w = (4.0 * w - w_lat(i, j, nz - 2)) / 3.0;
             }
             zv[q] = w;
+            if (RAW && xm && (image(dxc, dyc, ngV) || dxc <= 1 && dyc <= 1))
+                zm[q] = w * 0.5 * (rho(i, j, k > nz - 1 ? nz - 1 : k) + rho(i, j, k - 1 < 0 ? 0 : k - 1));
         }
     };
     if constexpr (!RAW) {
@@ -600,15 +663,60 @@ static void fill_points(const Params& P, const erfx_state& S, double* xv, double
     }
 }
 
+// MomentumToVelocity and VelocityToMomentum of the valid faces, with the density
+// ghosts the fill is about to write.  The z-faces of the bottom and the top take
+// their rule there.
+template <bool PER>
+static void valid_faces(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, hipStream_t s) {
+    const Lay L = P.L;
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    const double* c = S.cons;
+    double* xm = S.xmom;
+    double* ym = S.ymom;
+    double* zm = S.zmom;
+    const LatFill<PER> F = lat_fill<PER>(P);
+    launch_box(Box(0, 0, 0, nx, ny, nz - 1), s, [=] __device__(int i, int j, int k) {
+        const long q = L.ix(i, j, k);
+        auto rho = [&](int a, int b) __attribute__((always_inline)) {
+            double v = 0.0;
+            return F.cons_src(0, a, b, v) ? c[L.ix(a, b, k)] : v;
+        };
+        const double r = rho(i, j);
+        if (j < ny) {
+            const double d = r + rho(i - 1, j), u = xm[q] * 2.0 / d;
+            xv[q] = u;
+            xm[q] = u * 0.5 * d;
+        }
+        if (i < nx) {
+            const double d = r + rho(i, j - 1), v = ym[q] * 2.0 / d;
+            yv[q] = v;
+            ym[q] = v * 0.5 * d;
+        }
+        if (i < nx && j < ny && k > 0) {
+            const double d = r + c[q - L.sz], w = zm[q] * 2.0 / d;
+            zv[q] = w;
+            zm[q] = w * 0.5 * d;
+        }
+    });
+}
+
 // apply_bcs on a box with a periodic lateral axis in two launches instead of the
 // ~30 of the generic sequence below, point for point what that leaves behind:
 // fill_points, then the momenta: V2M where the sequence applies it, the periodic
 // image's V2M on the FillBoundary layers.  `synced`: every component's ghosts
 // take part in the one fill (its rho ghosts are valid on entry, as this forms
 // them again).
+//
+// At the full velocity ghost width the work is split by place instead: the valid
+// faces' momentum -> velocity -> momentum, point by point (valid_faces, or the
+// kernel that wrote the momenta: `ready`), then everything else in one launch
+// around the box.  512 x 512 x 96 with terrain: 857 us in the two launches over the
+// grown box; 158 so, and 135 more in the kernel that wrote the momenta.  161 x 97 x
+// 63 with inflow, where valid_faces does them: 49 us, and 20 + 26.  A narrower fill
+// leaves ghosts of the unruled faces beyond its width and keeps the two launches.
 template <bool PER>
 static void apply_bcs_fused(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, int ngc,
-                            int ngv, bool fast_only, bool synced, hipStream_t s) {
+                            int ngv, bool fast_only, bool synced, bool ready, hipStream_t s) {
     const Lay L = P.L;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const int ngC = P.ng_cons, ngV = P.ng_vel;
@@ -623,6 +731,11 @@ static void apply_bcs_fused(const Params& P, const erfx_state& S, double* xv, do
     for (int n = 0; n < 8; ++n) {
         R.r[n] = n == 0 ? ngu1 : (n < 1 + ncomp2 && n < nc ? (synced ? ngu1 : ngc) : 0);
         if (R.r[n] > rmax) rmax = R.r[n];
+    }
+    if (ngv == ngV) {
+        if (!ready) valid_faces<PER>(P, S, xv, yv, zv, s);
+        fill_points<PER, true>(P, S, xv, yv, zv, R, rmax, ngv, s);
+        return;
     }
     fill_points<PER, false>(P, S, xv, yv, zv, R, rmax, ngv, s);
     const double* c = S.cons;
@@ -676,12 +789,12 @@ void fill_intermediate_patch(const Params& P, const erfx_state& S, double* xv, d
 
 // apply_bcs (Source/TimeIntegration/ERF_TI_utils.H:53-150).
 void apply_bcs(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, int ngc, int ngv,
-               bool fast_only, bool synced, hipStream_t s, bool filled) {
+               bool fast_only, bool synced, hipStream_t s, bool filled, bool ready) {
     // synced: the sequence reads the density ghosts as they are, which the fused
     // form forms again: the same where the caller says that they are filled
     if ((!synced || filled) && ngc >= 1 && ngv >= 1 && bcs_fusable(P)) {
-        if (P.periodic[0] && P.periodic[1]) apply_bcs_fused<true>(P, S, xv, yv, zv, ngc, ngv, fast_only, synced, s);
-        else apply_bcs_fused<false>(P, S, xv, yv, zv, ngc, ngv, fast_only, synced, s);
+        if (P.periodic[0] && P.periodic[1]) apply_bcs_fused<true>(P, S, xv, yv, zv, ngc, ngv, fast_only, synced, ready, s);
+        else apply_bcs_fused<false>(P, S, xv, yv, zv, ngc, ngv, fast_only, synced, ready, s);
         return;
     }
     int scomp, ncomp, ngu;

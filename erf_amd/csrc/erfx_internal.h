@@ -20,7 +20,10 @@ void velocity_to_momentum(const Params& P, const double* xv, const double* yv, c
 void fill_intermediate_patch(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv,
                              int ngc, int ngv, bool cons_only, int icomp, int ncomp, hipStream_t s);
 void apply_bcs(const Params& P, const erfx_state& S, double* xv, double* yv, double* zv, int ngc, int ngv,
-               bool fast_only, bool synced, hipStream_t s, bool filled = false);
+               bool fast_only, bool synced, hipStream_t s, bool filled = false, bool ready = false);
+void velocity_round_trip(const Params& P, const double* xv, const double* yv, const double* zv, int gx, int gz_w,
+                         const double* dens, double* xm, double* ym, double* zm, double* xn, double* yn, double* zn,
+                         hipStream_t s);
 void fill_patch(const Params& P, double* c, double* u, double* v, double* w, hipStream_t s);
 void cons_to_prim(const Params& P, const double* c, double* prim, double* pi_stage, int ng, hipStream_t s);
 
@@ -189,7 +192,7 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
 void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                    const erfx_state& old,
                    const erfx_state& snew, const erfx_state& data, const double* prim,
-                   const erfx_state& scratch, const double* eddy, hipStream_t s, bool round_trip = false,
+                   const erfx_state& scratch, const double* eddy, hipStream_t s, double* const* trip = nullptr,
                    const double* stage_cons = nullptr);
 
 }  // namespace erfx

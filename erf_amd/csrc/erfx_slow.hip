@@ -1725,15 +1725,14 @@ static void post_block(const Params& P, const SlowWork& W, const ScalarBlock& B,
 // erf_slow_rhs_post (Source/TimeIntegration/ERF_slow_rhs_post.cpp:49-559): the
 // slow variables are RhoScalar (:168-172) and, with moisture, the n_qstate
 // species as one block with the moist advection types (:173-175, :364-434);
-// then S_new <- S_data.  round_trip: the momenta are the substep chain's, which
-// leaves the fill's momentum round trip to this copy.  stage_cons: the stage's
-// cons where S_new does not hold it yet (the first stage reads S_old's, so no
-// copy of S_old has to be made: that and the velocities, 14 fields of
-// 512 x 512 x 96, took 1.5 ms a step);
-// null for S_new's.
+// then S_new <- S_data.  trip: the new velocities, where the momenta are the
+// substep chain's, which leaves the fills' momentum round trips to this copy; null
+// otherwise.  stage_cons: the stage's cons where S_new does not hold it yet (the
+// first stage reads S_old's, so no copy of S_old has to be made: that and the
+// velocities, 14 fields of 512 x 512 x 96, took 1.5 ms a step); null for S_new's.
 void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                    const erfx_state& old, const erfx_state& snew, const erfx_state& data, const double* prim,
-                   const erfx_state& scratch, const double* eddy, hipStream_t s, bool round_trip,
+                   const erfx_state& scratch, const double* eddy, hipStream_t s, double* const* trip,
                    const double* stage_cons) {
     (void)nrk;
     if (!stage_cons) stage_cons = snew.cons;
@@ -1756,14 +1755,18 @@ void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, 
     // above).  The scalar blocks wrote their components to both, and with
     // copy_slow the other slow components went from S_new to S_data, so rho and
     // rho*theta are what is left of cons.
-    // round_trip (a stage's chained substeps on a laterally periodic box): data is
-    // as the last substep left it, and its momenta take the momentum -> velocity ->
-    // momentum round trip of the apply_bcs that follows that substep on the way,
-    // with the face densities of the periodic images.  The rest of that
-    // apply_bcs -- ghost cells, velocities, the wall faces -- the fill of S_new after
-    // this makes anew, so its two launches (816 us at 512 x 512 x 96) fall away.
+    // trip (a stage's chained substeps on a laterally periodic box): data is as the
+    // last substep left it, and its momenta take the momentum -> velocity -> momentum
+    // round trips of two fills on the way, with the face densities of the periodic
+    // images: that of the apply_bcs after that substep, whose ghost cells, velocities
+    // and wall faces the fill of S_new makes anew, and that of the fill of S_new
+    // itself, with the velocities it leaves on the valid faces.  512 x 512 x 96: 371 us
+    // without, 543 with both, for 816 + 857 us of fills of which 158 are left.
     const double* rho = cur;
     const long sy = L.sy, sz = L.sz;
+    const bool round_trip = trip != nullptr;
+    double *xv = nullptr, *yv = nullptr, *zv = nullptr;
+    if (round_trip) { xv = trip[0]; yv = trip[1]; zv = trip[2]; }
     launch_box(Box(0, 0, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
         const long q = L.ix(i, j, k);
         double xm = data.xmom[q], ym = data.ymom[q], zm = data.zmom[q];
@@ -1774,13 +1777,19 @@ void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, 
             const long qc = q - (i == nx ? nx : 0) - (j == ny ? (long)ny * sy : 0);
             const double rc = rho[qc];
             const double dx = rc + rho[i == 0 ? q + nx - 1 : q - 1], dy = rc + rho[j == 0 ? q + (long)(ny - 1) * sy : q - sy];
+            xm = xm * 2.0 / dx * 0.5 * dx;
+            ym = ym * 2.0 / dy * 0.5 * dy;
             const double u = xm * 2.0 / dx, v = ym * 2.0 / dy;
             xm = u * 0.5 * dx;
             ym = v * 0.5 * dy;
+            if (j <= ny - 1 && k <= nz - 1) xv[q] = u;
+            if (i <= nx - 1 && k <= nz - 1) yv[q] = v;
             if (k > 0 && k < nz) {
                 const double dz = rc + rho[qc - sz];
+                zm = zm * 2.0 / dz * 0.5 * dz;
                 const double w = zm * 2.0 / dz;
                 zm = w * 0.5 * dz;
+                if (i <= nx - 1 && j <= ny - 1) zv[q] = w;
             }
         }
         if (cell) { nc[q] = c0; nc[q + ne] = c1; }

@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 from erf_amd import config as C, problems as P
-from helpers import ALL_IDS
+from helpers import ALL_IDS, valid
 from oracle_lib import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -127,6 +127,38 @@ def test_apply_bcs(kind, which, fast_only, synced):
                                sim.ptr(C.F_ZVEL), ngc, ngv, fast_only, synced))
     sim.sync()
     assert _same(sim, orc, ids) == {}
+
+
+@pytest.mark.parametrize("kind", ["thermal", "inflow", "hill"])
+@pytest.mark.parametrize("shape", [(4, 4, 8), (5, 7, 8), (67, 6, 9), (8, 33, 17)])
+def test_apply_bcs_small_and_ragged(kind, shape):
+    """The launch around the box leaves out a core 1 .. n-2: boxes whose core is
+    two cells wide, ones that wrap several columns per work-group, odd sizes."""
+    from erf_amd.lib import Sim, lib, check
+    make = {"thermal": P.rising_thermal, "inflow": P.inflow_outflow, "hill": P.hill_flow}[kind]
+    cfg, f = make(*shape, seed=31)
+    orc = Oracle(cfg)
+    orc.load(f)
+    orc.step(0.0, 0.5, 1)
+    sim = Sim(cfg)
+    ids = list(ALL_IDS) + (TERRAIN_IDS if cfg.use_terrain else [])
+    for fid in ids:
+        sim.upload(fid, orc.get(fid))
+    ng = sim.L.ng
+    for which, synced in ((C.S_NEW, 0), (C.S_OLD, 1)):
+        orc.call("orc_apply_bcs", which, ng, ng - 1, 0, synced)
+        check(lib().erfx_apply_bcs(sim.ctx, _st(sim, which), sim.ptr(C.F_XVEL), sim.ptr(C.F_YVEL),
+                                   sim.ptr(C.F_ZVEL), ng, ng - 1, 0, synced))
+    sim.sync()
+    assert _same(sim, orc, ids) == {}
+    orc, sim = Oracle(cfg), Sim(cfg)
+    orc.load(f)
+    sim.load(f)
+    orc.step(0.0, 0.5, 3)
+    sim.step(0.0, 0.5, 3)
+    for fid in (C.F_CONS, C.F_XVEL, C.F_YVEL, C.F_ZVEL):
+        a, b = (valid(x.get(fid) if x is orc else x.download(fid), cfg, x.L, fid) for x in (sim, orc))
+        assert np.array_equal(a, b), fid
 
 
 @pytest.mark.parametrize("kind", KINDS)

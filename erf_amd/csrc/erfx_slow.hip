@@ -991,7 +991,6 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
     double* rvr = rhs.ymom;
     double* rwr = rhs.zmom;
     const double* om = P.terrain ? W.omega : rw;   // Omega = rho*w on a flat grid
-    const bool terr = P.terrain;
     const TAdvData TD{ru, rv, u, v, w, om, P.ax, P.ay, P.az, P.detJ, Zn{P.z_nd, L}, sy, sz, dxi, dyi, dzi, hf, vf,
                       ht, vt, nz, c2c2};
     const Zn zt{P.z_nd, L};
@@ -1013,8 +1012,9 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
     // U3 or U5 (tc; -1: the types at run time), so the face stencils compile
     // to straight-line code.
     const int ht_rt = ht, vt_rt = vt;
-    auto body = [=] __device__(int i, int j, int k, auto tc) {
+    auto body = [=] __device__(int i, int j, int k, auto tc, auto gc) {
         constexpr int TT = decltype(tc)::value;
+        constexpr bool terr = decltype(gc)::value;
         const int ht = TT >= 0 ? TT : ht_rt;
         const int vt = TT >= 0 ? TT : vt_rt;
         constexpr bool mixed = false;
@@ -1023,6 +1023,13 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
         td.vt = vt;
         const TAdv<mixed> TA{td};
         const long q = L.ix(i, j, k);
+        // the three components' stores come last: they may alias the inputs as far
+        // as the compiler knows, so a store between them would end the loads in
+        // flight of one component before the next one's begin (with the terrain
+        // test at compile time 64^3 20.6 -> 17.3 us, 256 x 256 x 80 428 -> 389, 161 x
+        // 97 x 63 85 -> 79; large boxes are bound by L1 requests: 512 x 512 x 96 with
+        // terrain 2667 -> 2643).
+        double out_x = 0.0, out_y = 0.0, out_z = 0.0;
         // ---- x-momentum on x-faces ----
         if (j <= ny - 1 && k <= nz - 1) {
             double src;
@@ -1090,7 +1097,7 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
             double qf = moist ? face_q(pq1, pq2, q, q - 1) : 0.0;
             r += (-gpx - apg0) / (1.0 + qf) + xs;
             if ((zero_xlo && i == 0) || (zero_xhi && i == nx)) r = 0.;
-            rur[q] = r;
+            out_x = r;
         }
         // ---- y-momentum on y-faces ----
         if (i <= nx - 1 && k <= nz - 1) {
@@ -1158,11 +1165,10 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
             double qf = moist ? face_q(pq1, pq2, q, q - sy) : 0.0;
             r += (-gpy - apg1) / (1.0 + qf) + ys;
             if ((zero_ylo && j == 0) || (zero_yhi && j == ny)) r = 0.;
-            rvr[q] = r;
+            out_y = r;
         }
         // ---- z-momentum on z-faces (rhs is zero on the bottom and top faces) ----
-        if (i <= nx - 1 && j <= ny - 1) {
-            if (k == 0 || k == nz) { rwr[q] = 0.0; return; }
+        if (i <= nx - 1 && j <= ny - 1 && k > 0 && k < nz) {
             const int hz = nz, lz = 0;
             double src;
             if (terr) {
@@ -1267,11 +1273,18 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
             double gpz = dzi * (pp[q] - pp[q - sz]) / met_h_zeta;
             double qf = moist ? face_q(pq1, pq2, q, q - sz) : 0.0;
             r += (zs - gpz - apg2) / (1.0 + qf);
-            rwr[q] = r;
+            out_z = r;
         }
+        if (j <= ny - 1 && k <= nz - 1) rur[q] = out_x;
+        if (i <= nx - 1 && k <= nz - 1) rvr[q] = out_y;
+        if (i <= nx - 1 && j <= ny - 1) rwr[q] = out_z;
     };
     auto go = [&](auto tc) {
-        launch_box_z(Box(0, 0, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) { body(i, j, k, tc); });
+        const Box b(0, 0, 0, nx, ny, nz);
+        if (P.terrain)
+            launch_box_z(b, s, [=] __device__(int i, int j, int k) { body(i, j, k, tc, std::true_type{}); });
+        else
+            launch_box_z(b, s, [=] __device__(int i, int j, int k) { body(i, j, k, tc, std::false_type{}); });
     };
     if (!c2c2 && ht == vt && ht == ERFX_ADV_UPWIND3) go(std::integral_constant<int, ERFX_ADV_UPWIND3>{});
     else if (!c2c2 && ht == vt && ht == ERFX_ADV_UPWIND5) go(std::integral_constant<int, ERFX_ADV_UPWIND5>{});

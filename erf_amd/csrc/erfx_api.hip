@@ -1057,7 +1057,7 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
         const erfx_state& stage = nrk == 0 && fused ? So : Sn;
         if (nrk > 0) cons_to_prim(P, Sn.cons, s->prim, s->pi_stage, P.ng_cons, st);
         const double slow_dt = sdt[nrk];
-        slow_rhs_pre(P, c->sw, nrk, slow_dt, Fs, stage, s->prim, Sc, un, vn, wn, s->eddy, s->r0, s->p0, st);
+        slow_rhs_pre(P, c->sw, nrk, slow_dt, Fs, stage, s->prim, Sc, un, vn, wn, s->eddy, s->r0, s->p0, st, P.terrain || nosub);
         const double inv_fac = 1.0 / static_cast<double>(nsub);
         if (nosub) {
             // no_substep_fun (ERF_TI_no_substep_fun.H:1-146): the fast
@@ -1076,6 +1076,7 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             ch.rt_prev = chain && ks > 0;
             ch.last = ks == nsub - 1;
             ch.own_coeffs = true;
+            ch.seed = ks == 0 && !P.terrain;
             ch.w_lo = P.vel_extdir[2][2];
             ch.w_hi = P.vel_extdir[2][5];
             if (ks == 0) make_fast_coeffs(P, s->fast_coeffs, stage, s->prim, s->pi_stage, s->r0, s->pi0, dtau, beta_s, st);

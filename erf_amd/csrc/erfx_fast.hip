@@ -257,6 +257,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     const bool first = (nrk == 0 && step == 0);
     const bool rt = ch.rt_prev && step > 0;
     const bool use_lag = step > 0;
+    const bool seed = ch.seed;
     const double* prho = prev.cons;
     const double gr = -Gamma * R_d;
     const bool moist = P.moist;
@@ -277,7 +278,8 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         const long qx = (rt && i == 0) ? q + nx - 1 : q - 1;
         const long qy = (rt && j == 0) ? q + (long)(ny - 1) * sy : q - sy;
         double pmx = pxm[q], pmy = pym[q];
-        const double sx = sxm[q], sy_ = sym[q], lx = slx[q], ly = sly[q], ax = axm[q], ay = aym[q];
+        const double sx = sxm[q], sy_ = sym[q], lx = slx[q], ly = sly[q];
+        const double ax = seed ? sx : axm[q], ay = seed ? sy_ : aym[q];
         double rc = 0.0, rx = 0.0, ry = 0.0;
         if (rt) { rc = prho[qc]; rx = prho[qx]; ry = prho[qy]; }
         double frx = 0.0, fry = 0.0;
@@ -485,8 +487,9 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 data.zmom[q] = bc.szz + sol;
                 double zflux_lo = beta_2 * sol + beta_1 * drw_k;
                 double zflux_hi = beta_2 * sol_next + beta_1 * drw_next;
-                scratch.zmom[q] += facinv * zflux_lo / (1.0 * 1.0);
-                if (k == nz - 1) scratch.zmom[q + sz] += facinv * zflux_hi / (1.0 * 1.0);
+                scratch.zmom[q] = (seed ? bc.szz : scratch.zmom[q]) + facinv * zflux_lo / (1.0 * 1.0);
+                if (k == nz - 1)
+                    scratch.zmom[q + sz] = (seed ? stage.zmom : scratch.zmom)[q + sz] + facinv * zflux_hi / (1.0 * 1.0);
                 double pcq = bc.pc;
                 double t0 = bc.t0 + dzi * (zflux_hi - zflux_lo);
                 double t1 = bc.t1 + 0.5 * dzi * (zflux_hi * (pcq + p_next) - zflux_lo * (pcq + bc.pm));
@@ -681,7 +684,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
             p_bot = prim[q0 + (long)(ka - 1) * sz];
 #pragma unroll
             for (int m = 0; m < CM; ++m)
-                if (ka + m <= kb) az[m] = scratch.zmom[q0 + (long)(ka + m) * sz];
+                if (ka + m <= kb) az[m] = seed ? sz_[m] : scratch.zmom[q0 + (long)(ka + m) * sz];
         };
         if (CM <= 6 && work) load3();
         // ---- phase 2: the sweeps ----
@@ -709,7 +712,8 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
                 double t1 = slot(T1, m) + 0.5 * dzi * (zflux_hi * (pcq + p_next) - zflux_lo * (pcq + pm));
                 data.zmom[q] = sz_[m] + sol;
                 scratch.zmom[q] = az[m] + facinv * zflux_lo / (1.0 * 1.0);
-                if (k == nz - 1) scratch.zmom[q + sz] += facinv * zflux_hi / (1.0 * 1.0);
+                if (k == nz - 1)
+                    scratch.zmom[q + sz] = (seed ? stage.zmom : scratch.zmom)[q + sz] + facinv * zflux_hi / (1.0 * 1.0);
                 cc0[q] = prr[m] + dtau * (slot(S0, m) - t0);
                 cc1[q] = ptr_[m] + dtau * (slot(S1, m) - t1);
             }

@@ -68,6 +68,11 @@ struct FastChain {
     // fc is what make_fast_coeffs made for this stage, dtau and beta_s
     bool own_coeffs = false;
     double w_lo = 0.0, w_hi = 0.0;   // Dirichlet w on the bottom and top faces
+    // flat grids: the averaged momenta start from the stage's momenta here, in the
+    // stage's first substep, which reads those anyway, and not from a copy that
+    // slow_rhs_pre makes (3 fields written and read again: 256 x 256 x 128 71 us a
+    // stage for the copy and 5 us a substep more, 64^3 5.5)
+    bool seed = false;
 };
 void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erfx_state& slow_rhs,
                 const erfx_state& prev, const erfx_state& stage, const double* prim, const double* pi_stage,
@@ -188,7 +193,7 @@ void turbulent_viscosity(const Params& P, const SlowWork& W, const double* cons,
 void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                   const erfx_state& data, const double* prim, const erfx_state& scratch, const double* u,
                   const double* v, const double* w, const double* eddy, const double* r0, const double* p0,
-                  hipStream_t s);
+                  hipStream_t s, bool seed = true);
 void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                    const erfx_state& old,
                    const erfx_state& snew, const erfx_state& data, const double* prim,

@@ -793,7 +793,7 @@ __device__ __forceinline__ double moist_buoyancy_dev(int btype, int nq, const do
 void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                   const erfx_state& data, const double* prim, const erfx_state& scratch, const double* u,
                   const double* v, const double* w, const double* eddy, const double* r0, const double* p0,
-                  hipStream_t s) {
+                  hipStream_t s, bool seed) {
     (void)nrk; (void)slow_dt;
     const Lay L = P.L;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
@@ -965,7 +965,8 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
         });
 
         // time-averaged momenta seeded with the stage momenta (ERF_AdvectionSrcForState.cpp:56-71)
-        launch_box(Box(0, 0, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
+        // unless the first substep does (FastChain::seed)
+        if (seed) launch_box(Box(0, 0, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
             const long q = L.ix(i, j, k);
             if (j <= ny - 1 && k <= nz - 1) scratch.xmom[q] = 1.0 * ru[q] / 1.0;
             if (i <= nx - 1 && k <= nz - 1) scratch.ymom[q] = 1.0 * rv[q] / 1.0;

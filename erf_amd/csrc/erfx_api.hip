@@ -1024,7 +1024,7 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
         copy_fields(cl, st);
     }
     apply_bcs(P, So, un, vn, wn, P.ng_cons, P.ng_vel, false, true, st, true, fused);
-    cons_to_prim(P, So.cons, s->prim, s->pi_stage, P.ng_cons, st);
+    cons_to_prim(P, So.cons, s->prim, s->pi_stage, P.ng_cons, st, c->sw.pp, s->p0);
     // MRI: S_new <- S_old (ERF_MRI.H:225-230)
     if (!fused) {
         CopyList cl;
@@ -1055,9 +1055,9 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             else { nsub = ratio; dtau = sub_timestep; }
         }
         const erfx_state& stage = nrk == 0 && fused ? So : Sn;
-        if (nrk > 0) cons_to_prim(P, Sn.cons, s->prim, s->pi_stage, P.ng_cons, st);
+        if (nrk > 0) cons_to_prim(P, Sn.cons, s->prim, s->pi_stage, P.ng_cons, st, c->sw.pp, s->p0);
         const double slow_dt = sdt[nrk];
-        slow_rhs_pre(P, c->sw, nrk, slow_dt, Fs, stage, s->prim, Sc, un, vn, wn, s->eddy, s->r0, s->p0, st, P.terrain || nosub);
+        slow_rhs_pre(P, c->sw, nrk, slow_dt, Fs, stage, s->prim, Sc, un, vn, wn, s->eddy, s->r0, s->p0, st, P.terrain || nosub, true);
         const double inv_fac = 1.0 / static_cast<double>(nsub);
         if (nosub) {
             // no_substep_fun (ERF_TI_no_substep_fun.H:1-146): the fast

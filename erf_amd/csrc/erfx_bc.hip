@@ -831,13 +831,19 @@ void fill_patch(const Params& P, double* c, double* u, double* v, double* w, hip
 }
 
 // cons_to_prim (ERF_TI_utils.H:4-45): prim on the box grown by ng, pi_stage
-// on the box grown by one.  One launch covers both.
-void cons_to_prim(const Params& P, const double* c, double* prim, double* pi_stage, int ng, hipStream_t s) {
+// on the box grown by one.  One launch covers both, and with `pp` the pressure
+// perturbation that erf_slow_rhs_pre begins with (ERF_slow_rhs_pre.cpp:337-358),
+// on cells grown by one from k = 0 up: this kernel waits for memory, that one for
+// its powers (two launches and one: 64^3 22 and 19 us, 256 x 256 x 128 258 and 230,
+// 512 x 512 x 96 moist 974 and 847).
+void cons_to_prim(const Params& P, const double* c, double* prim, double* pi_stage, int ng, hipStream_t s, double* pp,
+                  const double* p0) {
     const Lay L = P.L;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const int nprim = P.cfg.ncons - 1;
     const long ne = L.ne;
     const double rdOcp = P.rdOcp;
+    const bool moist = P.moist;
     Box b(-ng, -ng, -ng, nx - 1 + ng, ny - 1 + ng, nz - 1 + ng);
     launch_box(b, s, [=] __device__(int i, int j, int k) {
         long q = L.ix(i, j, k);
@@ -847,6 +853,8 @@ void cons_to_prim(const Params& P, const double* c, double* prim, double* pi_sta
         for (int n = 1; n < nprim; ++n) prim[q + n * ne] = c[q + (1 + n) * ne] / rho;
         if (i >= -1 && i <= nx && j >= -1 && j <= ny && k >= -1 && k <= nz)
             pi_stage[q] = eos_exner_of_rt(rho_theta, rdOcp);
+        if (pp && i >= -1 && i <= nx && j >= -1 && j <= ny && k >= 0 && k <= nz)
+            pp[q] = (moist ? eos_p_of_rt_qv(rho_theta, c[q + ERFX_RHOQ1 * ne] / rho) : eos_p_of_rt(rho_theta)) - p0[q];
     });
 }
 

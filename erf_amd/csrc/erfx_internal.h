@@ -25,7 +25,8 @@ void velocity_round_trip(const Params& P, const double* xv, const double* yv, co
                          const double* dens, double* xm, double* ym, double* zm, double* xn, double* yn, double* zn,
                          hipStream_t s);
 void fill_patch(const Params& P, double* c, double* u, double* v, double* w, hipStream_t s);
-void cons_to_prim(const Params& P, const double* c, double* prim, double* pi_stage, int ng, hipStream_t s);
+void cons_to_prim(const Params& P, const double* c, double* prim, double* pi_stage, int ng, hipStream_t s, double* pp = nullptr,
+                  const double* p0 = nullptr);
 
 // Device-to-device copy of up to COPY_MAX arrays in one launch over the whole
 // chip (the runtime's copy engine splits a large copy into many small blit
@@ -193,7 +194,7 @@ void turbulent_viscosity(const Params& P, const SlowWork& W, const double* cons,
 void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                   const erfx_state& data, const double* prim, const erfx_state& scratch, const double* u,
                   const double* v, const double* w, const double* eddy, const double* r0, const double* p0,
-                  hipStream_t s, bool seed = true);
+                  hipStream_t s, bool seed = true, bool pp_ready = false);
 void slow_rhs_post(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                    const erfx_state& old,
                    const erfx_state& snew, const erfx_state& data, const double* prim,

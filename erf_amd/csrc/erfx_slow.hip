@@ -793,7 +793,7 @@ __device__ __forceinline__ double moist_buoyancy_dev(int btype, int nq, const do
 void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, const erfx_state& rhs,
                   const erfx_state& data, const double* prim, const erfx_state& scratch, const double* u,
                   const double* v, const double* w, const double* eddy, const double* r0, const double* p0,
-                  hipStream_t s, bool seed) {
+                  hipStream_t s, bool seed, bool pp_ready) {
     (void)nrk; (void)slow_dt;
     const Lay L = P.L;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
@@ -809,19 +809,20 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
         }
     }
 
-    // p' on cells grown by one, k >= 0 (ERF_slow_rhs_pre.cpp:337-358)
+    // p' on cells grown by one, k >= 0 (ERF_slow_rhs_pre.cpp:337-358), unless
+    // cons_to_prim made it
     double* pp = W.pp;
     const double* rt = data.cons + ne;
     const bool moist = P.moist;
     if (!moist) {
-        launch_box(Box(-1, -1, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
+        if (!pp_ready) launch_box(Box(-1, -1, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
             const long q = L.ix(i, j, k);
             pp[q] = eos_p_of_rt(rt[q]) - p0[q];
         });
     } else {
         const double* rq1 = data.cons + ERFX_RHOQ1 * ne;
         const double* rho = data.cons;
-        launch_box(Box(-1, -1, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
+        if (!pp_ready) launch_box(Box(-1, -1, 0, nx, ny, nz), s, [=] __device__(int i, int j, int k) {
             const long q = L.ix(i, j, k);
             double qv_for_p = rq1[q] / rho[q];
             pp[q] = eos_p_of_rt_qv(rt[q], qv_for_p) - p0[q];

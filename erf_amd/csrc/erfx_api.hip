@@ -1556,6 +1556,11 @@ static int ens_record(const std::vector<erfx_sim*>& mem, double time, double dt,
     b->dt = dt;
     stage_dts(time, dt, b->sdt);
     b->variant = variant;
+    // boxes with one open axis step through the fused fills or, if they are only a
+    // few cells wide or high, through the generic sequence; a batch of both takes
+    // the generic one for all, so that its members record the same launches
+    bool generic = false;
+    for (const erfx_sim* s : mem) generic = generic || !bcs_fusable(s->ctx->P);
     for (int k = 0; k < n; ++k) {
         erfx_sim* s = mem[(size_t)k];
         Params& P = s->ctx->P;
@@ -1569,6 +1574,7 @@ static int ens_record(const std::vector<erfx_sim*>& mem, double time, double dt,
         P.tuner = nullptr;
         P.col_variant = variant;
         Recorder r;
+        r.generic_fills = generic;
         g_rec = &r;
         int rc = sim_one_step(s, time, dt, s->ctx->P.cfg.mri_ratio);
         g_rec = nullptr;

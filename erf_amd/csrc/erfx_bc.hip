@@ -350,6 +350,7 @@ void velocity_round_trip(const Params& P, const double* xv, const double* yv, co
 // periodic image on a periodic axis), that point's x position likewise.
 bool bcs_fusable(const Params& P) {
     if (!P.periodic[0] && !P.periodic[1]) return false;
+    if (g_rec && g_rec->generic_fills && !(P.periodic[0] && P.periodic[1])) return false;
     const int G = P.ng_cons > P.ng_vel ? P.ng_cons : P.ng_vel;
     if (P.L.nx < G + 1 || P.L.ny < G + 1 || P.L.nz < 2 * G) return false;
     for (int v = 0; v < 2; ++v)

@@ -113,6 +113,9 @@ struct RecItem {
 struct Recorder {
     std::vector<RecItem> items;
     const char* refused = nullptr;   // set by a launch that cannot be recorded
+    // a member of the batch does not take the fused boundary fills: the others keep
+    // to the generic sequence where that one has to be able to join them
+    bool generic_fills = false;
 };
 // the calling thread's active recorder (host only), or null
 extern thread_local Recorder* g_rec;

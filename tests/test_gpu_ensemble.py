@@ -155,6 +155,28 @@ def test_ensemble_autotune_keeps_results():
         s.close()
 
 
+@pytest.mark.parametrize("small", [(16, 16, 5), (16, 16, 4)])
+def test_ensemble_open_axis_with_a_small_member(small):
+    """Boxes open along x: one of 4 or 5 levels is below the fused fills' size
+    (twice the ghost layers) and steps through the generic sequence; a batch takes
+    it next to larger ones, every member as it steps alone."""
+    from erf_amd.lib import Ensemble
+    cases = [P.inflow_outflow(*sh, seed=s) for sh, s in (((16, 16, 16), 1), (small, 2), ((20, 12, 24), 3))]
+    a, b = _pairs(cases)
+    ens = Ensemble(a)
+    ens.set_streams(1)                 # all in one batch
+    ens.step(0.0, 0.5, 3)
+    for s in b:
+        s.step(0.0, 0.5, 3)
+    # the valid cells and faces: what ghost points no rule writes hold is left over
+    for x, y, (cfg, _) in zip(a, b, cases):
+        for fid in FIELDS:
+            assert np.array_equal(valid(x.download(fid), cfg, x.L, fid), valid(y.download(fid), cfg, y.L, fid)), fid
+    ens.close()
+    for s in a + b:
+        s.close()
+
+
 def test_ensemble_refuses_different_sequences():
     from erf_amd.lib import Ensemble, ErfxError
     c1, f1 = P.rising_thermal(16, 16, 16, seed=1)

@@ -456,8 +456,11 @@ constexpr int relay_lds_doubles() { return (NA * CM + NX) * 512 + (CM <= 4 ? 4 *
 // lanes sweep them: a hand-over costs more than a short chunk's levels (64 x 64
 // x 64, two levels per chunk: 18.0 us per launch relayed, 14.4 staged).
 // Every lane of the work-group calls it; `carry` is the LDS after the arrays.
+// Without `implicit` (the explicit substep) the right-hand sides are the solution,
+// and the lanes only pass each other what stands on their chunk's upper face, in
+// `line`, a row of one value per thread.
 template <int CM, int TC>
-__device__ __forceinline__ void relay_solve(double* carry, int nz, int chl, int col, bool valid, double (&rhs)[CM],
+__device__ __forceinline__ void relay_solve(double* carry, double* line, bool implicit, int nz, int chl, int col, bool valid, double (&rhs)[CM],
                                             const double (&av)[CM], const double (&bv)[CM], double (&cv)[CM],
                                             double r_top, double a_top, double b_top, double& s_top, double& x_hi) {
     constexpr int CPW = 64 / TC;               // chunks per wave
@@ -465,6 +468,14 @@ __device__ __forceinline__ void relay_solve(double* carry, int nz, int chl, int 
     const int ka = chunk * chl;
     const int kb = (ka + chl < nz ? ka + chl : nz) - 1;
     const bool has = ka <= kb, top = has && kb == nz - 1;
+    if (!implicit) {
+        __syncthreads();
+        line[tid] = rhs[0];
+        __syncthreads();
+        s_top = r_top;
+        x_hi = has && !top ? line[tid + TC] : r_top;
+        return;
+    }
     if constexpr (CM <= 4) {
         double* X = carry;
         double* Y = X + relay_rows<CM, TC>() * TC;

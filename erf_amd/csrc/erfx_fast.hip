@@ -528,6 +528,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     // (own_coeffs) a_k and c_k are formed again from P, Q and theta, by the
     // expressions that made them, instead of being read.
     const bool own = ch.own_coeffs;
+    const bool separate = step > 0 && prev.cons != data.cons;   // a hook's separate buffers
     const double Dc = dtau * dtau * beta_2 * beta_2 * dzi;
     auto relay = [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds, auto cmc, auto tcc) {
         constexpr int CM = decltype(cmc)::value;
@@ -685,11 +686,19 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
 #pragma unroll
             for (int m = 0; m < CM; ++m)
                 if (ka + m <= kb) az[m] = seed ? sz_[m] : scratch.zmom[q0 + (long)(ka + m) * sz];
+            if (separate) {    // the cells to update are not the ones read so far
+#pragma unroll
+                for (int m = 0; m < CM; ++m)
+                    if (ka + m <= kb) {
+                        prr[m] = cc0[q0 + (long)(ka + m) * sz];
+                        ptr_[m] = cc1[q0 + (long)(ka + m) * sz];
+                    }
+            }
         };
         if (CM <= 6 && work) load3();
         // ---- phase 2: the sweeps ----
         double x_hi = 0.0;       // the solution on the chunk's upper face
-        relay_solve<CM, TC>(carry, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
+        relay_solve<CM, TC>(carry, xch, implicit, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
         // ---- phase 3: the chunk's cells ----
         if (work) {
             if (CM > 6) load3();
@@ -729,11 +738,10 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     }
     // The tile form takes up to 128 levels; a recorded (batched) launch up to 96,
     // always in 32-column tiles of 6 levels per chunk, so every member of a batch
-    // records the same kernel.  It needs the state it updates to be the one it
-    // reads (every substep but a hook's with step > 0 and separate buffers) and
-    // the implicit solve.
-    const bool tiled = implicit && (step == 0 || prev.cons == data.cons) && nz <= (g_rec ? 96 : 128);
-    if (var == COL_TILE && !tiled) var = COL_FALLBACK;
+    // records the same kernel.  Separate buffers and the explicit substep included:
+    // 64 x 64 x 64 in separate buffers 27.6 us a substep, one lane per column 91.9
+    // us; 190 x 150 x 80 199 and 248.
+    if (var == COL_TILE && nz > (g_rec ? 96 : 128)) var = COL_FALLBACK;
     kt_start(P.timer, KT_FAST_COLUMN, s);
     if (var == COL_TILE) {
         if (!ch.active && g_rec) lagged_shell(shell, s);

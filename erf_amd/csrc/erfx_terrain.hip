@@ -496,7 +496,7 @@ void fast_rhs_T(const Params& P, const FastWork& W, const TerrainWork& T, int st
         }
         // ---- phase 2 ----
         double x_hi = 0.0;       // the solution on the chunk's upper face
-        relay_solve<CM, TC>(carry, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
+        relay_solve<CM, TC>(carry, xch, true, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
         // ---- phase 3: rho*w, the averaged Omega, rho and rho*theta of the chunk ----
         if (work) {
             if (top) {

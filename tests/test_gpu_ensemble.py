@@ -177,6 +177,23 @@ def test_ensemble_open_axis_with_a_small_member(small):
         s.close()
 
 
+def test_ensemble_implicit_and_explicit_members():
+    """the substep's solve is an option of a member, not another kernel"""
+    from erf_amd.lib import Ensemble
+    cases = [P.rising_thermal(*sh, seed=s) for sh, s in (((16, 16, 16), 1), ((20, 16, 24), 2))]
+    cases[1][0].implicit_substepping = 0
+    a, b = _pairs(cases)
+    ens = Ensemble(a)
+    ens.set_streams(1)                 # both in one batch
+    ens.step(0.0, 0.2, 2)
+    for s in b:
+        s.step(0.0, 0.2, 2)
+    assert _diff(a, b) == []
+    ens.close()
+    for s in a + b:
+        s.close()
+
+
 def test_ensemble_refuses_different_sequences():
     from erf_amd.lib import Ensemble, ErfxError
     c1, f1 = P.rising_thermal(16, 16, 16, seed=1)

@@ -357,7 +357,7 @@ inline void launch_cols(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f, 
     hipLaunchKernelGGL(col_kernel<F>, dim3(gx * gy), dim3((unsigned)width, 1, 1), 0, s, ilo, ihi, jlo, jhi, gx, f);
 }
 
-// ---- column tiles: one work-group of 8 waves per 32 or 16 columns ----------
+// ---- column tiles: one work-group of 8 waves per 64, 32 or 16 columns ------
 // For column solves whose per-level work is independent except for a
 // tridiagonal recurrence: the lanes of a column split its levels into chunks,
 // form the per-level terms of their chunk in parallel, pass the recurrence
@@ -431,7 +431,7 @@ struct TileItem {
     BHdr h;
     F f;
 };
-// Relay tiles: a work-group of 8 waves takes TC (32 or 16) consecutive columns
+// Relay tiles: a work-group of 8 waves takes TC (64, 32 or 16) consecutive columns
 // of the flattened range and splits their levels into 512 / TC chunks; thread t
 // works on column t % TC in chunk t / TC.  The functor is called on all lanes,
 // `valid` false past the range's end, so that every lane reaches the work-group
@@ -597,7 +597,7 @@ void launch_relay_batch(const void* items, const unsigned* starts, int n, unsign
 }
 template <int CM, int TC, int NA, int NX, class F, class X = NoExtra>
 inline void launch_relay(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f, unsigned nextra = 0, X extra = X()) {
-    static_assert(TC == 16 || TC == 32, "relay tile width");
+    static_assert(TC == 16 || TC == 32 || TC == 64, "relay tile width");
     const bool ok = ilo <= ihi && jlo <= jhi;
     const unsigned nxr = ok ? (unsigned)(ihi - ilo + 1) : 1u;
     const unsigned ncols = ok ? nxr * (unsigned)(jhi - jlo + 1) : 0u;
@@ -611,8 +611,9 @@ inline void launch_relay(int ilo, int ihi, int jlo, int jhi, hipStream_t s, F f,
     hipLaunchKernelGGL((relay_kernel<CM, TC, NA, NX, F, X>), dim3(tiles + (nextra + 511u) / 512u), dim3(512), 0, s, ilo,
                        jlo, nxr, ncols, tiles, f, extra);
 }
-// columns per relay tile for a box of ncols columns: 32 while that gives every
-// CU a tile, else 16 (the 4,096 columns of a 64 x 64 box make 256 tiles of 16)
+// columns per relay tile for a box of ncols columns: 32 (or more) while that
+// gives every CU a tile, else 16 (the 4,096 columns of a 64 x 64 box make 256
+// tiles of 16)
 inline int tile_columns(long ncols) {
     constexpr long CUS = 256;
     return (ncols + 31) / 32 >= CUS ? 32 : 16;

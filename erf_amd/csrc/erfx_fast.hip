@@ -503,7 +503,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
             }
         }
     };
-    // The same column work as a tile of TC (32 or 16) columns per work-group of 8
+    // The same column work as a tile of TC (64, 32 or 16) columns per work-group of 8
     // waves, the levels of a column split into 512 / TC chunks of at most CM, one
     // lane per chunk and column (launch_relay), for boxes of up to 128 levels:
     //  1. each lane reads its chunk's levels once and forms, as the column kernel
@@ -756,7 +756,18 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         using IC4 = std::integral_constant<int, 4>;
         using IC6 = std::integral_constant<int, 6>;
         using IC8 = std::integral_constant<int, 8>;
+        // Up to 32 levels on many columns, 64 columns per tile: 8 chunks instead of
+        // 16, of which short columns leave most idle, and up to 8 levels with the LDS
+        // of one level a chunk, which lets two work-groups run on a CU.  In 64-column
+        // tiles, in 32-column tiles: 512 x 512 x 4 86, 178 us; x 9 199, 274; x 16
+        // 333, 388; x 32 630, 682; 96 x 96 x 20 18.8, 23.8 (more levels have no room
+        // for their rows; fewer columns give fewer tiles than CUs: 64 x 64 x 32 in
+        // 16-column tiles 17.3, one lane per column 51).
+        using IC64 = std::integral_constant<int, 64>;
         if (!g_rec && tile_columns((long)nx * ny) == 16) launch(IC4{}, IC16{});   // 32 chunks: at most 4 levels each
+        else if (!g_rec && tile_chunk(nz, 8) <= 1) launch(std::integral_constant<int, 1>{}, IC64{});
+        else if (!g_rec && tile_chunk(nz, 8) <= 2) launch(std::integral_constant<int, 2>{}, IC64{});
+        else if (!g_rec && tile_chunk(nz, 8) <= 4) launch(IC4{}, IC64{});
         else if (!g_rec && tile_chunk(nz, 16) <= 4) launch(IC4{}, IC32{});
         else if (tile_chunk(nz, 16) <= 6) launch(IC6{}, IC32{});
         else launch(IC8{}, IC32{});

@@ -146,3 +146,24 @@ def test_tile_form_chunk_edges(shape, moist):
     assert _same(a, b) == []
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("moist", [False, True])
+@pytest.mark.parametrize("shape", [(96, 96, 4), (97, 95, 8), (97, 95, 9), (96, 96, 16), (97, 95, 17), (96, 96, 32),
+                                   (97, 95, 33), (91, 90, 20), (90, 90, 20)])
+def test_tile_form_few_levels(shape, moist):
+    """64-column tiles at the edges of their chunk sizes (one, two and four
+    levels: 8, 16 and 32 levels), one level past the last, a last tile that is
+    partial, the first column count that takes them and the last that does not:
+    bit-identical with one lane per column.  (4 levels are below the fused fills'
+    size, so there the launch carries the ghost layer as well.)"""
+    case = P.moist_bubble if moist else P.rising_thermal
+    cfg, f = case(*shape, seed=43, adv=C.ADV_UPWIND3)
+    a, b = _pair(cfg, f)
+    a.set_graph(False)
+    a.set_column_variant(7)          # one lane per column
+    a.step(0.0, 0.5, 2)
+    b.step(0.0, 0.5, 2)
+    assert _same(a, b) == []
+    a.close()
+    b.close()

@@ -274,7 +274,7 @@ def _substep(sim, prev, step, beta_s):
 
 
 @pytest.mark.parametrize("moist", [False, True])
-@pytest.mark.parametrize("shape", [(24, 20, 9), (41, 23, 128), (96, 96, 40), (97, 95, 65), (96, 96, 97)])
+@pytest.mark.parametrize("shape", [(24, 20, 9), (41, 23, 128), (96, 96, 7), (97, 95, 13), (96, 96, 31), (96, 96, 40), (97, 95, 65), (96, 96, 97)])
 @pytest.mark.parametrize("implicit,separate", [(True, True), (False, False), (False, True)])
 def test_substep_tiles_separate_and_explicit(shape, moist, implicit, separate):
     """The substep whose state is not the one it reads (S_prev and S_data in
@@ -300,16 +300,20 @@ def test_substep_tiles_separate_and_explicit(shape, moist, implicit, separate):
         assert np.array_equal(a, b, equal_nan=True), n
 
 
-@pytest.mark.parametrize("implicit,separate", [(True, False), (True, True), (False, False)])
-def test_substep_tiles_run(implicit, separate):
-    """64 x 64 x 64: the tile form takes a third of one lane per column's time
-    (31 us and 92 us a substep), in place and in separate buffers, implicit and
-    explicit; half is asked for."""
+@pytest.mark.parametrize("shape,implicit,separate,share",
+                         [((64, 64, 64), True, False, 0.5), ((64, 64, 64), True, True, 0.5),
+                          ((64, 64, 64), False, False, 0.5), ((512, 128, 4), True, False, 1.25)])
+def test_substep_tiles_run(shape, implicit, separate, share):
+    """The tile form runs where it is the faster one.  64 x 64 x 64, in place and
+    in separate buffers, implicit and explicit: a third of one lane per column's
+    time (28 us and 92 us a substep); half is asked for.  Few levels on many
+    columns: 23 us and 27 us; a quarter more than 27 is asked for (tiles of fewer
+    columns, most of whose lanes idle there, take 44)."""
     import time
     import torch
     assert torch.cuda.is_available()
     from erf_amd.lib import Sim
-    cfg, f = P.rising_thermal(64, 64, 64, seed=41, adv=C.ADV_UPWIND3)
+    cfg, f = P.rising_thermal(*shape, seed=41, adv=C.ADV_UPWIND3)
     cfg.implicit_substepping = int(implicit)
     sim = Sim(cfg)
     sim.load(f)
@@ -327,4 +331,4 @@ def test_substep_tiles_run(implicit, separate):
             best.append(time.perf_counter() - t)
         took[variant] = min(best)
     sim.close()
-    assert took[C.COL_VARIANTS - 1] < 0.5 * took[7], took
+    assert took[C.COL_VARIANTS - 1] < share * took[7], took

@@ -1321,13 +1321,16 @@ void slow_rhs_pre(const Params& P, const SlowWork& W, int nrk, double slow_dt, c
 // 1279 us at 4; mixed 717 us at 15 rows, 957 us at 9, 854 us at 4).  The
 // registers (106 VGPRs FP64, 90 mixed) allow one 16-wave work-group per CU,
 // so taller tiles mean more waves per CU as well as less y-halo.
+// The 4-row tiles of small boxes are held to 4 waves per SIMD too: with the
+// types at run time the compiler takes registers for 3 (512 x 128 x 12, C2: 44.3
+// us for the block, 37.3 us held).
 template <bool mixed>
 constexpr int march_rows() { return 15; }
 constexpr int MARCH_MK = 12;   // levels per work-group (one WENO5 scalar at 15 rows: 882 / 879 / 859 / 879 / 925 / 971 us at 8 / 10 / 12 / 16 / 24 / 32)
 constexpr int MARCH_PW = 72;   // LDS row of the level tile: columns i0-3 .. i0+66, padded
 
 template <class Op, int MR>
-__global__ void __launch_bounds__(64 * (MR + 1))
+__global__ void __launch_bounds__(64 * (MR + 1), 4)
 march_kernel(const Op op, int nx, int ny, int nz, unsigned gx, unsigned gy, unsigned per, int mk) {
     constexpr int NF = Op::NF;
     constexpr int PR = MR + 6;                        // rows of the level tile

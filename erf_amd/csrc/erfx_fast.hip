@@ -45,22 +45,22 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
     const double* pq1 = prim + PRIM_Q1 * ne;
     const double* pq2 = prim + PRIM_Q2 * ne;
     const double* J = P.terrain ? P.detJ : nullptr;
-    // cell values of a level, and the coefficients of the face between `lo` and `hi`
-    struct Lv { double r, pib, pis, rt_, q1, q2; };
-    struct Row { double a, b, c, P, Q; };
-    auto load = [=] __device__(long q) {
-        Lv v{r0[q], pi0[q], pi_stage[q], rt[q], 0.0, 0.0};
-        if (moist) { v.q1 = pq1[q]; v.q2 = pq2[q]; }
-        return v;
+    // cell values of a level with theta of the level above, and the coefficients of
+    // the face between `lo` and `hi`
+    struct Lv { double r, pib, pis, rt_, pkp1, q1, q2; };
+    struct Row { double a, b, c; };
+    auto load = [=] __device__(long q, Lv& v) {
+        v.r = r0[q]; v.pib = pi0[q]; v.pis = pi_stage[q]; v.rt_ = rt[q]; v.pkp1 = prim[q + sz];
+        if (moist) { v.q1 = pq1[q]; v.q2 = pq2[q]; } else { v.q1 = 0.0; v.q2 = 0.0; }
     };
-    // theta at levels k-2 .. k+1; detJ on the face (terrain)
-    auto face = [=] __device__(const Lv& lo, const Lv& hi, double pr_km2, double pr_km1, double pr_k, double pr_kp1,
-                               double detJ_on_kface) {
+    // face q, theta at levels k-2 .. k
+    auto face = [=] __device__(long q, const Lv& lo, const Lv& hi, double pr_km2, double pr_km1, double pr_k) {
         double rhobar_lo = lo.r, rhobar_hi = hi.r;
         double pibar_lo = lo.pib, pibar_hi = hi.pib;
         double pi_c = 0.5 * (lo.pis + hi.pis);
-        double coeff_P, coeff_Q;
+        double coeff_P, coeff_Q, detJ_on_kface = 1.0;
         if (J) {   // terrain (ERF_make_fast_coeffs.cpp:113-137)
+            detJ_on_kface = 0.5 * (J[q] + J[q - sz]);
             double inv_detJ_on_kface = 1. / detJ_on_kface;
             coeff_P = -Gamma * R_d * dzi * inv_detJ_on_kface + halfg * R_d * rhobar_hi / (c_v * pibar_hi * hi.rt_);
             coeff_Q = Gamma * R_d * dzi * inv_detJ_on_kface + halfg * R_d * rhobar_lo / (c_v * pibar_lo * lo.rt_);
@@ -71,8 +71,8 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
         coeff_P *= pi_c;
         coeff_Q *= pi_c;
         Row w;
-        w.P = coeff_P;
-        w.Q = coeff_Q;
+        Pc[q] = coeff_P;
+        Qc[q] = coeff_Q;
         if (moist) {   // ERF_make_fast_coeffs.cpp:183-188
             double qf = 0.5 * (hi.q1 + lo.q1 + hi.q2 + lo.q2);
             coeff_P /= (1.0 + qf);
@@ -80,7 +80,7 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
         }
         double theta_t_lo = 0.5 * (pr_km2 + pr_km1);
         double theta_t_mid = 0.5 * (pr_km1 + pr_k);
-        double theta_t_hi = 0.5 * (pr_k + pr_kp1);
+        double theta_t_hi = 0.5 * (pr_k + hi.pkp1);
         w.a = D * (halfg - coeff_Q * theta_t_lo);
         w.c = D * (-halfg + coeff_P * theta_t_hi);
         w.b = (J ? detJ_on_kface : 1.0) + D * (coeff_Q - coeff_P) * theta_t_mid;
@@ -92,9 +92,14 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
     // sequence; the recurrence, whose division per level is the serial part, runs
     // over LDS on one chunk's lanes and the inverses are taken in parallel again.
     // 64 x 64 x 64: 24.9 us one lane per column, 10.3 us; 161 x 97 x 63 moist: 39.8
-    // us, 34.2 us.  With more columns, or more than 4 levels per chunk at 8,192 or
-    // more, the lanes of the per-column form fill the chip and it reads each level
-    // once (190 x 150 x 80: 53 us against 86; 5.4 TB/s at 512 x 512 x 96).
+    // us, 34.2 us.  Two tiles fit the LDS of a CU, so 512 of 32 columns are one full
+    // round, and the line lies there, at 16,384 columns: tile and per-column form at 64 levels, dry and moist, 127 x 127 21.0 |
+    // 27.7, 24.5 | 30.8 us; 128 x 128 20.0 | 27.7, 23.8 | 30.8; 135 x 135 26.8 | 28.1,
+    // 30.6 | 30.8; 150 x 150 28.3 | 28.3, 33.4 | 31.3; 181 x 181 38.0 | 29.9 (16 and 40
+    // levels: 127 x 127 7.0 | 9.3 and 13.1 | 18.7, 181 x 181 11.1 | 10.5 and 25.0 |
+    // 20.2).  Chunks of more than 4 levels were slower too (190 x 150 x 80: 86 us
+    // against 53 profiled).  The lanes of the per-column form fill the chip there
+    // and it reads each level once (5.4 TB/s at 512 x 512 x 96).
     const long ncols = (long)nx * ny;
     auto tile = [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds, auto cmc, auto tcc) {
         constexpr int CM = decltype(cmc)::value;
@@ -115,9 +120,11 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
                 if (k > kb) break;
                 const long q = q0 + (long)k * sz;
                 if (k == 0) { A[q] = 0.0; B[q] = 1.0; Cc[q] = 0.0; continue; }
-                const Row w = face(load(q - sz), load(q), prim[q - 2 * sz], prim[q - sz], prim[q], prim[q + sz],
-                                   J ? 0.5 * (J[q] + J[q - sz]) : 1.0);
-                A[q] = w.a; Cc[q] = w.c; Pc[q] = w.P; Qc[q] = w.Q;
+                Lv lo, hi;
+                load(q - sz, lo);
+                load(q, hi);
+                const Row w = face(q, lo, hi, prim[q - 2 * sz], prim[q - sz], prim[q]);
+                A[q] = w.a; Cc[q] = w.c;
                 X[k * TC + col] = w.a; Y[k * TC + col] = w.b; Z[k * TC + col] = w.c;
             }
         }
@@ -145,7 +152,7 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
             }
         }
     };
-    if (!g_rec && nz <= 128 && (tile_columns(ncols) == 16 || (nz <= 64 && ncols < 16384))) {
+    if (!g_rec && nz <= 128 && (tile_columns(ncols) == 16 || (nz <= 64 && ncols <= 16384))) {
         auto launch = [&](auto cmc, auto tcc) {
             constexpr int CM = decltype(cmc)::value, TC = decltype(tcc)::value;
             launch_relay<CM, TC, 0, 0>(0, nx - 1, 0, ny - 1, s,
@@ -166,14 +173,14 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
         A[q0] = 0.0; B[q0] = 1.0; Cc[q0] = 0.0;
         double bet = 1.0;
         double c_prev = 0.0;
-        Lv lo = load(q0);
-        double pr_km2 = prim[q0 - sz], pr_km1 = prim[q0], pr_k = prim[q0 + sz];
+        Lv lo;
+        load(q0, lo);
+        double pr_km2 = prim[q0 - sz], pr_km1 = prim[q0], pr_k = lo.pkp1;
         constexpr int RD = 4;
         Lv ring[RD];
-        double pnext[RD];
 #pragma unroll
         for (int d = 0; d < RD; ++d)
-            if (1 + d <= nz - 1) { ring[d] = load(q0 + (1 + d) * sz); pnext[d] = prim[q0 + (2 + d) * sz]; }
+            if (1 + d <= nz - 1) load(q0 + (1 + d) * sz, ring[d]);
         for (int kb = 1; kb <= nz - 1; kb += RD) {
 #pragma unroll
             for (int d = 0; d < RD; ++d) {
@@ -181,11 +188,8 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
                 if (k > nz - 1) break;
                 const long q = q0 + k * sz;
                 const Lv v = ring[d];
-                const double pkp1 = pnext[d];
-                if (k + RD <= nz - 1) { ring[d] = load(q + RD * sz); pnext[d] = prim[q + (RD + 1) * sz]; }
-                const Row w = face(lo, v, pr_km2, pr_km1, pr_k, pkp1, J ? 0.5 * (J[q] + J[q - sz]) : 1.0);
-                Pc[q] = w.P;
-                Qc[q] = w.Q;
+                if (k + RD <= nz - 1) load(q + RD * sz, ring[d]);
+                const Row w = face(q, lo, v, pr_km2, pr_km1, pr_k);
                 A[q] = w.a;
                 Cc[q] = w.c;
                 double gam = c_prev / bet;
@@ -193,7 +197,7 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
                 c_prev = w.c;
                 B[q] = 1.0 / bet;                        // interior faces store 1/B (:287-290)
                 lo = v;
-                pr_km2 = pr_km1; pr_km1 = pr_k; pr_k = pkp1;
+                pr_km2 = pr_km1; pr_km1 = pr_k; pr_k = v.pkp1;
             }
         }
         // top face keeps B itself

@@ -173,6 +173,35 @@ def test_make_fast_coeffs(kind):
     assert _same(sim, orc, ids) == {}
 
 
+@pytest.mark.parametrize("kind", ["dry", "moist", "hill", "hill_moist"])
+@pytest.mark.parametrize("shape", [(64, 64, 128), (96, 96, 40), (97, 95, 64), (96, 96, 65), (128, 128, 9),
+                                   (129, 128, 9)])
+def test_make_fast_coeffs_forms(kind, shape):
+    """Each form by box size: 16-column tiles with the most levels they take,
+    32-column tiles (three and four levels per chunk, the last tile partial, the
+    largest column count), one lane per column past the tiles' levels and past their
+    columns.  All five components bit-identical to the oracle's from the same state
+    (one step on the GPU)."""
+    import torch
+    assert torch.cuda.is_available()
+    from erf_amd.lib import Sim, lib, check
+    make = {"dry": P.rising_thermal, "moist": P.moist_bubble}.get(kind)
+    cfg, f = make(*shape, seed=47) if make else P.hill_flow(*shape, seed=47, moist=(kind == "hill_moist"))
+    sim, orc = Sim(cfg), Oracle(cfg)
+    sim.load(f)
+    orc.load(f)
+    sim.step(0.0, 0.2, 1)
+    for fid in [C.state_id(C.S_NEW, 0), C.D_PRIM, C.D_PI_STAGE, C.F_R0, C.F_P0, C.F_PI0, C.D_FAST_COEFFS]:
+        orc.set(fid, sim.download(fid))
+    orc.call("orc_make_fast_coeffs", 0.05, 0.1)
+    check(lib().erfx_make_fast_coeffs(sim.ctx, sim.ptr(C.D_FAST_COEFFS), _st(sim, C.S_NEW), sim.ptr(C.D_PRIM),
+                                      sim.ptr(C.D_PI_STAGE), 0.05, 0.1))
+    sim.sync()
+    a, b = sim.download(C.D_FAST_COEFFS), orc.get(C.D_FAST_COEFFS)
+    assert np.array_equal(a, b, equal_nan=True), [int((x != y).sum()) for x, y in zip(a, b)]
+    assert np.abs(valid(b, cfg, sim.L, C.D_FAST_COEFFS)[1]).min() > 0.0
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("step,nrk", [(0, 0), (0, 2), (3, 2)])
 def test_fast_rhs_N(kind, step, nrk):

@@ -381,13 +381,27 @@ struct ConsRows {
 // faces.  Each `*_at` returns the value of a point of valid k at any lateral
 // index, from `base` at valid points.  PER: both axes periodic (the rules drop
 // out at compile time).
-template <bool PER>
-struct LatFill {
-    int nx, ny;
-    bool px, py;
+struct LatRules {
     int kind[4][6];                          // x-, y-, z-velocity, cons
     double vel[3][6];
     double ext[ERFX_NCONS_MOIST][6];
+    bool px, py;
+};
+struct LatImages {                           // both axes periodic: no rule is read (nor passed to the kernels)
+    static constexpr int kind[4][6] = {};
+    static constexpr double vel[3][6] = {};
+    static constexpr double ext[ERFX_NCONS_MOIST][6] = {};
+    static constexpr bool px = true, py = true;
+};
+template <bool PER>
+struct LatFill : std::conditional_t<PER, LatImages, LatRules> {
+    using Rules = std::conditional_t<PER, LatImages, LatRules>;
+    using Rules::kind;
+    using Rules::vel;
+    using Rules::ext;
+    using Rules::px;
+    using Rules::py;
+    int nx, ny;
     static __device__ __forceinline__ int wrap(int a, int n, int hi) { return a < 0 ? a + n : (a > hi ? a - n : a); }
     // cell-centred along an axis of n cells: moves `a` to the source index, false
     // for a Dirichlet ghost; `neg` flips the sign (odd reflection)
@@ -475,11 +489,14 @@ struct LatFill {
 template <bool PER>
 static LatFill<PER> lat_fill(const Params& P) {
     LatFill<PER> F;
-    F.nx = P.L.nx; F.ny = P.L.ny; F.px = P.periodic[0]; F.py = P.periodic[1];
-    for (int o = 0; o < 6; ++o) {
-        for (int f = 0; f < 4; ++f) F.kind[f][o] = P.bck[f][o];
-        for (int v = 0; v < 3; ++v) F.vel[v][o] = P.vel_extdir[v][o];
-        for (int n = 0; n < ERFX_NCONS_MOIST; ++n) F.ext[n][o] = P.cons_extdir[n][o];
+    F.nx = P.L.nx; F.ny = P.L.ny;
+    if constexpr (!PER) {
+        F.px = P.periodic[0]; F.py = P.periodic[1];
+        for (int o = 0; o < 6; ++o) {
+            for (int f = 0; f < 4; ++f) F.kind[f][o] = P.bck[f][o];
+            for (int v = 0; v < 3; ++v) F.vel[v][o] = P.vel_extdir[v][o];
+            for (int n = 0; n < ERFX_NCONS_MOIST; ++n) F.ext[n][o] = P.cons_extdir[n][o];
+        }
     }
     return F;
 }

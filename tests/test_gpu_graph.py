@@ -96,14 +96,12 @@ def test_autotune_picks_a_variant_and_keeps_results():
                                   "flat_tc32_40", "flat_tc32_80", "flat_tc32_deep100"])
 def test_tile_form_matches_column_form(case):
     """The tile form of the acoustic column kernel (the default) against the
-    one-lane-per-column form on level counts that leave the last wave's chunk
-    partial and trailing waves empty (37 levels: chunks of 3 over 16 waves;
-    21 levels on terrain: chunks of 3 over 8 waves), flat and terrain, dry
-    and moist: bit-identical after several steps.  Boxes of fewer than
-    16,384 columns take 16-column tiles (32 chunks of levels) and those of
-    8,192 or more 32-column tiles (16 chunks), also with 97..128 levels: 40 x
-    24 x 128 (16 columns, chunks of 4), 96 x 96 x 40 and x 80 (32 columns,
-    chunks of 3 and 5), 96 x 96 x 100 (32 columns, chunks of 7)."""
+    one-lane-per-column form on level counts that leave the last chunk partial and
+    trailing chunks empty, flat and terrain, dry and moist: bit-identical after
+    several steps.  Boxes of up to 8,160 columns take 16-column tiles (32 chunks
+    of levels: one level each at 21 and 30 levels, two at 37 and 50, four at 128),
+    larger ones 32-column tiles (16 chunks: three levels each at 40, five at 80,
+    seven at 100)."""
     if case == "flat37":
         cfg, f = P.rising_thermal(40, 24, 37, seed=21, adv=C.ADV_UPWIND3)
     elif case == "flat_deep128":
@@ -132,7 +130,7 @@ def test_tile_form_matches_column_form(case):
                                    (96, 96, 128)])
 def test_tile_form_chunk_edges(shape, moist):
     """The tile form where its chunks of levels change: one level per chunk (9
-    and 16 levels), one level past a full set of chunks (33 = 32 + 1 in 16-column
+    levels), two in 64-column tiles (16), one level past a full set of chunks (33 = 32 + 1 in 16-column
     tiles, 65 = 16 x 4 + 1 and 97 = 16 x 6 + 1 in 32-column tiles), the largest
     it takes (128), and a column count that leaves the last tile partial (41 x
     23, 97 x 95): bit-identical with one lane per column."""
@@ -164,6 +162,26 @@ def test_tile_form_few_levels(shape, moist):
     a.set_column_variant(7)          # one lane per column
     a.step(0.0, 0.5, 2)
     b.step(0.0, 0.5, 2)
+    assert _same(a, b) == []
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("moist", [False, True])
+@pytest.mark.parametrize("shape", [(97, 95, 65), (96, 96, 75), (96, 96, 96), (96, 96, 64), (97, 95, 97)])
+def test_terrain_tile_form_chunk_edges(shape, moist):
+    """The terrain grid's 32-column tiles: five levels per chunk with a last tile
+    that is partial (65 levels), five and six with a last chunk that is (75), six in
+    full (96), the four of the smaller form (64), and one level past what they take:
+    bit-identical with one lane per column."""
+    cfg, f = P.hill_flow(*shape, seed=59, moist=moist)
+    a, b = _pair(cfg, f)
+    a.set_graph(False)
+    a.set_column_variant(7)          # one lane per column
+    a.step(0.0, 0.2, 2)
+    b.step(0.0, 0.2, 2)
+    x = a.download(C.F_CONS)[C.RHO]
+    assert np.isfinite(x).all()
     assert _same(a, b) == []
     a.close()
     b.close()

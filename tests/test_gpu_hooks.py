@@ -129,6 +129,85 @@ def test_apply_bcs(kind, which, fast_only, synced):
     assert _same(sim, orc, ids) == {}
 
 
+# The open axis of a box: its lo and hi faces, with the other lateral axis
+# periodic.  (Inflow and symmetry on x are among KINDS.)
+LATERAL = {"x_slip": (0, C.BC_SLIP_WALL, C.BC_SLIP_WALL), "x_noslip": (0, C.BC_NO_SLIP_WALL, C.BC_SLIP_WALL),
+           "y_slip": (1, C.BC_SLIP_WALL, C.BC_SLIP_WALL), "y_noslip": (1, C.BC_SLIP_WALL, C.BC_NO_SLIP_WALL),
+           "y_symmetry": (1, C.BC_SYMMETRY, C.BC_OUTFLOW), "y_outflow": (1, C.BC_OUTFLOW, C.BC_SYMMETRY),
+           "y_inflow": (1, C.BC_INFLOW, C.BC_OUTFLOW), "y_inflow_moist": (1, C.BC_INFLOW, C.BC_OUTFLOW)}
+
+
+def _lateral(kind, shape):
+    """A box with rules on one lateral axis, in a wind oblique to its faces."""
+    d, lo, hi = LATERAL[kind]
+    moist = kind.endswith("moist")
+    cfg, f = (P.moist_bubble if moist else P.rising_thermal)(*shape, seed=53, adv=C.ADV_UPWIND3)
+    cfg.bc[d], cfg.bc[d + 3] = lo, hi
+    for o in (d, d + 3):
+        if cfg.bc[o] == C.BC_NO_SLIP_WALL:      # moving along itself
+            cfg.wall_velocity[o][1 - d], cfg.wall_velocity[o][2] = 2.5, 0.0
+        if cfg.bc[o] == C.BC_INFLOW:
+            cfg.inflow_velocity[o][d], cfg.inflow_velocity[o][1 - d] = 6.0, 1.5
+            cfg.inflow_density[o], cfg.inflow_theta[o], cfg.inflow_scalar[o] = 1.1, 300.0, 0.5
+            if moist:
+                cfg.inflow_qv[o] = 5.0e-3
+    L = C.layout_for(cfg)
+    ng = L.ng
+    for fid, c in ((C.F_XVEL, 0), (C.F_YVEL, 1)):
+        f[fid][0][ng:ng + cfg.nz, ng:ng + cfg.ny + c, ng:ng + cfg.nx + 1 - c] += 6.0 if c == d else 1.5
+    return cfg, f
+
+
+def _fill(sim, orc, which, ngc, ngv, fast_only, synced):
+    from erf_amd.lib import lib, check
+    orc.call("orc_apply_bcs", which, ngc, ngv, fast_only, synced)
+    check(lib().erfx_apply_bcs(sim.ctx, _st(sim, which), sim.ptr(C.F_XVEL), sim.ptr(C.F_YVEL),
+                               sim.ptr(C.F_ZVEL), ngc, ngv, fast_only, synced))
+    sim.sync()
+
+
+@pytest.mark.parametrize("kind", list(LATERAL))
+@pytest.mark.parametrize("shape", [(20, 18, 16), (9, 67, 8), (70, 7, 9)])
+def test_lateral_rules(kind, shape):
+    """Rules on the faces of one lateral axis, x or y: every fill (narrow and at full
+    width, fast variables alone and all, synced) and whole steps against the
+    oracle, bit for bit."""
+    import torch
+    assert torch.cuda.is_available()
+    from erf_amd.lib import Sim
+    cfg, f = _lateral(kind, shape)
+    orc, sim = Oracle(cfg), Sim(cfg)
+    orc.load(f)
+    orc.step(0.0, 0.5, 1)
+    ids = list(ALL_IDS) + ([C.D_RAIN_ACCUM] if cfg.moisture_type != C.MOIST_NONE else [])
+    for fid in ids:
+        sim.upload(fid, orc.get(fid))
+    ng = sim.L.ng
+    for args in ((C.S_SUM, 1, 1, 1, 0), (C.S_SUM, 2, 1, 0, 0), (C.S_SUM, ng, ng - 1, 1, 0),
+                 (C.S_NEW, ng, ng - 1, 0, 0), (C.S_OLD, ng, ng - 1, 0, 1)):
+        _fill(sim, orc, *args)
+        assert _same(sim, orc, ids) == {}, args
+    orc, sim = Oracle(cfg), Sim(cfg)
+    orc.load(f)
+    sim.load(f)
+    orc.step(0.0, 0.5, 3)
+    sim.step(0.0, 0.5, 3)
+    for fid in (C.F_CONS, C.F_XVEL, C.F_YVEL, C.F_ZVEL):
+        a, b = (valid(x.get(fid) if x is orc else x.download(fid), cfg, x.L, fid) for x in (sim, orc))
+        assert np.array_equal(a, b), fid
+
+
+@pytest.mark.parametrize("kind", ["thermal", "moist1", "walls", "inflow", "inflow_moist", "noslip", "hill"])
+def test_apply_bcs_fast_only_full_width(kind):
+    """the fill between substeps that are not chained: the fast variables at the full
+    velocity width; and with the ghost widths apart"""
+    cfg, orc, sim, ids, dt = _setup(kind)
+    ng = sim.L.ng
+    for ngc, ngv in ((ng, ng - 1), (1, ng - 1), (ng, 1)):
+        _fill(sim, orc, C.S_SUM, ngc, ngv, 1, 0)
+        assert _same(sim, orc, ids) == {}, (ngc, ngv)
+
+
 @pytest.mark.parametrize("kind", ["thermal", "inflow", "hill"])
 @pytest.mark.parametrize("shape", [(4, 4, 8), (5, 7, 8), (67, 6, 9), (8, 33, 17)])
 def test_apply_bcs_small_and_ragged(kind, shape):

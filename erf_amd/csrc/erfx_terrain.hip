@@ -1,11 +1,11 @@
 // erfx_terrain.hip -- terrain-following grid: the metrics of the node heights
 // and the acoustic substep erf_fast_rhs_T (static terrain, unit map factors).
 //
-// The substep runs as two phases: theta extrapolation, the horizontal momentum
-// increments and the new horizontal momenta on the faces; and one lane per
-// column that forms Omega of the old increments and the horizontal
-// divergence of the new ones as it sweeps up, solves the implicit vertical
-// system and updates rho, rho*theta and rho*w on the way down.  Every
+// The substep runs as two launches: theta extrapolation, the horizontal momentum
+// increments and the new horizontal momenta on the faces; and the columns (in
+// tiles whose lanes share a column's levels, or one lane each), which form Omega
+// of the old increments and the horizontal divergence of the new ones, solve the
+// implicit vertical system and update rho, rho*theta and rho*w.  Every
 // expression keeps the reference's operation order (FP contraction is off),
 // so each point carries the reference's rounding.
 #include "erfx_internal.h"

@@ -6,11 +6,11 @@
 //       extrapolated forward, horizontal momentum update, written straight into
 //       the current state (each lane reads prev and writes cur at its own
 //       index, so the S_prev == S_data aliasing is safe)
-//   K3-5 columns (one lane per (i, j), k loops): horizontal divergence of the
-//       increments, tridiagonal RHS, Thomas sweep, new rho*w, vertical
-//       fluxes, time-averaged rho*w, rho and rho*theta update; the lagged
-//       Delta(rho theta), which K1-2 of this substep has read, is replaced by
-//       the new one here, where each lane owns its column
+//   K3-5 columns (tiles of columns whose lanes share a column's levels, or one
+//       lane per column): horizontal divergence of the increments, tridiagonal
+//       RHS, Thomas sweep, new rho*w, vertical fluxes, time-averaged rho*w, rho
+//       and rho*theta update; the lagged Delta(rho theta), which K1-2 of this
+//       substep has read, is replaced by the new one here, each cell by one lane
 // The arithmetic of every point keeps the reference's operation order.
 #include "erfx_common.h"
 #include "erfx_internal.h"
@@ -254,10 +254,11 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
     // by each of the four faces that read it: 3 fields of neighbour reads, which
     // the four rows of a work-group share, in place of a field written and read
     // again by a launch of its own.  HBM bound at 13 fields read and 4 written
-    // (256 x 256 x 128: 283 us as two launches, 250 us as one, 4.6 TB/s).  With rt_prev the previous substep's
-    // apply_bcs is folded in: its momentum -> velocity -> momentum round trip
-    // (ERF_MomentumToVelocity.cpp, ERF_VelocityToMomentum.cpp) is applied to
-    // prev as it is read, and ghost cells are read at their periodic images.
+    // (256 x 256 x 128: 283 us as two launches, 250 us as one, 4.6 TB/s).  With
+    // rt_prev the previous substep's apply_bcs is folded in: its momentum ->
+    // velocity -> momentum round trip (ERF_MomentumToVelocity.cpp,
+    // ERF_VelocityToMomentum.cpp) is applied to prev as it is read, and ghost cells
+    // are read at their periodic images.
     const bool first = (nrk == 0 && step == 0);
     const bool rt = ch.rt_prev && step > 0;
     const bool use_lag = step > 0;
@@ -809,8 +810,8 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
 // For callers that cannot allocate device memory (code under stream / graph
 // capture, tight serving loops, harnesses that forbid hipMalloc): the work
 // fields of the substep (the rho*w increment, the two horizontal divergences
-// and the tridiagonal solution) and one field in reserve, 5 of the layout, live
-// in one static device array instead of a context's workspace.
+// and the tridiagonal solution), 4 of the layout, live in one static device
+// array instead of a context's workspace.
 // Each GPU holds its own copy of the array until the process ends; calls on
 // one GPU share it, so two calls that overlap on one GPU race.  No element of
 // it needs to start at zero: every launch of the substep writes each element
@@ -818,7 +819,8 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
 // before reading it, so whatever a previous call left there is never seen.
 namespace erfx {
 namespace noalloc {
-constexpr size_t SCRATCH_DOUBLES = size_t(8) << 20;      // 64 MiB
+constexpr size_t MAX_FIELD = (size_t(8) << 20) / 5;      // doubles of the largest box's layout
+constexpr size_t SCRATCH_DOUBLES = 4 * MAX_FIELD;         // 51.2 MiB
 constexpr int MAX_DEVICES = 64;
 static __device__ __align__(256) double scratch[SCRATCH_DOUBLES];
 // The array's device address per device, looked up once on the device's first
@@ -872,10 +874,10 @@ extern "C" int erfx_fast_rhs_N_noalloc(const erfx_config* cfg, void* stream, int
     erfx_layout lay;
     erfx_layout_for(cfg, &lay);
     const size_t ne = (size_t)lay.nelem;
-    if (5 * ne > noalloc::SCRATCH_DOUBLES) {
-        set_error("erfx_fast_rhs_N_noalloc: the box needs " + std::to_string(5 * ne) +
-                  " doubles of work space, the static buffer holds " + std::to_string(noalloc::SCRATCH_DOUBLES) +
-                  " (5 fields of the layout: boxes up to about 96 x 96 x 96 cells)");
+    if (ne > noalloc::MAX_FIELD) {
+        set_error("erfx_fast_rhs_N_noalloc: the box's layout has " + std::to_string(ne) +
+                  " doubles a field, the static buffer holds " + std::to_string(noalloc::MAX_FIELD) +
+                  " of each of its 4 (boxes up to about 108 x 108 x 108 cells)");
         return ERFX_ERR_ARG;
     }
     double* base = nullptr;
@@ -884,9 +886,9 @@ extern "C" int erfx_fast_rhs_N_noalloc(const erfx_config* cfg, void* stream, int
     Params P;
     make_params(*cfg, lay, P);
     FastWork W;
-    W.drw = base + ne;
-    W.trhs = base + 2 * ne;      // two components
-    W.soln = base + 4 * ne;
+    W.drw = base;
+    W.trhs = base + ne;          // two components
+    W.soln = base + 3 * ne;
     fast_rhs_N(P, W, step, nrk, *slow_rhs, *prev, *stage, prim, pi_stage, fast_coeffs, *data, *scratch, dtau,
                beta_s, facinv, static_cast<hipStream_t>(stream));
     hipError_t e = hipGetLastError();

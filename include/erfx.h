@@ -286,11 +286,11 @@ int erfx_fast_rhs_N(erfx_ctx* ctx, int step, int nrk,
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments and results as erfx_fast_rhs_N, with the configuration and the
  * stream (a hipStream_t, NULL for the default stream) in place of a context:
- * the substep's work fields live in a static device array of 64 MiB per GPU
+ * the substep's 4 work fields live in a static device array of 51.2 MiB per GPU
  * (held until the process ends) instead of a context's workspace, looked up
  * once per device on the first call made with that device current.  Boxes
- * whose 5 work fields of the layout exceed it (about 96 x 96 x 96 cells and
- * up) are refused with ERFX_ERR_ARG before any device work.  Calls on one GPU
+ * whose layout has more than 1,677,721 elements a field (about 108 x 108 x 108
+ * cells and up) are refused with ERFX_ERR_ARG before any device work.  Calls on one GPU
  * share the array: two calls that overlap on one GPU race.  Flat grids only
  * (a terrain grid returns ERFX_ERR_STATE). */
 int erfx_fast_rhs_N_noalloc(const erfx_config* cfg, void* stream, int step, int nrk,
@@ -524,9 +524,11 @@ int  erfx_sim_sync(erfx_sim* sim);
 int  erfx_sim_set_graph(erfx_sim* sim, int on);
 /* Variants of the acoustic column kernel of erf_fast_rhs_N: 0..8 one lane per
  * column (levels of loads in flight 2/3/4 x work-group width 64/128/256), 9
- * the tile form (64 columns per work-group of 16 waves, the sweep's
- * intermediates in LDS; boxes of up to 128 levels, variant 7 above that), the
- * default.  Every variant computes the same values. */
+ * the tile form (16, 32 or 64 columns per work-group of 8 waves, by the numbers
+ * of columns and levels; a column's levels are split over its lanes, which keep
+ * what they read; boxes of up to 128 levels, in an ensemble and on a terrain
+ * grid up to 96, variant 7 above that), the default.  Every variant computes the
+ * same values. */
 #define ERFX_COL_VARIANTS 10
 /* Autotuner of the acoustic column kernel (no counterpart in the reference):
  * with `on`, the next 3 x ERFX_COL_VARIANTS launches of the erf_fast_rhs_N

@@ -77,6 +77,38 @@ def test_noalloc_fast_rhs_N_matches_context_hook():
         assert not diff, "not bit-identical: %s" % diff
 
 
+@pytest.mark.parametrize("shape", [(106, 107, 107), (250, 74, 68)])
+def test_noalloc_just_within_its_scratch(shape):
+    """Boxes that fill the four work fields to a few per cent, and one level more
+    until the first that does not fit: the same values, then a refusal."""
+    import torch
+    assert torch.cuda.is_available()
+    from erf_amd.lib import Sim, lib, check
+    fn = _noalloc()
+    cfg, f = P.rising_thermal(*shape, seed=7, adv=C.ADV_UPWIND3)
+    limit = (8 << 20) // 5
+    assert 0.95 * limit < C.layout_for(cfg).nelem <= limit
+    out = []
+    for alloc in (True, False):
+        s = Sim(cfg)
+        s.load(f)
+        s.step(0.0, 0.2, 1)
+        st = [ctypes.byref(s.state(n)) for n in (C.F_SLOW, C.S_SUM, C.S_NEW, C.S_SUM, C.S_SCRATCH)]
+        args = (2, 2, st[0], st[1], st[2], s.ptr(C.D_PRIM), s.ptr(C.D_PI_STAGE), s.ptr(C.D_FAST_COEFFS),
+                st[3], st[4], 0.02, 0.1, 0.1)
+        check(lib().erfx_fast_rhs_N(s.ctx, *args) if alloc else fn(ctypes.byref(cfg), s.stream, *args))
+        s.sync()
+        out.append([s.download(C.state_id(n, c)) for n in (C.S_SUM, C.S_SCRATCH) for c in range(4)])
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b, equal_nan=True)
+    while C.layout_for(cfg).nelem <= limit:
+        cfg.nz += 1
+    from erf_amd.lib import State
+    d = ctypes.byref(State(1, 1, 1, 1))     # never dereferenced: the size check comes first
+    assert fn(ctypes.byref(cfg), None, 0, 0, d, d, d, 1, 1, 1, d, d, 0.1, 0.1, 1.0) == -1
+
+
 def test_noalloc_rejects_a_box_beyond_its_scratch():
     import torch
     assert torch.cuda.is_available()

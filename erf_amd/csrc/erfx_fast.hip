@@ -540,6 +540,9 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         constexpr int TC = decltype(tcc)::value;   // columns per tile
         constexpr int NCH = 512 / TC;              // chunks of levels
         const int tid = (int)threadIdx.x;
+        // read here once: in a batch captures are loads, and the wait for them in the
+        // middle of the sweeps took 2% of the kernel
+        const int mode = __builtin_amdgcn_readfirstlane((implicit ? 1 : 0) | (separate ? 2 : 0));
         const int chl = tile_chunk(nz, NCH);
         const int ka = chunk * chl;
         const int kb = (ka + chl < nz ? ka + chl : nz) - 1;
@@ -691,7 +694,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
 #pragma unroll
             for (int m = 0; m < CM; ++m)
                 if (ka + m <= kb) az[m] = seed ? sz_[m] : scratch.zmom[q0 + (long)(ka + m) * sz];
-            if (separate) {    // the cells to update are not the ones read so far
+            if (mode & 2) {    // the cells to update are not the ones read so far
 #pragma unroll
                 for (int m = 0; m < CM; ++m)
                     if (ka + m <= kb) {
@@ -703,7 +706,7 @@ void fast_rhs_N(const Params& P, const FastWork& W, int step, int nrk, const erf
         if (CM <= 6 && work) load3();
         // ---- phase 2: the sweeps ----
         double x_hi = 0.0;       // the solution on the chunk's upper face
-        relay_solve<CM, TC>(carry, xch, implicit, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
+        relay_solve<CM, TC>(carry, xch, (mode & 1) != 0, nz, chl, col, valid, rhs, av, bv, cv, r_top, a_top, b_top, s_top, x_hi);
         // ---- phase 3: the chunk's cells ----
         if (work) {
             if (CM > 6) load3();

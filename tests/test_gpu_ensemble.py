@@ -177,6 +177,25 @@ def test_ensemble_open_axis_with_a_small_member(small):
         s.close()
 
 
+def test_ensemble_open_axes_x_and_y():
+    """members open along different axes take the same fill kernels"""
+    from erf_amd.lib import Ensemble
+    cases = [P.rising_thermal(16, 16, 16, seed=1, adv=C.ADV_UPWIND3),
+             P.rising_thermal(20, 12, 16, seed=2, adv=C.ADV_UPWIND3), P.inflow_outflow(16, 16, 16, seed=3)]
+    for (cfg, _), d in zip(cases, (1, 0)):
+        cfg.bc[d] = cfg.bc[d + 3] = C.BC_SLIP_WALL
+    a, b = _pairs(cases)
+    ens = Ensemble(a)
+    ens.set_streams(1)                 # all in one batch
+    ens.step(0.0, 0.5, 3)
+    for s in b:
+        s.step(0.0, 0.5, 3)
+    assert _diff(a, b) == []
+    ens.close()
+    for s in a + b:
+        s.close()
+
+
 def test_ensemble_implicit_and_explicit_members():
     """the substep's solve is an option of a member, not another kernel"""
     from erf_amd.lib import Ensemble

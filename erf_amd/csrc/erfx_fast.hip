@@ -93,13 +93,14 @@ void make_fast_coeffs(const Params& P, double* fc, const erfx_state& stage, cons
     // over LDS on one chunk's lanes and the inverses are taken in parallel again.
     // 64 x 64 x 64: 24.9 us one lane per column, 10.3 us; 161 x 97 x 63 moist: 39.8
     // us, 34.2 us.  Two tiles fit the LDS of a CU, so 512 of 32 columns fill the
-    // chip once, and the line lies there, at 16,384 columns: tile and per-column form at 64 levels, dry and moist, 127 x 127 21.0 |
-    // 27.7, 24.5 | 30.8 us; 128 x 128 20.0 | 27.7, 23.8 | 30.8; 135 x 135 26.8 | 28.1,
-    // 30.6 | 30.8; 150 x 150 28.3 | 28.3, 33.4 | 31.3; 181 x 181 38.0 | 29.9 (16 and 40
-    // levels: 127 x 127 7.0 | 9.3 and 13.1 | 18.7, 181 x 181 11.1 | 10.5 and 25.0 |
-    // 20.2).  Chunks of more than 4 levels were slower too (190 x 150 x 80: 86 us
-    // against 53 profiled).  The lanes of the per-column form fill the chip there
-    // and it reads each level once (5.4 TB/s at 512 x 512 x 96).
+    // chip once, and the line lies there, at 16,384 columns.  Tile | per-column form
+    // at 64 levels, dry and moist: 127 x 127 21.0 | 27.7, 24.5 | 30.8 us; 128 x 128
+    // 20.0 | 27.7, 23.8 | 30.8; 135 x 135 26.8 | 28.1, 30.6 | 30.8; 150 x 150
+    // 28.3 | 28.3, 33.4 | 31.3; 181 x 181 dry 38.0 | 29.9.  At 16 and 40 levels, dry:
+    // 127 x 127 7.0 | 9.3 and 13.1 | 18.7, 181 x 181 11.1 | 10.5 and 25.0 | 20.2.
+    // Chunks of more than 4 levels were slower too (190 x 150 x 80: 86 us against 53
+    // profiled).  The lanes of the per-column form fill the chip there and it reads
+    // each level once (5.4 TB/s at 512 x 512 x 96).
     const long ncols = (long)nx * ny;
     auto tile = [=] __device__(int i, int j, bool valid, int col, int chunk, double* lds, auto cmc, auto tcc) {
         constexpr int CM = decltype(cmc)::value;
